@@ -129,22 +129,19 @@ __device__ inline void kahan_add(float& s, float& c, float x) {
     s = t;
 }
 
-// NT targets (weights w[t*ldw + lag - 1]); part[(c*NT + t)*ld + i].
-template <int NPL, int NT>
+template <int NPL>
 __global__ __launch_bounds__(kMemtermThreads) void k_memterm_f32c(
     const float* __restrict__ hist, int64_t ld, int depth, int first, const float* __restrict__ w,
-    int ldw, int chunk, double* __restrict__ part) {
+    int chunk, double* __restrict__ part) {
     typedef float vt __attribute__((ext_vector_type(NPL)));
     const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * NPL;
     if (i >= ld) return;
     const int c = blockIdx.y;
     const int s0 = first + c * chunk;
     const int s1 = min(depth, s0 + chunk);
-    float sm[NT][NPL], cm[NT][NPL];
+    float sm[NPL], cm[NPL];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int q = 0; q < NPL; ++q) sm[t][q] = cm[t][q] = 0.f;
+    for (int q = 0; q < NPL; ++q) sm[q] = cm[q] = 0.f;
     const int64_t ldv = ld / NPL;
     const vt* p = reinterpret_cast<const vt*>(hist + (int64_t)s0 * ld + i);
     const float* wp = w + (depth - 1 - s0);
@@ -155,33 +152,24 @@ __global__ __launch_bounds__(kMemtermThreads) void k_memterm_f32c(
         for (int u = 0; u < 8; ++u) x[u] = __builtin_nontemporal_load(p + (int64_t)u * ldv);
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
+            const float wt = wp[-u];
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const float wt = wp[t * ldw - u];
-#pragma unroll
-                for (int q = 0; q < NPL; ++q) kahan_add(sm[t][q], cm[t][q], wt * x[u][q]);
-            }
+            for (int q = 0; q < NPL; ++q) kahan_add(sm[q], cm[q], wt * x[u][q]);
         }
         p += 8 * ldv;
         wp -= 8;
     }
     for (; s < s1; ++s) {
         const vt x = __builtin_nontemporal_load(p);
+        const float wt = wp[0];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const float wt = wp[t * ldw];
-#pragma unroll
-            for (int q = 0; q < NPL; ++q) kahan_add(sm[t][q], cm[t][q], wt * x[q]);
-        }
+        for (int q = 0; q < NPL; ++q) kahan_add(sm[q], cm[q], wt * x[q]);
         p += ldv;
         wp -= 1;
     }
+    double* o = part + (int64_t)c * ld + i;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        double* o = part + ((int64_t)c * NT + t) * ld + i;
-#pragma unroll
-        for (int q = 0; q < NPL; ++q) o[q] = (double)sm[t][q] - (double)cm[t][q];
-    }
+    for (int q = 0; q < NPL; ++q) o[q] = (double)sm[q] - (double)cm[q];
 }
 
 // out[t*n + i] = scale * sum_c part[(c*NT+t)*ld + i] (+ out)
@@ -205,6 +193,13 @@ __global__ void k_sub(const double* __restrict__ a, const double* __restrict__ b
 }
 
 // ---------------------------------------------------------------- host side
+// Time chunks that make kMemtermWaves wavefronts of ld nodes: one, unless the
+// nodes alone give fewer; at most kMaxChunks.
+static int node_chunks(int64_t ld) {
+    const int64_t waves = ld / (2 * kWave);
+    return (int)std::min<int64_t>(kMaxChunks, std::max<int64_t>(1, (kMemtermWaves + waves - 1) / waves));
+}
+
 int hist_alloc(frm_ctx* ctx, int64_t n_nodes, int32_t capacity, int32_t precision,
                frm_hist** out) {
     FRM_REQUIRE(ctx, ctx && out && n_nodes > 0 && capacity > 0, "frm_hist_create: bad arguments");
@@ -221,7 +216,8 @@ int hist_alloc(frm_ctx* ctx, int64_t n_nodes, int32_t capacity, int32_t precisio
     h->ld = (n_nodes + kLdAlign - 1) / kLdAlign * kLdAlign;
     h->capacity = capacity;
     h->precision = precision;
-    h->max_chunks = kMaxChunks;
+    // partial sums of as many time chunks as a launch can take (pick_chunks)
+    h->max_chunks = node_chunks(h->ld);
     size_t bytes = (size_t)capacity * h->ld * esz;
     hipError_t e = hipMalloc(&h->data, bytes);
     if (e != hipSuccess) {
@@ -247,15 +243,11 @@ int hist_alloc(frm_ctx* ctx, int64_t n_nodes, int32_t capacity, int32_t precisio
     return FRM_OK;
 }
 
-// Number of time chunks for a launch: one, unless the nodes alone give fewer
-// than kMemtermWaves wavefronts; chunks never get shorter than kMinChunk.
+// Number of time chunks for a launch: the nodes' own, never shorter than
+// kMinChunk slots.
 static int pick_chunks(const frm_hist* h, int depth) {
     if (depth <= 0) return 0;
-    const int64_t waves = h->ld / (2 * kWave);
-    int nch = 1;
-    if (waves < kMemtermWaves) nch = (int)((kMemtermWaves + waves - 1) / waves);
-    nch = std::min<int>(nch, (depth + kMinChunk - 1) / kMinChunk);
-    return std::max(1, std::min(nch, h->max_chunks));
+    return std::max(1, std::min(h->max_chunks, (depth + kMinChunk - 1) / kMinChunk));
 }
 
 int memterm_chunks(const frm_hist* h, int first) {
@@ -280,8 +272,8 @@ int memterm_partials(frm_ctx* ctx, frm_hist* h, int ntargets, const double* d_w,
     const int threads = kMemtermThreads;
     dim3 grid((unsigned)(h->ld / 2 / threads), (unsigned)nchunks);
     if (h->precision == FRM_PREC_F32C) {
-        FRM_REQUIRE(ctx, (ntargets == 1 || ntargets == 2) && d_w32,
-                    "memterm_partials: FP32 store takes one or two targets and FP32 weights");
+        FRM_REQUIRE(ctx, ntargets == 1 && d_w32,
+                    "memterm_partials: FP32 store takes one target and FP32 weights");
         LaunchTimer timer(tctx, FRM_K_MEMTERM,
                           (double)span * h->n_nodes * sizeof(float) +
                               (double)ntargets * h->n_nodes * sizeof(double));
@@ -289,19 +281,11 @@ int memterm_partials(frm_ctx* ctx, frm_hist* h, int ntargets, const double* d_w,
         if (h->ld >= kF32WideLd) {
             // ld is a multiple of 4 * 256: the last workgroup may be half idle
             dim3 g4((unsigned)((h->ld / 4 + threads - 1) / threads), (unsigned)nchunks);
-            if (ntargets == 1)
-                hipLaunchKernelGGL((k_memterm_f32c<4, 1>), g4, dim3(threads), 0, ctx->stream, hf,
-                                   h->ld, depth, first, d_w32, ldw, chunk, part);
-            else
-                hipLaunchKernelGGL((k_memterm_f32c<4, 2>), g4, dim3(threads), 0, ctx->stream, hf,
-                                   h->ld, depth, first, d_w32, ldw, chunk, part);
+            hipLaunchKernelGGL(k_memterm_f32c<4>, g4, dim3(threads), 0, ctx->stream, hf, h->ld,
+                               depth, first, d_w32, chunk, part);
         } else {
-            if (ntargets == 1)
-                hipLaunchKernelGGL((k_memterm_f32c<2, 1>), grid, dim3(threads), 0, ctx->stream, hf,
-                                   h->ld, depth, first, d_w32, ldw, chunk, part);
-            else
-                hipLaunchKernelGGL((k_memterm_f32c<2, 2>), grid, dim3(threads), 0, ctx->stream, hf,
-                                   h->ld, depth, first, d_w32, ldw, chunk, part);
+            hipLaunchKernelGGL(k_memterm_f32c<2>, grid, dim3(threads), 0, ctx->stream, hf, h->ld,
+                               depth, first, d_w32, chunk, part);
         }
         FRM_HIP(ctx, hipGetLastError());
         return FRM_OK;

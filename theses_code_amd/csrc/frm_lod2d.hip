@@ -8,15 +8,17 @@
 // OpenCL version launches Om, Al, Bt and U separately, with Al/Bt/U on one
 // work-item per system and a Finish() after each launch.
 //
-// Here one step is three launches on one stream:
-//   1. memterm: both half-step history sums in one pass over the increments
-//      (rows use kb(s,1/2,0,1), columns kb(s,1,0,1); both depend only on the
-//      lag n-s for g(t) = t), split along time into FP64 partials -- or, for
-//      the chosen forms, the sum-of-exponentials recurrences or the blocked
-//      Toeplitz parts (frm_mfma.hip);
+// Here one step is two or three launches on one stream:
+//   1. memterm, both half-step history sums (rows use kb(s,1/2,0,1), columns
+//      kb(s,1,0,1)).  Where they depend on the lag n-s only (g(t) = t) the
+//      full-history forms sum the settled past once per block of steps
+//      (frm_blockhist.hip) and the row kernel adds the newest slots; the
+//      sum-of-exponentials recurrences, the blocked Toeplitz parts
+//      (frm_mfma.hip) and the other series run every step;
 //   2. rows: one to four wavefronts per row -- RHS assembly, Thomas forward
 //      and back substitution (chunked over lanes, scan seeds), boundary
-//      nodes, and a copy of C_n for step 3;
+//      nodes; the half-step field goes to a buffer of its own, so that C_n
+//      stays for step 3;
 //   3. cols: the same per column, plus the push of Delta_n = C_{n+1} - C_n
 //      into the history store.
 // With g(t) = t and a time-independent operator the tridiagonal matrices do
@@ -27,6 +29,7 @@
 #include <cstring>
 #include <vector>
 
+#include "frm_blockhist.hpp"
 #include "frm_gpow.hpp"
 #include "frm_history.hpp"
 #include "frm_iaibk.hpp"
@@ -54,9 +57,10 @@ struct frm_lod2d {
     double kr0 = 0, kc0 = 0, kch = 0;  // current-step weights
     frm_hist* hist = nullptr;
     double* C = nullptr;       // state, reference layout
-    double* Cprev = nullptr;   // C_n at interior nodes, compact node order
-    double* w = nullptr;       // [2][capacity] lag-indexed history weights
-    float* w32 = nullptr;      // FRM_PREC_F32C: the same in FP32
+    double* Cmid = nullptr;    // the field after the rows, interior nodes, compact order
+    double* w = nullptr;       // [2][ldw] lag-indexed history weights, 0 past the capacity
+    int ldw = 0;               // capacity + kHistBlock
+    double* far = nullptr;     // blocked full-history forms: [2][kHistBlock][hist->ld] far sums
     double* rcoef = nullptr;   // rows:    a, f, al interleaved per line (load_coefs)
     double* ccoef = nullptr;   // columns: the same
     frm::SweepShape rsh, csh;  // launch shapes of the row / column sweeps
@@ -134,19 +138,95 @@ __device__ inline void load_coefs(const double* coef, int line, int g, double (&
     }
 }
 
+// Where the row kernel takes its memory term from.
+enum RowSrc {
+    kRowPart,    // FP64 partial sums of both targets, formed by an earlier launch
+    kRowNear64,  // FP64 far sums of the block + its newest FP64 slots
+    kRowNear32,  // FP64 far sums of the block + its newest FP32 slots
+};
+
+// The newest slots s0 .. s0 + cnt - 1 of a block (cnt = n - s0) and the far
+// sums of step n for both targets.
+struct NearArgs {
+    const void* hist;
+    int64_t ld;
+    int s0, cnt;
+    const double* w;       // lag-indexed weights [2][ldw]
+    int ldw;
+    const double *f0, *f1; // far sums of the row / column target, or null
+    double* colpart;       // out: the column target's sum
+};
+
 struct RowArgs {
     double* C;
-    double* Cprev;
+    double* Cmid;
     const double* coef;  // interleaved, see load_coefs
-    const double* part;  // partial sums [nch][2][ldh], target 0
+    const double* part;  // kRowPart: partial sums [nch][2][ldh], target 0
     int64_t ldh;
     int nch;
     int ld, lines, n, NX;
     double negsk, S_half, sg, b0, al1;
+    NearArgs near;
 };
 
+// Both targets' sums of nodes q0 + r NL + g (r < CM, clamped to the line's
+// last): far sums, then the newest slots oldest first, all in FP64.  Reading
+// them here instead of in a kernel of their own saves that launch and, per
+// node, the row target's sum written and read back.
+template <typename HT, int CM, int NL>
+__device__ __forceinline__ void near_sums(const NearArgs& a, int64_t q0, int g, int n,
+                                          double (&ts)[CM], double (&tc)[CM]) {
+    int e[CM];
+#pragma unroll
+    for (int r = 0; r < CM; ++r) {
+        e[r] = min(r * NL + g, n - 1);
+        ts[r] = tc[r] = 0.0;
+    }
+    if (a.f0) {
+        const double* __restrict__ f0 = a.f0 + q0;
+        const double* __restrict__ f1 = a.f1 + q0;
+#pragma unroll
+        for (int r = 0; r < CM; ++r) {
+            ts[r] = f0[e[r]];
+            tc[r] = f1[e[r]];
+        }
+    }
+    constexpr int U = CM >= 16 ? 1 : 16 / CM;  // slots whose loads go out together
+    const HT* __restrict__ h = static_cast<const HT*>(a.hist) + (int64_t)a.s0 * a.ld + q0;
+    const double* __restrict__ w0 = a.w + a.cnt - 1;  // the oldest near slot's lag
+    const double* __restrict__ w1 = w0 + a.ldw;
+    int u = 0;
+    for (; u + U <= a.cnt; u += U) {
+        HT x[U][CM];
+#pragma unroll
+        for (int v = 0; v < U; ++v)
+#pragma unroll
+            for (int r = 0; r < CM; ++r) x[v][r] = h[(int64_t)(u + v) * a.ld + e[r]];
+#pragma unroll
+        for (int v = 0; v < U; ++v) {
+            const double p = w0[-(u + v)], q = w1[-(u + v)];
+#pragma unroll
+            for (int r = 0; r < CM; ++r) {
+                ts[r] += p * (double)x[v][r];
+                tc[r] += q * (double)x[v][r];
+            }
+        }
+    }
+    for (; u < a.cnt; ++u) {
+        HT x[CM];
+#pragma unroll
+        for (int r = 0; r < CM; ++r) x[r] = h[(int64_t)u * a.ld + e[r]];
+        const double p = w0[-u], q = w1[-u];
+#pragma unroll
+        for (int r = 0; r < CM; ++r) {
+            ts[r] += p * (double)x[r];
+            tc[r] += q * (double)x[r];
+        }
+    }
+}
+
 // Rows: 4 wavefronts per workgroup, 4/W lines.
-template <int CM, int W>
+template <int CM, int W, int SRC>
 __global__ __launch_bounds__(256) void k_lod_rows(RowArgs p) {
     constexpr int S = CM + 1;
     constexpr int LPB = 4 / W;
@@ -164,44 +244,52 @@ __global__ __launch_bounds__(256) void k_lod_rows(RowArgs p) {
     const int64_t qbase = (int64_t)line * p.NX;
     double* Crow = p.C + (int64_t)(line + 1) * p.ld;
     // The coefficients do not depend on the staging: their loads go out
-    // first and overlap the state loads (up to 16 elements per lane; at 32
-    // the registers would spill).
-    constexpr bool kEarly = CM <= 16;
+    // first and overlap the state loads (up to 16 elements per lane, 8 with
+    // the newest slots' sums; above that the registers would spill).
+    constexpr bool kEarly = CM <= (SRC == kRowPart ? 16 : 8);
     double a[CM], f[CM], al[CM], v[CM];
 #pragma unroll
     for (int k = 0; k < CM; ++k) a[k] = f[k] = al[k] = v[k] = 0.0;
     if (kEarly && live) load_coefs<CM, W>(p.coef, line, g, a, f, al);
     if (live) {
-        // om in element order: C_n (copied to Cprev) and the history sum.
-        // Every load is issued before the first store (clamped, unguarded
-        // indices; the pointers do not alias), so the row costs one memory
-        // latency instead of one per element group.  The first partial-sum
-        // chunk is loaded with the state (0 + p0 = p0 exactly, so the sum
-        // order is unchanged); further chunks follow.
+        // om in element order: C_n and the history sum.  Every load is
+        // issued before the first store (clamped, unguarded indices; the
+        // pointers do not alias), so the row costs one memory latency
+        // instead of one per element group.
         const double* __restrict__ cr = Crow + 1;
-        const double* __restrict__ pt = p.part + qbase;
-        double* __restrict__ cpv = p.Cprev + qbase;
-        const bool any = p.nch > 0;
         double u[CM], ts[CM];
 #pragma unroll
-        for (int r = 0; r < CM; ++r) {
-            const int e = min(r * NL + g, n - 1);
-            u[r] = cr[e];
-            ts[r] = any ? pt[e] : 0.0;
-        }
-        for (int c = 1; c < p.nch; ++c) {
-            const double* __restrict__ pc = pt + (int64_t)c * 2 * p.ldh;
-            double x[CM];
+        for (int r = 0; r < CM; ++r) u[r] = cr[min(r * NL + g, n - 1)];
+        if constexpr (SRC == kRowPart) {
+            // the first partial-sum chunk is loaded with the state (0 + p0 =
+            // p0 exactly, so the sum order is unchanged); further chunks follow
+            const double* __restrict__ pt = p.part + qbase;
+            const bool any = p.nch > 0;
 #pragma unroll
-            for (int r = 0; r < CM; ++r) x[r] = pc[min(r * NL + g, n - 1)];
+            for (int r = 0; r < CM; ++r) ts[r] = any ? pt[min(r * NL + g, n - 1)] : 0.0;
+            for (int c = 1; c < p.nch; ++c) {
+                const double* __restrict__ pc = pt + (int64_t)c * 2 * p.ldh;
+                double x[CM];
 #pragma unroll
-            for (int r = 0; r < CM; ++r) ts[r] += x[r];
+                for (int r = 0; r < CM; ++r) x[r] = pc[min(r * NL + g, n - 1)];
+#pragma unroll
+                for (int r = 0; r < CM; ++r) ts[r] += x[r];
+            }
+        } else {
+            double tc[CM];
+            if constexpr (SRC == kRowNear64)
+                near_sums<double, CM, NL>(p.near, qbase, g, n, ts, tc);
+            else
+                near_sums<float, CM, NL>(p.near, qbase, g, n, ts, tc);
+            double* __restrict__ cp = p.near.colpart + qbase;
+#pragma unroll
+            for (int r = 0; r < CM; ++r)
+                if (r * NL + g < n) cp[r * NL + g] = tc[r];
         }
 #pragma unroll
         for (int r = 0; r < CM; ++r) {
             const int e = r * NL + g;
             if (e < n) {
-                cpv[e] = u[r];
                 double om = p.negsk * u[r];
                 om += p.S_half;
                 om += p.sg * ts[r];
@@ -223,10 +311,12 @@ __global__ __launch_bounds__(256) void k_lod_rows(RowArgs p) {
     }
     __syncthreads();
     if (live) {
+        double* __restrict__ cm = p.Cmid + qbase;
         for (int r = 0; r < CM; ++r) {
             const int e = r * NL + g;
-            if (e < n) Crow[e + 1] = buf[e + e / CM];
+            if (e < n) cm[e] = buf[e + e / CM];
         }
+        // the boundary nodes, which neither sweep reads, go to the state
         if (g == 0) {
             Crow[0] = p.al1 * v[0] + p.b0;
             Crow[n + 1] = un;
@@ -236,8 +326,8 @@ __global__ __launch_bounds__(256) void k_lod_rows(RowArgs p) {
 }
 
 struct ColArgs {
-    double* C;
-    const double* Cprev;
+    double* C;           // in: C_n; out: C_{n+1}
+    const double* Cmid;  // the field after the rows
     double* slot;        // history slot for Delta_n (compact node order)
     float* slotf;        // FP32 history slot instead of slot when non-null
     const double* coef;  // interleaved, see load_coefs
@@ -283,7 +373,8 @@ __global__ __launch_bounds__((col_width<CM, W>() * kWave * W)) void k_lod_cols(C
     const int tline = grp * kColW + tc;
     const bool tlive = tline < p.lines;
     // coefficient loads first (they overlap the staging loads); the staging
-    // thread keeps its C_n values of Cprev for the increment push
+    // thread keeps its C_n values for the increment push and is the only one
+    // that overwrites them
     constexpr bool kEarly = CM <= 8;
     double a[CM], f[CM], al[CM], v[CM], cp[CM];
 #pragma unroll
@@ -293,15 +384,15 @@ __global__ __launch_bounds__((col_width<CM, W>() * kWave * W)) void k_lod_cols(C
         // all loads first (clamped indices), then the LDS writes
         const int i = tline + 1;
         const double* __restrict__ cc = p.C + i;
-        const double* __restrict__ cpv = p.Cprev + (i - 1);
+        const double* __restrict__ cm = p.Cmid + (i - 1);
         const bool any = p.nch > 0;
         const double* __restrict__ p0 = p.part + p.ldh + (i - 1);
         double u[CM], ts[CM];
 #pragma unroll
         for (int r = 0; r < CM; ++r) {
             const int e = min(r * NL + tr, n - 1);
-            u[r] = cc[(int64_t)(e + 1) * ld];
-            cp[r] = cpv[(int64_t)e * p.NX];  // node (i, j = e+1)
+            cp[r] = cc[(int64_t)(e + 1) * ld];
+            u[r] = cm[(int64_t)e * p.NX];  // node (i, j = e+1)
             ts[r] = any ? p0[(int64_t)e * p.NX] : 0.0;
         }
         for (int c = 1; c < p.nch; ++c) {
@@ -611,17 +702,33 @@ static int pick_cm(int n, int W) {
 #define FRM_SWEEP_CASES(X) X(4, 1) X(8, 1) X(16, 1) X(32, 1) X(4, 2) X(8, 2) X(16, 2) X(32, 2) \
     X(4, 4) X(8, 4) X(16, 4) X(32, 4)
 
+template <int SRC>
 static hipError_t launch_rows(SweepShape sh, hipStream_t st, const RowArgs& a) {
     const int lpb = 4 / sh.w;
     const dim3 grid((unsigned)((a.lines + lpb - 1) / lpb));
 #define X(CM, W)                                                                     \
     if (sh.cm == CM && sh.w == W) {                                                  \
-        hipLaunchKernelGGL((k_lod_rows<CM, W>), grid, dim3(256), 0, st, a);          \
+        hipLaunchKernelGGL((k_lod_rows<CM, W, SRC>), grid, dim3(256), 0, st, a);     \
         return hipGetLastError();                                                    \
     }
     FRM_SWEEP_CASES(X)
 #undef X
     return hipErrorInvalidValue;
+}
+
+// The row kernel's memory-term source for a solver's form.
+static RowSrc row_src(const frm_lod2d* s) {
+    if (s->g_func == 0 && s->precision == FRM_PREC_F64) return kRowNear64;
+    if (s->precision == FRM_PREC_F32C) return kRowNear32;
+    return kRowPart;
+}
+
+static hipError_t launch_rows(const frm_lod2d* s, hipStream_t st, const RowArgs& a) {
+    switch (row_src(s)) {
+        case kRowNear64: return launch_rows<kRowNear64>(s->rsh, st, a);
+        case kRowNear32: return launch_rows<kRowNear32>(s->rsh, st, a);
+        default: return launch_rows<kRowPart>(s->rsh, st, a);
+    }
 }
 
 static int col_groups(SweepShape sh, int lines) {
@@ -646,11 +753,23 @@ static hipError_t launch_cols(SweepShape sh, hipStream_t st, const ColArgs& a) {
     return hipErrorInvalidValue;
 }
 
-// Kernel arguments of one step's sweeps (n = step index, for the push slot).
-static RowArgs row_args(frm_lod2d* s, int nch) {
+// Kernel arguments of one step's sweeps (n = step index).  far: the block's
+// far sums are in s->far (the near forms; otherwise there are none yet).
+static RowArgs row_args(frm_lod2d* s, int nch, int n, bool far) {
     RowArgs a;
     a.C = s->C;
-    a.Cprev = s->Cprev;
+    a.Cmid = s->Cmid;
+    const int64_t hld = s->hist->ld;
+    const int N0 = n / kHistBlock * kHistBlock, j = n - N0;
+    a.near.hist = s->hist->data;
+    a.near.ld = hld;
+    a.near.s0 = N0;
+    a.near.cnt = j;
+    a.near.w = s->w;
+    a.near.ldw = s->ldw;
+    a.near.f0 = far ? s->far + (int64_t)j * hld : nullptr;
+    a.near.f1 = far ? s->far + (int64_t)(kHistBlock + j) * hld : nullptr;
+    a.near.colpart = s->hist->part + hld;
     a.coef = s->rcoef;
     a.part = s->hist->part;
     a.ldh = s->hist->ld;
@@ -672,7 +791,7 @@ static ColArgs col_args(frm_lod2d* s, int nch, int n) {
     const bool f32 = s->precision == FRM_PREC_MFMA_BF16 || s->precision == FRM_PREC_F32C;
     ColArgs a;
     a.C = s->C;
-    a.Cprev = s->Cprev;
+    a.Cmid = s->Cmid;
     const bool ring = soe || s->precision == FRM_PREC_BINOMIAL || s->precision == FRM_PREC_IAIBK;
     a.slot = (double*)s->hist->data +
              (int64_t)(ring ? (n % kSoeLag0) : s->hist->depth) * s->hist->ld;
@@ -719,6 +838,7 @@ static int tune_sweeps(frm_lod2d* s, int force) {
     FRM_HIP(ctx, hipEventCreate(&e0));
     FRM_HIP(ctx, hipEventCreate(&e1));
     constexpr int kWarm = 3, kReps = 20;
+    const int mid = std::min(kHistBlock / 2, s->hist->capacity);
     int rc = FRM_OK;
     for (int pass = 0; pass < 2 && rc == FRM_OK; ++pass) {
         const bool rows = pass == 0;
@@ -735,7 +855,8 @@ static int tune_sweeps(frm_lod2d* s, int force) {
             for (int it = 0; it < kWarm + kReps && e == hipSuccess; ++it) {
                 if (it == kWarm) e = hipEventRecord(e0, ctx->stream);
                 if (e != hipSuccess) break;
-                e = rows ? launch_rows(sh, ctx->stream, row_args(s, 1))
+                // a step in the middle of a block, without far sums
+                e = rows ? launch_rows(s, ctx->stream, row_args(s, 1, mid, false))
                          : launch_cols(sh, ctx->stream, col_args(s, 1, 0));
             }
             if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
@@ -785,7 +906,7 @@ static int gpow_prepare(frm_lod2d* s, int n) {
         LaunchTimer t(ctx, FRM_K_OTHER, 0.0);
         hipLaunchKernelGGL(k_gpow_weights, dim3((unsigned)((2 * n + 255) / 256)), dim3(256), 0,
                            ctx->stream, n, s->alpha, s->tau, s->g_pow, s->int_err, s->Da,
-                           s->capacity, s->w, s->flag);
+                           s->ldw, s->w, s->flag);
         FRM_HIP(ctx, hipGetLastError());
     }
     const int64_t nr = (int64_t)(s->M - 1) * s->NX, nc = (int64_t)(s->sN - 1) * s->NY;
@@ -805,9 +926,9 @@ static void lod_free(frm_lod2d* s) {
     if (!s) return;
     if (s->hist) frm_hist_destroy(s->hist);
     (void)hipFree(s->C);
-    (void)hipFree(s->Cprev);
+    (void)hipFree(s->Cmid);
     (void)hipFree(s->w);
-    (void)hipFree(s->w32);
+    (void)hipFree(s->far);
     (void)hipFree(s->rcoef);
     (void)hipFree(s->ccoef);
     (void)hipFree(s->soe_H);
@@ -954,8 +1075,12 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         return rc;
     }
     hipError_t e = hipMalloc(&s->C, nn * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&s->Cprev, nodes * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&s->w, (size_t)2 * d->capacity * sizeof(double));
+    if (e == hipSuccess) e = hipMalloc(&s->Cmid, nodes * sizeof(double));
+    s->ldw = d->capacity + kHistBlock;
+    if (e == hipSuccess) e = hipMalloc(&s->w, (size_t)2 * s->ldw * sizeof(double));
+    // far sums: a block past the first needs them
+    if (e == hipSuccess && row_src(s) != kRowPart && d->capacity > kHistBlock)
+        e = hipMalloc(&s->far, sizeof(double) * 2 * kHistBlock * s->hist->ld);
     // coefficient buffers sized for the longest padded line of any shape
     auto padded = [](int n) {
         int mx = 0;
@@ -1162,12 +1287,12 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
             return check_hip(ctx, e, "hipMalloc(lod2d MFMA)");
         }
     }
-    e = hipMemcpy(s->w, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice);
-    if (e == hipSuccess && d->precision == FRM_PREC_F32C) {
-        std::vector<float> w32(w.begin(), w.end());
-        e = hipMalloc(&s->w32, w32.size() * sizeof(float));
-        if (e == hipSuccess)
-            e = hipMemcpy(s->w32, w32.data(), w32.size() * sizeof(float), hipMemcpyHostToDevice);
+    {
+        std::vector<double> wp((size_t)2 * s->ldw, 0.0);
+        for (int t = 0; t < 2; ++t)
+            std::copy(w.begin() + (size_t)t * d->capacity, w.begin() + (size_t)(t + 1) * d->capacity,
+                      wp.begin() + (size_t)t * s->ldw);
+        e = hipMemcpy(s->w, wp.data(), wp.size() * sizeof(double), hipMemcpyHostToDevice);
     }
     if (e == hipSuccess) e = hipMemset(s->C, 0, nn * sizeof(double));
     if (e != hipSuccess) {
@@ -1179,14 +1304,14 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         lod_free(s);
         return rc;
     }
-    // leave no trace of the tuning runs: zero state, Cprev and history slots
+    // leave no trace of the tuning runs: zero state, Cmid and history slots
     {
         const size_t hb = (s->precision == FRM_PREC_MFMA_BF16 || s->precision == FRM_PREC_F32C
                                ? sizeof(float)
                                : sizeof(double)) *
                           (size_t)std::min(s->hist->capacity, kSoeLag0) * s->hist->ld;
         e = hipMemset(s->C, 0, nn * sizeof(double));
-        if (e == hipSuccess) e = hipMemset(s->Cprev, 0, nodes * sizeof(double));
+        if (e == hipSuccess) e = hipMemset(s->Cmid, 0, nodes * sizeof(double));
         if (e == hipSuccess) e = hipMemset(s->hist->data, 0, hb);
         if (e != hipSuccess) {
             lod_free(s);
@@ -1239,6 +1364,7 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
     for (int it = 0; it < nsteps; ++it) {
         const int n = s->tstep;
         int nch = 0;
+        bool far = false;
         if (s->g_func == 3) {
             const int rc = gpow_prepare(s, n);
             if (rc) return rc;
@@ -1326,7 +1452,7 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
             const int N1 = n / kSubSteps * kSubSteps;
             if (N1 > P0 && n == N1) {
                 LaunchTimer t(ctx, FRM_K_MEMTERM, (double)ld * ((N1 - P0) * 4.0 + 2 * kSubSteps * 4));
-                if (block_mid(ctx->stream, h32, ld, P0, N1, s->w, s->capacity, s->G))
+                if (block_mid(ctx->stream, h32, ld, P0, N1, s->w, s->ldw, s->G))
                     return check_hip(ctx, hipGetLastError(), "block_mid");
             }
             nch = 1;
@@ -1334,17 +1460,35 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
             LaunchTimer t(ctx, FRM_K_MEMTERM,
                           (double)ld * ((n - N1) * 4.0 + (useF ? 2 * 4 : 0) + (useG ? 2 * 4 : 0) +
                                         2 * 8));
-            if (block_near(ctx->stream, h32, ld, N0, N1, n, s->w, s->capacity, Fcur, useF, s->G, useG,
+            if (block_near(ctx->stream, h32, ld, N0, N1, n, s->w, s->ldw, Fcur, useF, s->G, useG,
                            s->hist->part))
                 return check_hip(ctx, hipGetLastError(), "block_near");
-        } else {
-            int rc = memterm_partials(ctx, s->hist, 2, s->w, s->capacity, &nch,
-                                      s->hist->depth - s->trunc_L, s->w32);
+        } else if (s->g_func == 3) {
+            int rc = memterm_partials(ctx, s->hist, 2, s->w, s->ldw, &nch);
             if (rc) return rc;
+        } else {
+            // the far sums of the block that starts here; the row kernel
+            // adds the block's own slots.  Restricted sums leave out the
+            // slots beyond their longest lag, whose weights are zero.
+            nch = 1;
+            const int N0 = n / kHistBlock * kHistBlock;
+            const int first = std::max(0, N0 - s->trunc_L);
+            far = first < N0;
+            if (far && n == N0) {
+                const bool f32 = s->precision == FRM_PREC_F32C;
+                LaunchTimer t(ctx, FRM_K_MEMTERM,
+                              (double)s->hist->n_nodes *
+                                  ((double)(N0 - first) * (f32 ? 4 : 8) + 2.0 * kHistBlock * 8));
+                const int rc = f32 ? hist_far(ctx->stream, (const float*)s->hist->data, s->hist->ld,
+                                              first, N0, s->w, s->ldw, s->far)
+                                   : hist_far(ctx->stream, (const double*)s->hist->data, s->hist->ld,
+                                              first, N0, s->w, s->ldw, s->far);
+                if (rc) return check_hip(ctx, hipGetLastError(), "hist_far");
+            }
         }
         {
             LaunchTimer t(ctx, FRM_K_ROWS, 0.0);
-            FRM_HIP(ctx, launch_rows(s->rsh, ctx->stream, row_args(s, nch)));
+            FRM_HIP(ctx, launch_rows(s, ctx->stream, row_args(s, nch, n, far)));
         }
         {
             LaunchTimer t(ctx, FRM_K_COLS, 0.0);

@@ -3,7 +3,7 @@ in the sweep) at the edges of a block and at grids of every launch variant.
 
 Tolerances: FP64, 1e-12 norm-wise relative error against the oracle, as the
 plain path's; FP32 increments, 1e-6 (each rounds at 2^-24 of itself, the sums
-are FP64)."""
+are FP64); the SOE form, 1e-6 (the bar its fit is held to at creation)."""
 import numpy as np
 import pytest
 
@@ -34,7 +34,8 @@ def _case(sN, M):
 
 
 # fewer nodes than 2^15, than 2^18, and more (one launch variant each)
-@pytest.mark.parametrize("precision,tol", [(N.PREC_F64, 1e-12), (N.PREC_F32C, 1e-6)])
+@pytest.mark.parametrize("precision,tol", [(N.PREC_F64, 1e-12), (N.PREC_F32C, 1e-6),
+                                           (N.PREC_SOE, 1e-6), (N.PREC_MFMA_BF16, 1e-6)])
 @pytest.mark.parametrize("sN,M", [(3, 2), (41, 33), (201, 188), (530, 511)])
 def test_lod2d_blocks_match_oracle(ctx, sN, M, precision, tol):
     coefs, C0 = _case(sN, M)
@@ -43,7 +44,7 @@ def test_lod2d_blocks_match_oracle(ctx, sN, M, precision, tol):
     g = S.TGSolver(ctx, sN, M, 0.7, 1e-3, 1.0, coefs, C0, capacity=steps, C1=0.0, S=0.05,
                    precision=precision)
     t = 0
-    for k in (1, B - 1, B, B + 1, 2 * B, steps):  # calls that end on, before and after a block
+    for k in (1, B // 2 - 1, B // 2, B // 2 + 1, B - 1, B, B + 1, 2 * B, steps):  # calls that end on, before and after a block
         o.step(k - t)
         g.calc_step(k - t)
         t = k

@@ -63,10 +63,10 @@ __device__ __forceinline__ void load_nodes(const HT* p, int m, double (&x)[NC]) 
 // four rows 4 r + l/16 of D.  KS wavefronts of a workgroup share a tile's
 // slots and add their sums through LDS in wavefront order, so that a small
 // grid, which has too few tiles to fill the chip, still uses all of it.
-template <typename HT, int NC, int KS>
+template <typename HT, typename GT, int NC, int KS>
 __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_hist_far(
     const HT* __restrict__ hist, int64_t ld, int first, int N0, const double* __restrict__ w,
-    int ldw, double* __restrict__ G) {
+    int ldw, GT* __restrict__ G) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int m = lane & 15, kg = lane >> 4;
     const int64_t tile = KS == 1 ? (int64_t)blockIdx.x * 4 + wv : blockIdx.x;
@@ -122,9 +122,9 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_hist_far(
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                double* g = G + (int64_t)(t * kHistBlock + 4 * r + kg) * ld + i0;
+                GT* g = G + (int64_t)(t * kHistBlock + 4 * r + kg) * ld + i0;
 #pragma unroll
-                for (int c = 0; c < NC; ++c) g[node_of<NC, HT>(c, m)] = acc[t][c][r];
+                for (int c = 0; c < NC; ++c) g[node_of<NC, HT>(c, m)] = (GT)acc[t][c][r];
             }
     } else {
         __shared__ double part[KS][2 * NC * 4][64];
@@ -140,26 +140,26 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_hist_far(
 #pragma unroll
             for (int p = 0; p < KS; ++p) v += part[p][q][lane];
             const int r = q & 3, c = (q >> 2) % NC, t = (q >> 2) / NC;
-            G[(int64_t)(t * kHistBlock + 4 * r + kg) * ld + i0 + node_of<NC, HT>(c, m)] = v;
+            G[(int64_t)(t * kHistBlock + 4 * r + kg) * ld + i0 + node_of<NC, HT>(c, m)] = (GT)v;
         }
     }
 }
 
-template <typename HT>
+template <typename HT, typename GT>
 static int far_launch(hipStream_t st, const HT* hist, int64_t ld, int first, int N0,
-                      const double* w, int ldw, double* G) {
+                      const double* w, int ldw, GT* G) {
     if (!hist || !w || !G || ld <= 0 || ld % 1024 || N0 <= 0 || N0 % kHistBlock || first < 0 ||
         first >= N0 || ldw < N0 + kHistBlock - 1)
         return -1;
     first = first / 4 * 4;
     if (ld >= 262144) {
-        hipLaunchKernelGGL((k_hist_far<HT, 4, 1>), dim3((unsigned)(ld / 256)), dim3(256), 0, st,
+        hipLaunchKernelGGL((k_hist_far<HT, GT, 4, 1>), dim3((unsigned)(ld / 256)), dim3(256), 0, st,
                            hist, ld, first, N0, w, ldw, G);
     } else if (ld >= 32768) {
-        hipLaunchKernelGGL((k_hist_far<HT, 4, 4>), dim3((unsigned)(ld / 64)), dim3(256), 0, st, hist,
+        hipLaunchKernelGGL((k_hist_far<HT, GT, 4, 4>), dim3((unsigned)(ld / 64)), dim3(256), 0, st, hist,
                            ld, first, N0, w, ldw, G);
     } else {
-        hipLaunchKernelGGL((k_hist_far<HT, 1, 8>), dim3((unsigned)(ld / 16)), dim3(512), 0, st, hist,
+        hipLaunchKernelGGL((k_hist_far<HT, GT, 1, 8>), dim3((unsigned)(ld / 16)), dim3(512), 0, st, hist,
                            ld, first, N0, w, ldw, G);
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
@@ -172,6 +172,11 @@ int hist_far(hipStream_t st, const double* hist, int64_t ld, int first, int N0, 
 
 int hist_far(hipStream_t st, const float* hist, int64_t ld, int first, int N0, const double* w,
              int ldw, double* G) {
+    return far_launch(st, hist, ld, first, N0, w, ldw, G);
+}
+
+int hist_far(hipStream_t st, const float* hist, int64_t ld, int first, int N0, const double* w,
+             int ldw, float* G) {
     return far_launch(st, hist, ld, first, N0, w, ldw, G);
 }
 

@@ -16,10 +16,13 @@ constexpr int kHistBlock = 16;
 // 1024, N0 > 0 a multiple of kHistBlock).  Slots before `first` are left out:
 // the caller's weights are zero there.  w is lag-indexed (w[0] for lag 1) and
 // readable up to lag N0 + kHistBlock - 1, ldw >= N0 + kHistBlock - 1.
+// An FP32 G rounds the FP64 sums once.
 // Returns nonzero on arguments outside these bounds or a failed launch.
 int hist_far(hipStream_t st, const double* hist, int64_t ld, int first, int N0, const double* w,
              int ldw, double* G);
 int hist_far(hipStream_t st, const float* hist, int64_t ld, int first, int N0, const double* w,
              int ldw, double* G);
+int hist_far(hipStream_t st, const float* hist, int64_t ld, int first, int N0, const double* w,
+             int ldw, float* G);
 
 }  // namespace frm

@@ -60,7 +60,9 @@ struct frm_lod2d {
     double* Cmid = nullptr;    // the field after the rows, interior nodes, compact order
     double* w = nullptr;       // [2][ldw] lag-indexed history weights, 0 past the capacity
     int ldw = 0;               // capacity + kHistBlock
-    double* far = nullptr;     // blocked full-history forms: [2][kHistBlock][hist->ld] far sums
+    double* far = nullptr;     // far sums of the current block: [2][kHistBlock][hist->ld]
+                               // (full history) or [2][kSoeBlock][hist->ld] (SOE, FP64 states)
+    int ring = 0;              // slots of an increment ring (0: the whole history is stored)
     double* rcoef = nullptr;   // rows:    a, f, al interleaved per line (load_coefs)
     double* ccoef = nullptr;   // columns: the same
     frm::SweepShape rsh, csh;  // launch shapes of the row / column sweeps
@@ -71,8 +73,9 @@ struct frm_lod2d {
     int soe_L = 0, soe_f32 = 0;
     double soe_err = 0.0;
     void* soe_H = nullptr;     // [L][ld] mode states (FP32 or FP64)
-    double* soe_q = nullptr;   // [L]
+    double* soe_q = nullptr;   // [L] (FP32 states)
     double* soe_c = nullptr;   // [2][L]
+    double* soe_tab = nullptr; // FP64 states: per mode the block's factors (k_soe_block)
     double soe_w1r = 0.0, soe_w1c = 0.0;  // exact lag-1 weights
     // FRM_PREC_BINOMIAL: moments [2][terms][ld] and per-step coefficient tables
     int bin_terms = 0;
@@ -92,7 +95,7 @@ struct frm_lod2d {
     int mfma_nprod = 6;        // 3 (two parts) or 6 (three parts)
     int far_slices = 8;        // node slices of a block's far product (1 to 64)
     float* F = nullptr;        // [2][128][ld]: far parts of this block and the next
-    float* G = nullptr;        // [16][ld] mid part of the current 8-step sub-block
+    float* G = nullptr;        // [2][kHistBlock][ld] mid part of the current sub-block
     // g(t) = t^p (g_func 3): the weights and the sweeps' Thomas coefficients
     // are rebuilt every step
     int g_func = 0;
@@ -143,6 +146,7 @@ enum RowSrc {
     kRowPart,    // FP64 partial sums of both targets, formed by an earlier launch
     kRowNear64,  // FP64 far sums of the block + its newest FP64 slots
     kRowNear32,  // FP64 far sums of the block + its newest FP32 slots
+    kRowNearMx,  // FP32 far and mid sums + the newest FP32 slots
 };
 
 // The newest slots s0 .. s0 + cnt - 1 of a block (cnt = n - s0) and the far
@@ -150,10 +154,11 @@ enum RowSrc {
 struct NearArgs {
     const void* hist;
     int64_t ld;
-    int s0, cnt;
+    int s0, cnt, mask;     // slot s is stored at s & mask (-1: the whole history)
     const double* w;       // lag-indexed weights [2][ldw]
     int ldw;
-    const double *f0, *f1; // far sums of the row / column target, or null
+    const void *f0, *f1;   // far sums of the row / column target, or null
+    const float *m0, *m1;  // kRowNearMx: mid sums, or null
     double* colpart;       // out: the column target's sum
 };
 
@@ -173,7 +178,7 @@ struct RowArgs {
 // last): far sums, then the newest slots oldest first, all in FP64.  Reading
 // them here instead of in a kernel of their own saves that launch and, per
 // node, the row target's sum written and read back.
-template <typename HT, int CM, int NL>
+template <typename HT, typename FT, int CM, int NL>
 __device__ __forceinline__ void near_sums(const NearArgs& a, int64_t q0, int g, int n,
                                           double (&ts)[CM], double (&tc)[CM]) {
     int e[CM];
@@ -183,16 +188,25 @@ __device__ __forceinline__ void near_sums(const NearArgs& a, int64_t q0, int g, 
         ts[r] = tc[r] = 0.0;
     }
     if (a.f0) {
-        const double* __restrict__ f0 = a.f0 + q0;
-        const double* __restrict__ f1 = a.f1 + q0;
+        const FT* __restrict__ f0 = static_cast<const FT*>(a.f0) + q0;
+        const FT* __restrict__ f1 = static_cast<const FT*>(a.f1) + q0;
 #pragma unroll
         for (int r = 0; r < CM; ++r) {
             ts[r] = f0[e[r]];
             tc[r] = f1[e[r]];
         }
     }
+    if constexpr (sizeof(FT) == 4) {
+        if (a.m0) {
+#pragma unroll
+            for (int r = 0; r < CM; ++r) {
+                ts[r] += (double)a.m0[q0 + e[r]];
+                tc[r] += (double)a.m1[q0 + e[r]];
+            }
+        }
+    }
     constexpr int U = CM >= 16 ? 1 : 16 / CM;  // slots whose loads go out together
-    const HT* __restrict__ h = static_cast<const HT*>(a.hist) + (int64_t)a.s0 * a.ld + q0;
+    const HT* __restrict__ h = static_cast<const HT*>(a.hist) + q0;
     const double* __restrict__ w0 = a.w + a.cnt - 1;  // the oldest near slot's lag
     const double* __restrict__ w1 = w0 + a.ldw;
     int u = 0;
@@ -201,7 +215,8 @@ __device__ __forceinline__ void near_sums(const NearArgs& a, int64_t q0, int g, 
 #pragma unroll
         for (int v = 0; v < U; ++v)
 #pragma unroll
-            for (int r = 0; r < CM; ++r) x[v][r] = h[(int64_t)(u + v) * a.ld + e[r]];
+            for (int r = 0; r < CM; ++r)
+                x[v][r] = h[(int64_t)((a.s0 + u + v) & a.mask) * a.ld + e[r]];
 #pragma unroll
         for (int v = 0; v < U; ++v) {
             const double p = w0[-(u + v)], q = w1[-(u + v)];
@@ -215,7 +230,7 @@ __device__ __forceinline__ void near_sums(const NearArgs& a, int64_t q0, int g, 
     for (; u < a.cnt; ++u) {
         HT x[CM];
 #pragma unroll
-        for (int r = 0; r < CM; ++r) x[r] = h[(int64_t)u * a.ld + e[r]];
+        for (int r = 0; r < CM; ++r) x[r] = h[(int64_t)((a.s0 + u) & a.mask) * a.ld + e[r]];
         const double p = w0[-u], q = w1[-u];
 #pragma unroll
         for (int r = 0; r < CM; ++r) {
@@ -278,9 +293,11 @@ __global__ __launch_bounds__(256) void k_lod_rows(RowArgs p) {
         } else {
             double tc[CM];
             if constexpr (SRC == kRowNear64)
-                near_sums<double, CM, NL>(p.near, qbase, g, n, ts, tc);
+                near_sums<double, double, CM, NL>(p.near, qbase, g, n, ts, tc);
+            else if constexpr (SRC == kRowNear32)
+                near_sums<float, double, CM, NL>(p.near, qbase, g, n, ts, tc);
             else
-                near_sums<float, CM, NL>(p.near, qbase, g, n, ts, tc);
+                near_sums<float, float, CM, NL>(p.near, qbase, g, n, ts, tc);
             double* __restrict__ cp = p.near.colpart + qbase;
 #pragma unroll
             for (int r = 0; r < CM; ++r)
@@ -565,8 +582,10 @@ constexpr int kSoeLag0 = 2;
 // replaces that frm_lod2d_create accepts
 constexpr double kSoeFitTol = 1e-6;
 
-template <typename HT, bool NT>
-__global__ __launch_bounds__(256) void k_soe_memterm(HT* __restrict__ H, const double* __restrict__ ring,
+// FP32 states take this step every step: their rounding after each is part of
+// the form.  FP64 states advance once per block (k_soe_block).
+template <bool NT>
+__global__ __launch_bounds__(256) void k_soe_memterm(float* __restrict__ H, const double* __restrict__ ring,
                                                      int64_t ld, int n, int L,
                                                      const double* __restrict__ q,
                                                      const double* __restrict__ c, double w1r,
@@ -582,8 +601,8 @@ __global__ __launch_bounds__(256) void k_soe_memterm(HT* __restrict__ H, const d
         double h = (double)stream_load<NT>(H + (int64_t)l * ld + i);
         if (fold) {
             h = q[l] * h + x;
-            stream_store<NT>((HT)h, H + (int64_t)l * ld + i);
-            h = (double)(HT)h;
+            stream_store<NT>((float)h, H + (int64_t)l * ld + i);
+            h = (double)(float)h;
         }
         s0 += c[l] * h;
         s1 += c[L + l] * h;
@@ -595,6 +614,64 @@ __global__ __launch_bounds__(256) void k_soe_memterm(HT* __restrict__ H, const d
     }
     part[i] = s0;
     part[ld + i] = s1;
+}
+
+// FP64 states, kSoeBlock = J steps at a time.  At a block start N0 the states
+// are H_l = sum_{s <= N0-2} q_l^(N0-2-s) Delta_s; a step n = N0 + j of the
+// block sums sum_l (c_{t,l} q_l^j) H_l over the slots before N0 - 1, formed
+// here for all j at once, and takes the at most J newer slots N0-1 .. n-1 with
+// their lags' weights (the exact one at lag 1, the fitted sum's values after)
+// in the row kernel.  One pass over the mode planes, which are read and
+// written once per J steps instead of every step, folds the J increments
+// N0-1-J .. N0-2 that have left the last block's reach (q_l^J H_l +
+// sum_i q_l^(J-1-i) Delta) and forms the 2 J sums.  The planes bound it (512 B
+// per node and block at 32 modes, against 24 multiply-adds per mode); with
+// J = 8 the sums add 128 B and the factors of a mode are 24 scalars.
+// Measured at 1024 x 1024, 32 modes: 104 us every step before.
+constexpr int kSoeBlock = 8;
+constexpr int kSoeRing = 16;  // increment slots: this block's and the last one's
+constexpr int kSoeTab = 3 * kSoeBlock;  // q^7 .. q^1, q^8, c_0 q^j, c_1 q^j
+
+template <bool NT>
+__global__ __launch_bounds__(256) void k_soe_block(double* __restrict__ H,
+                                                   const double* __restrict__ ring, int64_t ld,
+                                                   int N0, int L, const double* __restrict__ tab,
+                                                   double* __restrict__ G) {
+    constexpr int J = kSoeBlock;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= ld) return;
+    double x[J], g[2][J];
+#pragma unroll
+    for (int k = 0; k < J; ++k) {
+        const int s = N0 - 1 - J + k;  // before the first increment: nothing
+        x[k] = s >= 0 ? ring[(int64_t)(s & (kSoeRing - 1)) * ld + i] : 0.0;
+        g[0][k] = g[1][k] = 0.0;
+    }
+    constexpr int U = 4;  // modes whose loads go out together
+    for (int l0 = 0; l0 < L; l0 += U) {
+        double h[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) h[u] = stream_load<NT>(H + (int64_t)min(l0 + u, L - 1) * ld + i);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (l0 + u < L) {
+                const double* __restrict__ f = tab + (l0 + u) * kSoeTab;
+                double v = f[J - 1] * h[u] + x[J - 1];
+#pragma unroll
+                for (int k = 0; k < J - 1; ++k) v += f[k] * x[k];
+                stream_store<NT>(v, H + (int64_t)(l0 + u) * ld + i);
+#pragma unroll
+                for (int j = 0; j < J; ++j) {
+                    g[0][j] += f[J + j] * v;
+                    g[1][j] += f[2 * J + j] * v;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < J; ++j) G[(int64_t)(t * J + j) * ld + i] = g[t][j];
 }
 
 // ------------------------------------------------------------- binomial-series memory term
@@ -719,7 +796,9 @@ static hipError_t launch_rows(SweepShape sh, hipStream_t st, const RowArgs& a) {
 // The row kernel's memory-term source for a solver's form.
 static RowSrc row_src(const frm_lod2d* s) {
     if (s->g_func == 0 && s->precision == FRM_PREC_F64) return kRowNear64;
+    if (s->precision == FRM_PREC_SOE && !s->soe_f32) return kRowNear64;
     if (s->precision == FRM_PREC_F32C) return kRowNear32;
+    if (s->precision == FRM_PREC_MFMA_BF16) return kRowNearMx;
     return kRowPart;
 }
 
@@ -727,6 +806,7 @@ static hipError_t launch_rows(const frm_lod2d* s, hipStream_t st, const RowArgs&
     switch (row_src(s)) {
         case kRowNear64: return launch_rows<kRowNear64>(s->rsh, st, a);
         case kRowNear32: return launch_rows<kRowNear32>(s->rsh, st, a);
+        case kRowNearMx: return launch_rows<kRowNearMx>(s->rsh, st, a);
         default: return launch_rows<kRowPart>(s->rsh, st, a);
     }
 }
@@ -753,22 +833,36 @@ static hipError_t launch_cols(SweepShape sh, hipStream_t st, const ColArgs& a) {
     return hipErrorInvalidValue;
 }
 
-// Kernel arguments of one step's sweeps (n = step index).  far: the block's
-// far sums are in s->far (the near forms; otherwise there are none yet).
-static RowArgs row_args(frm_lod2d* s, int nch, int n, bool far) {
+// Kernel arguments of one step's sweeps (n = step index).  far, mid: the
+// block's far and mid sums are formed (the near forms; otherwise there are
+// none yet).
+static RowArgs row_args(frm_lod2d* s, int nch, int n, bool far, bool mid) {
     RowArgs a;
     a.C = s->C;
     a.Cmid = s->Cmid;
     const int64_t hld = s->hist->ld;
-    const int N0 = n / kHistBlock * kHistBlock, j = n - N0;
+    const bool soe = s->precision == FRM_PREC_SOE;
+    const int J = soe ? kSoeBlock : kHistBlock;
+    const int N0 = n / J * J, j = n - N0;
     a.near.hist = s->hist->data;
     a.near.ld = hld;
-    a.near.s0 = N0;
-    a.near.cnt = j;
+    a.near.s0 = soe ? std::max(0, N0 - 1) : N0;
+    a.near.cnt = n - a.near.s0;
+    a.near.mask = s->ring ? s->ring - 1 : -1;
     a.near.w = s->w;
     a.near.ldw = s->ldw;
     a.near.f0 = far ? s->far + (int64_t)j * hld : nullptr;
-    a.near.f1 = far ? s->far + (int64_t)(kHistBlock + j) * hld : nullptr;
+    a.near.f1 = far ? s->far + (int64_t)(J + j) * hld : nullptr;
+    a.near.m0 = a.near.m1 = nullptr;
+    if (s->precision == FRM_PREC_MFMA_BF16) {
+        // the 64-step block's far rows (by block parity), the sub-block's mid rows
+        const int b = n / kBlockSteps, q = n % kBlockSteps;
+        const float* F = s->F + (size_t)(b & 1) * 2 * kBlockSteps * hld;
+        a.near.f0 = far ? F + (int64_t)q * hld : nullptr;
+        a.near.f1 = far ? F + (int64_t)(kBlockSteps + q) * hld : nullptr;
+        a.near.m0 = mid ? s->G + (int64_t)j * hld : nullptr;
+        a.near.m1 = mid ? s->G + (int64_t)(kHistBlock + j) * hld : nullptr;
+    }
     a.near.colpart = s->hist->part + hld;
     a.coef = s->rcoef;
     a.part = s->hist->part;
@@ -787,14 +881,12 @@ static RowArgs row_args(frm_lod2d* s, int nch, int n, bool far) {
 }
 
 static ColArgs col_args(frm_lod2d* s, int nch, int n) {
-    const bool soe = s->precision == FRM_PREC_SOE;
     const bool f32 = s->precision == FRM_PREC_MFMA_BF16 || s->precision == FRM_PREC_F32C;
     ColArgs a;
     a.C = s->C;
     a.Cmid = s->Cmid;
-    const bool ring = soe || s->precision == FRM_PREC_BINOMIAL || s->precision == FRM_PREC_IAIBK;
     a.slot = (double*)s->hist->data +
-             (int64_t)(ring ? (n % kSoeLag0) : s->hist->depth) * s->hist->ld;
+             (int64_t)(s->ring ? (n % s->ring) : s->hist->depth) * s->hist->ld;
     a.slotf = f32 ? (float*)s->hist->data + (int64_t)s->hist->depth * s->hist->ld : nullptr;
     a.coef = s->ccoef;
     a.part = s->hist->part;
@@ -856,7 +948,7 @@ static int tune_sweeps(frm_lod2d* s, int force) {
                 if (it == kWarm) e = hipEventRecord(e0, ctx->stream);
                 if (e != hipSuccess) break;
                 // a step in the middle of a block, without far sums
-                e = rows ? launch_rows(s, ctx->stream, row_args(s, 1, mid, false))
+                e = rows ? launch_rows(s, ctx->stream, row_args(s, 1, mid, false, false))
                          : launch_cols(sh, ctx->stream, col_args(s, 1, 0));
             }
             if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
@@ -934,6 +1026,7 @@ static void lod_free(frm_lod2d* s) {
     (void)hipFree(s->soe_H);
     (void)hipFree(s->soe_q);
     (void)hipFree(s->soe_c);
+    (void)hipFree(s->soe_tab);
     (void)hipFree(s->bin_H);
     (void)hipFree(s->bin_upd);
     (void)hipFree(s->bin_er);
@@ -1062,12 +1155,17 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
     const int64_t nodes = (int64_t)s->NX * s->NY;
     const size_t nn = (size_t)s->ld * (d->M + 2);
     s->precision = d->precision;
-    // the SOE and binomial forms keep only a two-slot ring of increments,
-    // the blocked MFMA and compensated FP32 forms FP32 increments
+    // the SOE, binomial and ia/ibk forms keep only a ring of increments (two
+    // slots, or a block's with FP64 mode states), the blocked MFMA and
+    // compensated FP32 forms FP32 increments
     const bool mf = d->precision == FRM_PREC_MFMA_BF16;
-    const bool ring = d->precision == FRM_PREC_SOE || d->precision == FRM_PREC_BINOMIAL ||
-                      d->precision == FRM_PREC_IAIBK;
-    int rc = hist_alloc(ctx, nodes, ring ? kSoeLag0 : d->capacity,
+    s->soe_f32 = d->precision == FRM_PREC_SOE && d->soe_f32;
+    if (d->precision == FRM_PREC_SOE && !s->soe_f32)
+        s->ring = kSoeRing;
+    else if (d->precision == FRM_PREC_SOE || d->precision == FRM_PREC_BINOMIAL ||
+             d->precision == FRM_PREC_IAIBK)
+        s->ring = kSoeLag0;
+    int rc = hist_alloc(ctx, nodes, s->ring ? s->ring : d->capacity,
                         mf || d->precision == FRM_PREC_F32C ? d->precision : FRM_PREC_F64,
                         &s->hist);
     if (rc) {
@@ -1078,9 +1176,10 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
     if (e == hipSuccess) e = hipMalloc(&s->Cmid, nodes * sizeof(double));
     s->ldw = d->capacity + kHistBlock;
     if (e == hipSuccess) e = hipMalloc(&s->w, (size_t)2 * s->ldw * sizeof(double));
-    // far sums: a block past the first needs them
-    if (e == hipSuccess && row_src(s) != kRowPart && d->capacity > kHistBlock)
-        e = hipMalloc(&s->far, sizeof(double) * 2 * kHistBlock * s->hist->ld);
+    // far sums: a block past the first needs them (the MFMA form has its own)
+    const int block = d->precision == FRM_PREC_SOE ? kSoeBlock : kHistBlock;
+    if (e == hipSuccess && row_src(s) != kRowPart && !mf && d->capacity > block)
+        e = hipMalloc(&s->far, sizeof(double) * 2 * block * s->hist->ld);
     // coefficient buffers sized for the longest padded line of any shape
     auto padded = [](int n) {
         int mx = 0;
@@ -1164,9 +1263,9 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
     s->cplain = std::move(cc3);
     s->hw.assign({s->kr0, s->kc0, s->kch});
     s->hw.insert(s->hw.end(), w.begin(), w.end());
+    std::vector<double> near_w;  // SOE with FP64 states: [2][kSoeBlock] weights by lag
     if (d->precision == FRM_PREC_SOE) {
         s->soe_L = d->soe_terms > 0 ? d->soe_terms : 32;
-        s->soe_f32 = d->soe_f32;
         s->soe_w1r = w[0];
         s->soe_w1c = w[d->capacity];
         frm::SoeFit fit = frm::soe_fit({w.data(), w.data() + d->capacity}, d->capacity, kSoeLag0,
@@ -1184,10 +1283,35 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         }
         const size_t hsz = (s->soe_f32 ? sizeof(float) : sizeof(double)) * (size_t)s->soe_L * s->hist->ld;
         e = hipMalloc(&s->soe_H, hsz);
-        if (e == hipSuccess) e = hipMalloc(&s->soe_q, sizeof(double) * s->soe_L);
-        if (e == hipSuccess) e = hipMalloc(&s->soe_c, sizeof(double) * 2 * s->soe_L);
-        if (e == hipSuccess) e = hipMemcpy(s->soe_q, fit.q.data(), sizeof(double) * s->soe_L, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(s->soe_c, fit.c.data(), sizeof(double) * 2 * s->soe_L, hipMemcpyHostToDevice);
+        if (s->soe_f32) {
+            if (e == hipSuccess) e = hipMalloc(&s->soe_q, sizeof(double) * s->soe_L);
+            if (e == hipSuccess) e = hipMalloc(&s->soe_c, sizeof(double) * 2 * s->soe_L);
+            if (e == hipSuccess) e = hipMemcpy(s->soe_q, fit.q.data(), sizeof(double) * s->soe_L, hipMemcpyHostToDevice);
+            if (e == hipSuccess) e = hipMemcpy(s->soe_c, fit.c.data(), sizeof(double) * 2 * s->soe_L, hipMemcpyHostToDevice);
+        } else {
+            // a block's factors per mode, and the near weights: the exact one
+            // at lag 1, then the fitted sum's
+            constexpr int J = kSoeBlock;
+            const int L = s->soe_L;
+            std::vector<double> tab((size_t)L * kSoeTab);
+            near_w.assign(2 * J, 0.0);
+            for (int l = 0; l < L; ++l) {
+                double* f = tab.data() + (size_t)l * kSoeTab;
+                const double q = fit.q[l];
+                for (int k = 0; k < J - 1; ++k) f[k] = std::pow(q, J - 1 - k);
+                f[J - 1] = std::pow(q, J);
+                for (int t = 0; t < 2; ++t)
+                    for (int j = 0; j < J; ++j) {
+                        f[(1 + t) * J + j] = fit.c[(size_t)t * L + l] * std::pow(q, j);
+                        if (j + 2 <= J) near_w[t * J + j + 1] += f[(1 + t) * J + j];
+                    }
+            }
+            near_w[0] = s->soe_w1r;
+            near_w[J] = s->soe_w1c;
+            if (e == hipSuccess) e = hipMalloc(&s->soe_tab, sizeof(double) * tab.size());
+            if (e == hipSuccess)
+                e = hipMemcpy(s->soe_tab, tab.data(), sizeof(double) * tab.size(), hipMemcpyHostToDevice);
+        }
         if (e == hipSuccess) e = hipMemset(s->soe_H, 0, hsz);
         if (e != hipSuccess) {
             lod_free(s);
@@ -1279,7 +1403,7 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         e = hipMalloc(&s->atab, tab.size() * sizeof(uint16_t));
         // two far buffers: the current block's and the next one's, formed in slices
         if (e == hipSuccess) e = hipMalloc(&s->F, sizeof(float) * 2 * 2 * kBlockSteps * s->hist->ld);
-        if (e == hipSuccess) e = hipMalloc(&s->G, sizeof(float) * 2 * kSubSteps * s->hist->ld);
+        if (e == hipSuccess) e = hipMalloc(&s->G, sizeof(float) * 2 * kHistBlock * s->hist->ld);
         if (e == hipSuccess)
             e = hipMemcpy(s->atab, tab.data(), tab.size() * sizeof(uint16_t), hipMemcpyHostToDevice);
         if (e != hipSuccess) {
@@ -1289,7 +1413,10 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
     }
     {
         std::vector<double> wp((size_t)2 * s->ldw, 0.0);
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2 && !near_w.empty(); ++t)
+            std::copy(near_w.begin() + t * kSoeBlock, near_w.begin() + (t + 1) * kSoeBlock,
+                      wp.begin() + (size_t)t * s->ldw);
+        for (int t = 0; t < 2 && near_w.empty(); ++t)
             std::copy(w.begin() + (size_t)t * d->capacity, w.begin() + (size_t)(t + 1) * d->capacity,
                       wp.begin() + (size_t)t * s->ldw);
         e = hipMemcpy(s->w, wp.data(), wp.size() * sizeof(double), hipMemcpyHostToDevice);
@@ -1309,7 +1436,7 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         const size_t hb = (s->precision == FRM_PREC_MFMA_BF16 || s->precision == FRM_PREC_F32C
                                ? sizeof(float)
                                : sizeof(double)) *
-                          (size_t)std::min(s->hist->capacity, kSoeLag0) * s->hist->ld;
+                          (size_t)std::min(s->hist->capacity, std::max(s->ring, 1)) * s->hist->ld;
         e = hipMemset(s->C, 0, nn * sizeof(double));
         if (e == hipSuccess) e = hipMemset(s->Cmid, 0, nodes * sizeof(double));
         if (e == hipSuccess) e = hipMemset(s->hist->data, 0, hb);
@@ -1364,31 +1491,37 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
     for (int it = 0; it < nsteps; ++it) {
         const int n = s->tstep;
         int nch = 0;
-        bool far = false;
+        bool far = false, mid = false;
         if (s->g_func == 3) {
             const int rc = gpow_prepare(s, n);
             if (rc) return rc;
         }
-        if (soe) {
+        if (soe && s->soe_f32) {
             nch = 1;
             const int64_t ld = s->hist->ld;
-            LaunchTimer t(ctx, FRM_K_MEMTERM,
-                          (double)ld * (2.0 * s->soe_L * (s->soe_f32 ? 4 : 8) + 2 * 8 + 2 * 8));
+            LaunchTimer t(ctx, FRM_K_MEMTERM, (double)ld * (2.0 * s->soe_L * 4 + 2 * 8 + 2 * 8));
             const dim3 grid((unsigned)((ld + 255) / 256));
-            const bool nt = (double)ld * s->soe_L * (s->soe_f32 ? 4 : 8) >= kStreamBypassBytes;
-            auto launch = [&](auto kern, auto* H) {
-                hipLaunchKernelGGL(kern, grid, dim3(256), 0, ctx->stream, H,
-                                   (const double*)s->hist->data, ld, n, s->soe_L, s->soe_q,
-                                   s->soe_c, s->soe_w1r, s->soe_w1c, s->hist->part);
-            };
-            if (s->soe_f32) {
-                if (nt) launch(k_soe_memterm<float, true>, (float*)s->soe_H);
-                else launch(k_soe_memterm<float, false>, (float*)s->soe_H);
-            } else {
-                if (nt) launch(k_soe_memterm<double, true>, (double*)s->soe_H);
-                else launch(k_soe_memterm<double, false>, (double*)s->soe_H);
-            }
+            auto kern = (double)ld * s->soe_L * 4 >= kStreamBypassBytes ? k_soe_memterm<true>
+                                                                       : k_soe_memterm<false>;
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, ctx->stream, (float*)s->soe_H,
+                               (const double*)s->hist->data, ld, n, s->soe_L, s->soe_q, s->soe_c,
+                               s->soe_w1r, s->soe_w1c, s->hist->part);
             FRM_HIP(ctx, hipGetLastError());
+        } else if (soe) {
+            // the modes advance, and the block's far sums are formed, once per block
+            nch = 1;
+            const int64_t ld = s->hist->ld;
+            far = n >= kSoeBlock;
+            if (far && n % kSoeBlock == 0) {
+                LaunchTimer t(ctx, FRM_K_MEMTERM,
+                              (double)ld * 8 * (2.0 * s->soe_L + 3.0 * kSoeBlock));
+                const dim3 grid((unsigned)((ld + 255) / 256));
+                auto kern = (double)ld * s->soe_L * 8 >= kStreamBypassBytes ? k_soe_block<true>
+                                                                           : k_soe_block<false>;
+                hipLaunchKernelGGL(kern, grid, dim3(256), 0, ctx->stream, (double*)s->soe_H,
+                                   (const double*)s->hist->data, ld, n, s->soe_L, s->soe_tab, s->far);
+                FRM_HIP(ctx, hipGetLastError());
+            }
         } else if (iab) {
             // nothing to sum before the first increment
             nch = n > 0 ? 1 : 0;
@@ -1432,7 +1565,6 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
             const int P0 = std::max(0, N0 - kBlockSteps);
             const float* h32 = (const float*)s->hist->data;
             const size_t fsz = (size_t)2 * kBlockSteps * ld;
-            float* Fcur = s->F + (size_t)((N0 / kBlockSteps) & 1) * fsz;
             float* Fnext = s->F + (size_t)(((N0 / kBlockSteps) + 1) & 1) * fsz;
             const int every = kBlockSteps / s->far_slices;
             const int q = (n - N0) / every;
@@ -1448,21 +1580,18 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
                         return check_hip(ctx, hipGetLastError(), "block_far");
                 }
             }
-            // the slots from P0 up to the sub-block start, every 8 steps, summed in FP64
-            const int N1 = n / kSubSteps * kSubSteps;
-            if (N1 > P0 && n == N1) {
-                LaunchTimer t(ctx, FRM_K_MEMTERM, (double)ld * ((N1 - P0) * 4.0 + 2 * kSubSteps * 4));
-                if (block_mid(ctx->stream, h32, ld, P0, N1, s->w, s->ldw, s->G))
-                    return check_hip(ctx, hipGetLastError(), "block_mid");
-            }
+            // the slots from P0 up to the sub-block start, once per sub-block,
+            // summed in FP64; the row kernel adds the newest ones
+            const int N1 = n / kHistBlock * kHistBlock;
             nch = 1;
-            const bool useF = P0 > 0, useG = N1 > P0;
-            LaunchTimer t(ctx, FRM_K_MEMTERM,
-                          (double)ld * ((n - N1) * 4.0 + (useF ? 2 * 4 : 0) + (useG ? 2 * 4 : 0) +
-                                        2 * 8));
-            if (block_near(ctx->stream, h32, ld, N0, N1, n, s->w, s->ldw, Fcur, useF, s->G, useG,
-                           s->hist->part))
-                return check_hip(ctx, hipGetLastError(), "block_near");
+            far = P0 > 0;
+            mid = N1 > P0;
+            if (mid && n == N1) {
+                LaunchTimer t(ctx, FRM_K_MEMTERM,
+                              (double)ld * ((N1 - P0) * 4.0 + 2 * kHistBlock * 4));
+                if (hist_far(ctx->stream, h32, ld, P0, N1, s->w, s->ldw, s->G))
+                    return check_hip(ctx, hipGetLastError(), "hist_far");
+            }
         } else if (s->g_func == 3) {
             int rc = memterm_partials(ctx, s->hist, 2, s->w, s->ldw, &nch);
             if (rc) return rc;
@@ -1488,7 +1617,7 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
         }
         {
             LaunchTimer t(ctx, FRM_K_ROWS, 0.0);
-            FRM_HIP(ctx, launch_rows(s, ctx->stream, row_args(s, nch, n, far)));
+            FRM_HIP(ctx, launch_rows(s, ctx->stream, row_args(s, nch, n, far, mid)));
         }
         {
             LaunchTimer t(ctx, FRM_K_COLS, 0.0);

@@ -14,9 +14,9 @@
 // The reference forms every step's sum from scratch (fr_d_t_g_2d.cpp:
 // 3340-3437).  W and Delta are split into two or three BF16 parts whose
 // cross products accumulate in FP32 on v_mfma_f32_16x16x32_bf16.  The rest
-// is summed in FP64: every 8 steps the settled slots from P0 on
-// (k_block_mid, up to 120 slots), every step the F row, the mid row and at
-// most 7 recent slots (k_block_near).
+// is summed in FP64: every 16 steps the settled slots from P0 on (hist_far,
+// frm_blockhist.hip, up to 112 slots), every step, in the row kernel, the F
+// row, the mid row and at most 15 recent slots.
 #include <cstring>
 
 #include "frm_mfma.hpp"
@@ -201,131 +201,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     }
 }
 
-// Mid part of a 64-step block, refreshed every kSubSteps steps: for the
-// sub-block starting at N1 and the first slot P0 the far part leaves out
-// (P0 < N1 <= P0 + 120),
-//   G[t*8 + j][i] = sum_{P0 <= s < N1} w_t(N1 + j - s) Delta_s[i],  j < 8,
-// summed in FP64 and stored in FP32 like the far part F (two nodes per
-// thread, 8-byte loads of the FP32 slots; the weights are
-// wavefront-uniform).  FP32 storage rounds G at 2^-24, below the far part's
-// split-BF16 error; the FP64 store cost 64 more bytes per node and sub-block
-// and 8 more per node and step on the reading side.  N1 - P0 is a multiple
-// of 8: the slots go in batches of 8 whose loads are all issued before the
-// first product, and a batch's 8 x 8 products touch only the 15 lags
-// N1 - s0 - 7 .. N1 - s0 + 7.  Terms are added in increasing s, as a plain
-// loop over s would add them.
-__global__ __launch_bounds__(256) void k_block_mid(const float* __restrict__ hist, int64_t ld,
-                                                   int N0, int N1, const double* __restrict__ w,
-                                                   int ldw, float* __restrict__ G) {
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 2;
-    if (i >= ld) return;
-    double g[2][kSubSteps][2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int j = 0; j < kSubSteps; ++j) g[t][j][0] = g[t][j][1] = 0.0;
-    for (int s0 = N0; s0 < N1; s0 += kSubSteps) {
-        float2 x[kSubSteps];
-#pragma unroll
-        for (int u = 0; u < kSubSteps; ++u)
-            x[u] = *reinterpret_cast<const float2*>(hist + (int64_t)(s0 + u) * ld + i);
-        // wl[t][k] = w_t(L0 + k), L0 = N1 - s0 - 7 >= 1; lags past the
-        // capacity belong to no step and read as 0
-        const int L0 = N1 - s0 - (kSubSteps - 1);
-        double wl[2][2 * kSubSteps - 1];
-#pragma unroll
-        for (int k = 0; k < 2 * kSubSteps - 1; ++k) {
-            const bool ok = L0 + k <= ldw;
-            const int l = ok ? L0 + k : ldw;  // in bounds either way: unconditional loads
-            const double v0 = w[l - 1], v1 = w[ldw + l - 1];
-            wl[0][k] = ok ? v0 : 0.0;
-            wl[1][k] = ok ? v1 : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < kSubSteps; ++u) {
-            const double x0 = (double)x[u].x, x1 = (double)x[u].y;
-#pragma unroll
-            for (int j = 0; j < kSubSteps; ++j) {
-                // lag of step N1 + j from slot s0 + u
-                const int k = kSubSteps - 1 - u + j;
-                g[0][j][0] += wl[0][k] * x0;
-                g[0][j][1] += wl[0][k] * x1;
-                g[1][j][0] += wl[1][k] * x0;
-                g[1][j][1] += wl[1][k] * x1;
-            }
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int j = 0; j < kSubSteps; ++j)
-            *reinterpret_cast<float2*>(G + (int64_t)(t * kSubSteps + j) * ld + i) =
-                make_float2((float)g[t][j][0], (float)g[t][j][1]);
-}
-
-// part[t*ld + i] = F[t*64 + n - N0][i] + G[t*8 + n - N1][i]
-//                  + sum_{N1 <= s < n} w_t(n - s) Delta_s[i],
-// four nodes per thread (16-byte loads of the FP32 slots), FP64 sums.  The
-// slot count CNT = n - N1 (< 8) is a template parameter, so the CNT slot
-// loads, the F row and the G row are all in flight together.
-template <int CNT>
-__device__ __forceinline__ void near_part(const float* __restrict__ hist, int64_t ld, int64_t i,
-                                          int N0, int N1, int n, const double* __restrict__ w,
-                                          int ldw, const float* __restrict__ F, int use_F,
-                                          const float* __restrict__ G, int use_G,
-                                          double* __restrict__ part) {
-    float4 x[CNT > 0 ? CNT : 1];
-#pragma unroll
-    for (int u = 0; u < CNT; ++u)
-        x[u] = *reinterpret_cast<const float4*>(hist + (int64_t)(N1 + u) * ld + i);
-    double s0[4] = {0, 0, 0, 0}, s1[4] = {0, 0, 0, 0};
-    if (use_F) {
-        const int j = n - N0;
-        const float4 f0 = *reinterpret_cast<const float4*>(F + (int64_t)j * ld + i);
-        const float4 f1 = *reinterpret_cast<const float4*>(F + (int64_t)(kBlockSteps + j) * ld + i);
-        s0[0] = f0.x, s0[1] = f0.y, s0[2] = f0.z, s0[3] = f0.w;
-        s1[0] = f1.x, s1[1] = f1.y, s1[2] = f1.z, s1[3] = f1.w;
-    }
-    if (use_G) {
-        const int j = n - N1;
-        const float4 g0 = *reinterpret_cast<const float4*>(G + (int64_t)j * ld + i);
-        const float4 g1 = *reinterpret_cast<const float4*>(G + (int64_t)(kSubSteps + j) * ld + i);
-        s0[0] += g0.x, s0[1] += g0.y, s0[2] += g0.z, s0[3] += g0.w;
-        s1[0] += g1.x, s1[1] += g1.y, s1[2] += g1.z, s1[3] += g1.w;
-    }
-#pragma unroll
-    for (int u = 0; u < CNT; ++u) {
-        const int lag = CNT - u;  // slot N1 + u, step n = N1 + CNT
-        const double a = w[lag - 1], b = w[ldw + lag - 1];
-        s0[0] += a * (double)x[u].x, s1[0] += b * (double)x[u].x;
-        s0[1] += a * (double)x[u].y, s1[1] += b * (double)x[u].y;
-        s0[2] += a * (double)x[u].z, s1[2] += b * (double)x[u].z;
-        s0[3] += a * (double)x[u].w, s1[3] += b * (double)x[u].w;
-    }
-    *reinterpret_cast<double2*>(part + i) = make_double2(s0[0], s0[1]);
-    *reinterpret_cast<double2*>(part + i + 2) = make_double2(s0[2], s0[3]);
-    *reinterpret_cast<double2*>(part + ld + i) = make_double2(s1[0], s1[1]);
-    *reinterpret_cast<double2*>(part + ld + i + 2) = make_double2(s1[2], s1[3]);
-}
-
-__global__ __launch_bounds__(256) void k_block_near(const float* __restrict__ hist, int64_t ld,
-                                                    int N0, int N1, int n,
-                                                    const double* __restrict__ w, int ldw,
-                                                    const float* __restrict__ F, int use_F,
-                                                    const float* __restrict__ G, int use_G,
-                                                    double* __restrict__ part) {
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    if (i >= ld) return;
-#define FRM_NEAR_CASE(c) \
-    case c: near_part<c>(hist, ld, i, N0, N1, n, w, ldw, F, use_F, G, use_G, part); break;
-    switch (n - N1) {
-        FRM_NEAR_CASE(0) FRM_NEAR_CASE(1) FRM_NEAR_CASE(2) FRM_NEAR_CASE(3)
-        FRM_NEAR_CASE(4) FRM_NEAR_CASE(5) FRM_NEAR_CASE(6) FRM_NEAR_CASE(7)
-        default: break;
-    }
-#undef FRM_NEAR_CASE
-}
-
 int block_far(hipStream_t st, const float* hist, int64_t ld, int N0, int K, const void* atab,
               int atab_chunks, int nprod, float* F, int wg0, int nwg) {
     // the table must reach d = N0 + 32 (the carried fragment of the first
@@ -377,26 +252,6 @@ std::vector<uint16_t> atab_build(const float* wparts, int ldw, int chunks) {
                     }
     }
     return out;
-}
-
-int block_mid(hipStream_t st, const float* hist, int64_t ld, int N0, int N1, const double* w,
-              int ldw, float* G) {
-    if (ld % 2 || N0 < 0 || N1 <= N0 || N1 - N0 >= 2 * kBlockSteps || (N1 - N0) % kSubSteps) return -1;
-    const int64_t threads = ld / 2;
-    const dim3 grid((unsigned)((threads + 255) / 256)), block(256);
-    hipLaunchKernelGGL(k_block_mid, grid, block, 0, st, hist, ld, N0, N1, w, ldw, G);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-int block_near(hipStream_t st, const float* hist, int64_t ld, int N0, int N1, int n,
-               const double* w, int ldw, const float* F, int use_F, const float* G, int use_G,
-               double* part) {
-    if (ld % 4 || n < N1 || N1 < N0 || n - N1 >= kSubSteps || n - N0 >= kBlockSteps) return -1;
-    const int64_t threads = ld / 4;
-    const dim3 grid((unsigned)((threads + 255) / 256)), block(256);
-    hipLaunchKernelGGL(k_block_near, grid, block, 0, st, hist, ld, N0, N1, n, w, ldw, F, use_F, G,
-                       use_G, part);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 }  // namespace frm

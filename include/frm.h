@@ -254,9 +254,9 @@ int frm_lod2d_far_slices(const frm_lod2d* s, int32_t* slices);
  * Kind PSI forms kb_time every step on the GPU by calc_int's series
  * (mt_psi_caputo.cpp:720-740), and by its _kb quadrature fallback where a
  * series is not finite; frm_mt1d_get_state returns FRM_E_STATE if a weight
- * is still not finite.  The weights of step k + 1 are formed on the
- * context's second stream while step k runs (in order while per-launch
- * timing is on or in graph mode; the results are the same).
+ * is still not finite.  The weights of the next 16 steps are formed on the
+ * context's second stream while the 16 before run (in order while per-launch
+ * timing is on; the results are the same).
  * The history sum keeps the reference's index convention: the first two
  * snapshot increments never enter (mt_minimal.cpp:917-921).  Coefficient
  * forms: CONST (KK = D, C = 1), CV2 (KK = k, 1/C piecewise in U as cv_form 2,
@@ -300,15 +300,14 @@ typedef struct frm_mt1d_desc {
                           per run), built and instantiated the first time, then
                           replayed with these steps' arguments and grids set on
                           its nodes (hipGraphExecKernelNodeSetParams); kind psi
-                          forms the next step's weights on a branch beside the
-                          step.  Not while per-launch timing events are on */
-    int32_t hist_block; /* history block length: the shortest time chunk, in
-                           slots, into which the memory term splits the history
-                           when the nodes alone give too few wavefronts (the
-                           sweep adds one partial sum per chunk).  0: chosen at
-                           creation by timing the memory term and sweep at depth
-                           capacity/2 for 16..512 (frm_mt1d_hist_block reports
-                           it); > 0: that length */
+                          forms the next block's weights on a branch beside the
+                          steps.  Not while per-launch timing events are on */
+    int32_t hist_block; /* history block length: the fewest settled slots a
+                           wavefront takes where the memory term splits the
+                           history among several, when the nodes alone give too
+                           few of them (at most 16 share a node's history).
+                           0: 32 (frm_mt1d_hist_block reports it); > 0: that
+                           length */
 } frm_mt1d_desc;
 
 int frm_mt1d_create(frm_ctx* ctx, const frm_mt1d_desc* desc, frm_mt1d** out);

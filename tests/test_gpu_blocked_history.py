@@ -68,3 +68,47 @@ def test_lod2d_restricted_sums_across_blocks(ctx, keep):
     g.calc_step(steps)
     assert relerr(g.b_C, o.state().reshape(M + 2, sN + 2)) <= 1e-12
     g.close()
+
+
+def _mt_prob(n, rng, kind):
+    p = dict(N=n, L=1.0, alpha=float(rng.uniform(0.5, 0.9)))
+    if kind == N.MT_AB:
+        p.update(src=int(rng.integers(0, 3)), ab_maxl=50, ab_maxkiter=1000, ab_eps=1e-10)
+        return p, np.zeros(n + 2)
+    p.update(beta=float(rng.uniform(0.6, 1.4)), form=N.FORM_KEXP, k0=2e-3, b=1.0,
+             top=N.TOP_DIRICHLET, top_val=0.4, bottom_cond=1, Hbottom=0.2)
+    u = rng.uniform(0.1, 0.4, n + 2)
+    u[0], u[n], u[n + 1] = 0.4, 0.2, 0.2
+    return p, u
+
+
+# A batch large enough that every wavefront of the far sums takes four nodes
+# of one problem and its whole history, against its problems one by one (a
+# node's history split among wavefronts).  The sums are the same products in
+# FP64 in two orders; FP32 increments may round differently where the states
+# differ in the last bit.  Calls that end on and around a block's edges.
+@pytest.mark.parametrize("kind", [N.MT_L1, N.MT_PSI, N.MT_AB])
+@pytest.mark.parametrize("precision,tol", [(N.PREC_F64, 1e-12), (N.PREC_F32C, 1e-6)])
+def test_mt1d_large_batch_matches_single_problems(ctx, kind, precision, tol):
+    if kind == N.MT_AB and precision == N.PREC_F32C:
+        pytest.skip("the Atangana-Baleanu batch is FP64")
+    rng = np.random.default_rng(7)
+    sizes = [2, 3, 65, 66, 129, 256, 257, 258, 513, 770, 1025] + [128] * 1024
+    pairs = [_mt_prob(n, rng, kind) for n in sizes]
+    tau, steps = (1.0 / 400 if kind == N.MT_AB else 1e-3), 3 * B + 4
+    probs, U0 = [p for p, _ in pairs], [u for _, u in pairs]
+    b = S.MT1DBatch(ctx, probs, tau, steps, U0, kind=kind, precision=precision)
+    t = 0
+    for k in (1, 2, 3, B - 1, B + 1, B + 2, B + 3, 2 * B, steps):
+        b.calc_step(k - t)
+        t = k
+    got = b.state()
+    b.set_state(U0)
+    b.calc_step(steps)
+    assert all(np.array_equal(x, y) for x, y in zip(got, b.state()))
+    b.close()
+    for q in list(range(12)) + [500, len(sizes) - 1]:
+        s = S.MT1DBatch(ctx, [probs[q]], tau, steps, [U0[q]], kind=kind, precision=precision)
+        s.calc_step(steps)
+        assert relerr(got[q], s.state()[0]) <= tol, sizes[q]
+        s.close()

@@ -7,15 +7,18 @@
 // 1315-1342) over heap snapshots, the progonka back-substitution (1021-1022)
 // and, for psi, a full rebuild of kb_time with series integrals every step
 // (mt_psi_caputo.cpp:1481-1489).  Here a whole batch of problems of uneven
-// size advances together, three launches per step:
-//   1. (psi only) weights: one lane per (problem, interval), FP64 series;
-//   2. memory term: per node, over the stored increments; the problems are
-//      padded to 128-node groups so that each wavefront belongs to one
-//      problem and reads its weights through the scalar cache;
-//   3. sweep: one wavefront per problem -- coefficients from the current
+// size advances together, a block of kHistBlock steps at a time:
+//   1. (psi only) weights of the block's steps, which do not depend on the
+//      state: one lane per (problem, interval, step), FP64 series, formed on
+//      a second stream while the block before runs;
+//   2. far sums: the history of the block's steps up to its start, one pass
+//      over the stored increments for all of them (FP64 matrix cores);
+//   3. steps: one wavefront per problem runs the block's steps one after
+//      another -- the block's own increments, coefficients from the current
 //      iterate (held in LDS), Thomas alpha/beta/back-substitution with
-//      wavefront-scan chunk seeds, boundary rules, Picard iterations, and
-//      the push of the new increment.
+//      wavefront-scan chunk seeds, boundary rules, Picard iterations, and the
+//      push of the new increment.  Problems are independent, so nothing else
+//      has to be waited for between steps.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -24,6 +27,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "frm_blockhist.hpp"
 #include "frm_diag.h"
 #include "frm_history.hpp"
 #include "frm_wavescan.hpp"
@@ -32,15 +36,14 @@
 namespace frm {
 
 constexpr int kGroup = 128;       // nodes per memory-term wavefront
-constexpr int kMtCM = 16;         // largest unknowns per lane in the sweep (N - 1 <= 1024)
-constexpr int kMtMaxN = 64 * kMtCM + 1;
-
-// unknowns per lane for a batch whose largest problem has maxN intervals
-static int mt_pick_cm(int maxN) {
-    if (maxN - 1 <= 64 * 4) return 4;
-    if (maxN - 1 <= 64 * 8) return 8;
-    return 16;
-}
+// The step kernels run a problem on up to kMtMaxW wavefronts of one workgroup,
+// kMtCM unknowns per lane (N - 1 <= 1024).  Measured per step at 4 / 8 / 16
+// unknowns per lane: 4096 uneven psi problems 84 / 81 / 97 us, 1024 AB problems
+// 11.3 / 11.6 us, one 200-node problem 2.8 / 3.7 us; one wavefront per problem
+// of up to 16 per lane ran the psi problems in 215 us and spilled.
+constexpr int kMtCM = 4;
+constexpr int kMtMaxW = 4;
+constexpr int kMtMaxN = 64 * kMtCM * kMtMaxW + 1;
 
 struct MtProbDev {
     int N, form, top, bottom_cond, src;
@@ -51,31 +54,6 @@ struct MtProbDev {
     int ser, ser_maxl;
     int64_t ser_off, ser_coff;
 };
-
-// The memory term's time-chunk partials added per node, in chunk order (the
-// consumers of a chunked launch), for the CM nodes q0 + e0 + k (k < CM,
-// e0 + k < n) of a lane: the loads of 32 / CM chunks of every node are
-// issued together (clamped indices, so every load is in bounds).
-template <int CM>
-__device__ __forceinline__ void chunk_sums(const double* __restrict__ part, int64_t ldh, int nch,
-                                           int64_t q0, int e0, int n, double (&hs)[CM]) {
-    constexpr int B = CM >= 32 ? 1 : 32 / CM;
-#pragma unroll
-    for (int k = 0; k < CM; ++k) hs[k] = 0.0;
-    for (int c0 = 0; c0 < nch; c0 += B) {
-        double x[CM][B];
-#pragma unroll
-        for (int k = 0; k < CM; ++k)
-#pragma unroll
-            for (int u = 0; u < B; ++u)
-                x[k][u] = part[(int64_t)min(c0 + u, nch - 1) * ldh + q0 + min(e0 + k, n - 1)];
-#pragma unroll
-        for (int k = 0; k < CM; ++k)
-#pragma unroll
-            for (int u = 0; u < B; ++u)
-                if (c0 + u < nch && e0 + k < n) hs[k] += x[k][u];
-    }
-}
 
 // ---------------------------------------------------------------- physics
 // KK(i) and inv_dw_dh(i) of H_solver at state value x (mt_minimal.cpp:481-562
@@ -94,131 +72,186 @@ __device__ inline double mt_inv(const MtProbDev& P, double x) {
     return Ch != 0.0 ? 1.0 / Ch : 1e20;
 }
 
-// ---------------------------------------------------------------- memory term
-// part[c*ldh + j] = sum over slots of chunk c of w[prob(j)*ldw + depth-1-s] * Delta_s[j]
-// One wavefront = one 128-node group = one problem (gprob), so the weight
-// address is wavefront-uniform.  gvalid holds each group's count of real
-// nodes: the lanes past it (the padding of a problem's last group) issue no
-// loads, so the stream carries only the problems' own nodes (with 128-node
-// padding it carried 12% more on the 4096 uneven problems of the psi batch).
-typedef double mt_dv2 __attribute__((ext_vector_type(2)));
+// ---------------------------------------------------------------- far sums
+// G[j*ldh + i] = sum_{s < N0} w(N0 + j, s) Delta_s[i], j < J = kHistBlock, for
+// the node i of its problem p: the settled part of the history sums of the J
+// steps N0 .. N0 + J - 1 (history index: the number of increments before the
+// step).  One FP64 product per problem on v_mfma_f64_16x16x4_f64: the J steps
+// are its 16 rows, 16 NC nodes a wavefront's columns, four slots per
+// instruction (A[l%16][l/16] = w(N0 + l%16, s0 + l/16), B[l/16][l%16] =
+// Delta_{s0 + l/16}, D row 4 r + l/16).  The history is read once per J steps
+// instead of every step: 223 -> 16 us per step on 1024 uneven FP64 problems at
+// 300 slots, 302 -> 29 us on 4096 psi problems with FP32 increments at 200.
+//
+// Weights: lag-indexed per problem (w[p*ldw + lag - 1]), or (TAB) the psi
+// table w[(p*ldw + s)*J + j], whose four slots x 16 steps are one contiguous
+// load per instruction.  gprob/gvalid give each 128-node group's problem (-1:
+// none) and its count of real nodes; tiles past it are skipped, and a partial
+// tile's lanes repeat its last nodes, so the stream carries the problems' own
+// nodes only.  SPLIT: the wavefronts of a workgroup share a tile's slots and
+// add their sums through LDS in wavefront order, for batches with too few
+// tiles to fill the chip.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(kMemtermThreads) void k_mt_memterm_f64(
-    const double* __restrict__ hist, int64_t ldh, int depth, const double* __restrict__ w,
-    int ldw, const int* __restrict__ gprob, const int* __restrict__ gvalid, int chunk,
-    double* __restrict__ part) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t j = t * 2;
-    if (j >= ldh) return;
-    const int p = gprob[t >> 6];
-    const bool live = p >= 0 && (int)(j & (kGroup - 1)) < gvalid[t >> 6];
-    const int c = blockIdx.y;
-    const int s0 = c * chunk;
-    const int s1 = min(depth, s0 + chunk);
-    double a0 = 0.0, a1 = 0.0;
-    if (live) {
-        const int64_t ldv = ldh / 2;
-        const mt_dv2* q = reinterpret_cast<const mt_dv2*>(hist + (int64_t)s0 * ldh + j);
-        const double* wp = w + (int64_t)p * ldw + (depth - 1 - s0);
-        int s = s0;
-        for (; s + 4 <= s1; s += 4) {
-            mt_dv2 x[4];
+constexpr int kFarSplit = 16;  // wavefronts that share a tile at most
+
+template <typename HT, bool TAB, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * kFarSplit : 256) void k_mt_far(
+    const HT* __restrict__ hist, int64_t ldh, int N0, const double* __restrict__ w, int ldw,
+    const int* __restrict__ gprob, const int* __restrict__ gvalid, double* __restrict__ G) {
+    constexpr int NC = SPLIT ? 1 : 4;  // one node per lane, or four in 16-byte loads
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int m = lane & 15, kg = lane >> 4;
+    const int64_t i0 = (SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wv) * (16 * NC);
+    if (i0 >= ldh) return;
+    const int64_t grp = i0 / kGroup;
+    const int p = __builtin_amdgcn_readfirstlane(gprob[grp]);
+    const int left = __builtin_amdgcn_readfirstlane(gvalid[grp]) - (int)(i0 % kGroup);
+    if (p < 0 || left <= 0) return;  // SPLIT: the same for the whole workgroup
+    int a = 0, b = N0;
+    if constexpr (SPLIT) {
+        const int ks = blockDim.x >> 6, per = (N0 / 4 + ks - 1) / ks * 4;
+        a = min(N0, wv * per);
+        b = min(N0, a + per);
+    }
+    // the lane's nodes of column tile c: NC == 1: m; four FP32: 4 m + c; four
+    // FP64: 32 (c / 2) + 2 m + c % 2
+    typedef HT v2 __attribute__((ext_vector_type(2)));
+    typedef HT v4 __attribute__((ext_vector_type(4)));
+    auto nodes = [&](const HT* q, double (&x)[NC]) {
+        if constexpr (NC == 1) {
+            x[0] = (double)__builtin_nontemporal_load(q + min(m, left - 1));
+        } else if constexpr (sizeof(HT) == 4) {
+            const v4 v = __builtin_nontemporal_load(
+                reinterpret_cast<const v4*>(q + min(4 * m, (left - 1) & ~3)));
 #pragma unroll
-            for (int u = 0; u < 4; ++u) x[u] = __builtin_nontemporal_load(q + (int64_t)u * ldv);
+            for (int c = 0; c < 4; ++c) x[c] = (double)v[c];
+        } else {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                a0 = fma(wp[-u], x[u].x, a0);
-                a1 = fma(wp[-u], x[u].y, a1);
+            for (int h = 0; h < 2; ++h) {
+                const v2 v = __builtin_nontemporal_load(
+                    reinterpret_cast<const v2*>(q + min(32 * h + 2 * m, (left - 1) & ~1)));
+                x[2 * h] = (double)v.x;
+                x[2 * h + 1] = (double)v.y;
             }
-            q += 4 * ldv;
-            wp -= 4;
         }
-        for (; s < s1; ++s) {
-            const mt_dv2 x = __builtin_nontemporal_load(q);
-            a0 = fma(wp[0], x.x, a0);
-            a1 = fma(wp[0], x.y, a1);
-            q += ldv;
-            wp -= 1;
+    };
+    f64x4 acc[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] = f64x4{0.0, 0.0, 0.0, 0.0};
+    const HT* hp = hist + (int64_t)(a + kg) * ldh + i0;
+    const double* wp = TAB ? w + ((int64_t)p * ldw + a) * kHistBlock + lane % 16 + 16 * kg
+                           : w + (int64_t)p * ldw + (N0 - a - 1 + m - kg);
+    constexpr int ws = TAB ? 4 * kHistBlock : -4;  // weight stride of four slots
+    constexpr int U = NC == 1 ? 8 : 4;             // products whose loads go out together
+    int s = a;
+    for (; s + 4 * U <= b; s += 4 * U) {
+        double x[U][NC], v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            nodes(hp + (int64_t)(4 * u) * ldh, x[u]);
+            v[u] = wp[ws * u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[u], x[u][c], acc[c], 0, 0, 0);
+        hp += (int64_t)(4 * U) * ldh;
+        wp += ws * U;
+    }
+    for (; s < b; s += 4) {
+        double x[NC];
+        nodes(hp, x);
+        const double v = wp[0];
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(v, x[c], acc[c], 0, 0, 0);
+        hp += 4 * ldh;
+        wp += ws;
+    }
+    auto node = [&](int c) {
+        return NC == 1 ? m : sizeof(HT) == 4 ? 4 * m + c : 32 * (c >> 1) + 2 * m + (c & 1);
+    };
+    if constexpr (!SPLIT) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                if (node(c) < left) G[(int64_t)(4 * r + kg) * ldh + i0 + node(c)] = acc[c][r];
+    } else {
+        __shared__ double part[kFarSplit][4][64];
+        const int ks = blockDim.x >> 6;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[wv][r][lane] = acc[0][r];
+        __syncthreads();
+        for (int r = wv; r < 4; r += ks) {
+            double v = 0.0;
+            for (int k = 0; k < ks; ++k) v += part[k][r][lane];
+            if (m < left) G[(int64_t)(4 * r + kg) * ldh + i0 + m] = v;
         }
     }
-    part[(int64_t)c * ldh + j] = a0;
-    part[(int64_t)c * ldh + j + 1] = a1;
 }
 
-// FP32 increments, FP32 weights, Kahan-compensated FP32 sums; the chunk's
-// compensated sum is returned in FP64.  NPL nodes per lane: 2 (8-byte
-// loads, a wavefront is one 128-node group) or 4 (16-byte loads, each half
-// wavefront one group, each lane taking its half's problem weights).  Large
-// batches take 4 (4096 uneven psi problems: 5.8 -> 6.4 TB/s); small ones
-// keep 2, whose twice as many wavefronts fill the GPU with fewer time
-// chunks.
-
-__device__ inline void kahan_add(float& s, float& c, float x) {
-    const float y = x - c;
-    const float t = s + y;
-    c = (t - s) - y;
-    s = t;
+// A value that is the same on every lane, as the compiler can know it: it then
+// lives in scalar registers and its uses as an address are scalar.
+template <typename T>
+__device__ __forceinline__ T same_on_lanes(const T& v) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    union U {
+        T t;
+        int w[sizeof(T) / 4];
+        __device__ U() {}
+    } u;
+    u.t = v;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; ++i) u.w[i] = __builtin_amdgcn_readfirstlane(u.w[i]);
+    return u.t;
 }
 
-template <int NPL>
-__global__ __launch_bounds__(kMemtermThreads) void k_mt_memterm_f32c(
-    const float* __restrict__ hist, int64_t ldh, int depth, const float* __restrict__ w, int ldw,
-    const int* __restrict__ gprob, const int* __restrict__ gvalid, int chunk,
-    double* __restrict__ part) {
-    static_assert(NPL == 2 || NPL == 4, "two or four nodes per lane");
-    typedef float vt __attribute__((ext_vector_type(NPL)));
-    constexpr int SL = NPL == 2 ? 8 : 4;  // slots in flight per lane: 64 bytes
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t j = t * NPL;
-    const bool in = j < ldh;
-    const int64_t grp = in ? j / kGroup : 0;
-    const int p = in ? gprob[grp] : -1;
-    const bool live = in && p >= 0 && (int)(j & (kGroup - 1)) < gvalid[grp];
-    // the problems of the wavefront's groups, wavefront-uniform values (lanes
-    // past ldh carry p = -1; a dead group's weight pointer is problem 0's,
-    // in bounds and never used)
-    const int pa = __builtin_amdgcn_readfirstlane(p);
-    const int pb = NPL == 4 ? __builtin_amdgcn_readlane(p, 32) : pa;
-    const bool upper = NPL == 4 && (threadIdx.x & 63) >= 32;
-    const int c = blockIdx.y;
-    const int s0 = c * chunk;
-    const int s1 = min(depth, s0 + chunk);
-    float sm[NPL], cm[NPL];
+// Read-only data (written by earlier launches) at addresses that are the same
+// on every lane: scalar loads.
+typedef const __attribute__((address_space(4))) double* const_doubles;
+__device__ __forceinline__ const_doubles scalar_ptr(const double* p) { return (const_doubles)p; }
+
+// A problem's history sums of the step with history index n in a block that
+// starts at N0 (n - N0 < kHistBlock), for its elements e = r*nl + g < len
+// (r < CM; lanes past len repeat the last one): the far sums G (null: none),
+// then the slots N0 .. n - 1, oldest first.  w: the step's weight of slot n - 1
+// (the newest), ws: from a slot's weight to that of the one before it.
+template <typename HT, int CM>
+__device__ __forceinline__ void mt_sums(const HT* hist, int64_t ldh, int64_t hoff, int len, int N0,
+                                        int n, const double* G, const double* w, int ws, int g,
+                                        int nl, double (&hs)[CM]) {
+    const const_doubles wc = scalar_ptr(w);
+    int e[CM];
 #pragma unroll
-    for (int k = 0; k < NPL; ++k) sm[k] = cm[k] = 0.f;
-    if (live) {
-        const int64_t ldv = ldh / NPL;
-        const vt* q = reinterpret_cast<const vt*>(hist + (int64_t)s0 * ldh + j);
-        const float* wa = w + (int64_t)max(pa, 0) * ldw + (depth - 1 - s0);
-        const float* wb = w + (int64_t)max(pb, 0) * ldw + (depth - 1 - s0);
-        int s = s0;
-        for (; s + SL <= s1; s += SL) {
-            vt x[SL];
+    for (int r = 0; r < CM; ++r) e[r] = min(r * nl + g, len - 1);
 #pragma unroll
-            for (int u = 0; u < SL; ++u) x[u] = __builtin_nontemporal_load(q + (int64_t)u * ldv);
+    for (int r = 0; r < CM; ++r) hs[r] = G ? G[(int64_t)(n - N0) * ldh + hoff + e[r]] : 0.0;
+    constexpr int U = CM >= 16 ? 1 : 16 / CM;  // slots whose loads go out together
+    const HT* h = hist + hoff;
+    int s = N0;
+    for (; s + U <= n; s += U) {
+        HT x[U][CM];
 #pragma unroll
-            for (int u = 0; u < SL; ++u) {
-                const float wu = upper ? wb[-u] : wa[-u];
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-                for (int k = 0; k < NPL; ++k) kahan_add(sm[k], cm[k], wu * x[u][k]);
-            }
-            q += SL * ldv;
-            wa -= SL;
-            wb -= SL;
-        }
-        for (; s < s1; ++s) {
-            const vt x = __builtin_nontemporal_load(q);
-            const float wu = upper ? wb[0] : wa[0];
+            for (int r = 0; r < CM; ++r) x[u][r] = h[(int64_t)(s + u) * ldh + e[r]];
 #pragma unroll
-            for (int k = 0; k < NPL; ++k) kahan_add(sm[k], cm[k], wu * x[k]);
-            q += ldv;
-            wa -= 1;
-            wb -= 1;
+        for (int u = 0; u < U; ++u) {
+            const double v = wc[(n - 1 - s - u) * ws];
+#pragma unroll
+            for (int r = 0; r < CM; ++r) hs[r] = fma(v, (double)x[u][r], hs[r]);
         }
     }
-    if (in) {
+    for (; s < n; ++s) {
+        HT x[CM];
 #pragma unroll
-        for (int k = 0; k < NPL; ++k) part[(int64_t)c * ldh + j + k] = (double)sm[k] - (double)cm[k];
+        for (int r = 0; r < CM; ++r) x[r] = h[(int64_t)s * ldh + e[r]];
+        const double v = wc[(n - 1 - s) * ws];
+#pragma unroll
+        for (int r = 0; r < CM; ++r) hs[r] = fma(v, (double)x[r], hs[r]);
     }
 }
 
@@ -241,9 +274,8 @@ __device__ inline double psi_inv_der(double beta, double t, int n, double d) {
 
 // v_first = f'(gtj) gtj^(1-alpha), the series' first factor (the same for
 // every interval of a step)
-__device__ double psi_kb_row(double beta, double t0, double t1, double gtj, double alpha,
+__device__ double psi_kb_row(double beta, double gt0, double gt1, double gtj, double alpha,
                              double v_first) {
-    const double gt1 = pow(t1, beta), gt0 = pow(t0, beta);
     double sum = 0.0, i = 0.0;
     int niter = 0;
     double v = v_first;
@@ -268,17 +300,15 @@ __device__ double psi_kb_row(double beta, double t0, double t1, double gtj, doub
     return sum;
 }
 
-// gtj_na = gtj^-alpha (the same for every interval of a step)
-__device__ double psi_kb_row2(double beta, double t0, double t1, double gtj, double alpha,
-                              double gtj_na) {
-    const double gt0 = pow(t0, beta), gt1 = pow(t1, beta);
+// gtj_na = gtj^-alpha (the same for every interval of a step); v4_first: the
+// first derivative of the inverse at g(t1), which starts every term's inner
+// series (the same in every step)
+__device__ double psi_kb_row2(double beta, double t0, double t1, double gt0, double gt1, double gtj,
+                              double alpha, double gtj_na, double v4_first) {
     double sum = 0.0, v1 = 1.0, v2, v3, v4, v5, v6, v7, i = 0.0, m;
     int niter = 0;
     v2 = gtj_na * gt1;
     v6 = gt0 / gt1;
-    // the first derivative of the inverse at g(t1) starts every term's inner
-    // series; it depends on the interval only (three pow calls, made once)
-    const double v4_first = psi_inv_der(beta, gt1, 1, psi_inv_der(beta, gt1, 0, 0));
     const double ib = 1.0 / beta, rg = (gt0 - gt1) / gt1;
     do {
         if (i != 0.0) {
@@ -336,10 +366,28 @@ __device__ inline PsiStep psi_step(double alpha, double beta, int A, double tau)
     return q;
 }
 
-__device__ double psi_calc_int(double alpha, double beta, int a, int A, double tau, const PsiStep& q) {
+// g(a tau) and the inverse's first derivative there, per problem, a = 0 ..
+// gl - 1: the series' factors that depend on the interval only (five of the
+// up to nine pow calls of a weight), made once per solver.
+__global__ __launch_bounds__(256) void k_psi_tables(const MtProbDev* __restrict__ pr, int gl,
+                                                    double tau, double* __restrict__ g,
+                                                    double* __restrict__ dg) {
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a >= gl) return;
+    const double beta = pr[blockIdx.y].beta;
+    const double gt = pow(a * tau, beta);
+    g[(int64_t)blockIdx.y * gl + a] = gt;
+    dg[(int64_t)blockIdx.y * gl + a] = psi_inv_der(beta, gt, 1, psi_inv_der(beta, gt, 0, 0));
+}
+
+// g, dg: the problem's rows of k_psi_tables
+__device__ double psi_calc_int(double alpha, double beta, int a, int A, double tau,
+                               const double* __restrict__ g, const double* __restrict__ dg,
+                               const PsiStep& q) {
     if ((a + 1 <= 0.5 * A) && !(beta == 1))
-        return psi_kb_row2(beta, a * tau, (a + 1) * tau, q.gtj, alpha, q.gtj_na);
-    return psi_kb_row(beta, a * tau, (a + 1) * tau, q.gtj, alpha, q.v_first);
+        return psi_kb_row2(beta, a * tau, (a + 1) * tau, g[a], g[a + 1], q.gtj, alpha, q.gtj_na,
+                           dg[a + 1]);
+    return psi_kb_row(beta, g[a], g[a + 1], q.gtj, alpha, q.v_first);
 }
 
 // The reference's fallback where a series is not finite: _kb(1, t0, t1,
@@ -433,72 +481,92 @@ __device__ double psi_kb_quad(double beta, double t0, double t1, double gtj, boo
     }
 }
 
-// Stores the value of interval x of problem p at step k as a history weight
-// (x < depth) or the current-step factor d0.
-__device__ inline void psi_store(const MtProbDev& P, int p, int x, int depth, double v,
-                                 double* __restrict__ w, int ldw, float* __restrict__ w32,
-                                 double* __restrict__ d0) {
-    if (x < depth) {
-        const double wl = v * (1 - P.alpha);
-        const int l = depth - (x + 1);
-        w[(int64_t)p * ldw + l] = wl;
-        if (w32) w32[(int64_t)p * ldw + l] = (float)wl;
-    } else {
-        d0[p] = P.Da * v * (1 - P.alpha);
-    }
+// The weights of a block of steps (kind psi).  Step j of the block that starts
+// at history index N0 is k = N0 + j + 3; its weight of slot s < N0 + j is
+// (1-alpha) kb_time of interval s + 1, stored at w[(p*ldw + s)*kHistBlock + j],
+// and its current-step factor Da (1-alpha) kb_time[k] at d0[(j + 2)*nprob + p]
+// (j = -2, -1: the two steps before the first increment is stored).
+struct PsiArgs {
+    const MtProbDev* pr;
+    int nprob, N0, capacity;
+    double tau;
+    const double *g, *dg;  // k_psi_tables
+    int gl;
+    double* w;
+    int ldw;
+    double* d0;
+    int* bad;
+    int2* queue;           // (problem, slot * 32 + j, or -(j + 3) for a current-step factor)
+    int qcap;
+    int* qcount;           // [2] queue lengths, by the block's parity
+};
+
+__device__ inline void psi_store(const PsiArgs& a, const MtProbDev& P, int p, int s, int j,
+                                 double v) {
+    if (s >= 0)
+        a.w[((int64_t)p * a.ldw + s) * kHistBlock + j] = v * (1 - P.alpha);
+    else
+        a.d0[(int64_t)(j + 2) * a.nprob + p] = P.Da * v * (1 - P.alpha);
 }
 
-// Step k (= tstep): w[p*ldw + l] = (1-alpha) kb_time[depth-l] for l < depth
-// (depth = k-3 history terms) and d0[p] = Da (1-alpha) kb_time[k].
-// Thread x of row p handles interval a = x+1 (x < depth) or a = k (x = depth).
-__global__ void k_psi_weights(const MtProbDev* __restrict__ pr, int nprob, int k, int depth,
-                              double tau, double* __restrict__ w, int ldw, float* __restrict__ w32,
-                              double* __restrict__ d0, int* __restrict__ bad,
-                              int2* __restrict__ queue, int qcap, int* __restrict__ qcount) {
+// One workgroup: 16 slots x the block's 16 steps of one problem (grid row), a
+// lane per weight with the steps fastest, so that its stores are contiguous;
+// the last workgroup of a row: the current-step factors.
+__global__ __launch_bounds__(256) void k_psi_weights(PsiArgs a) {
+    constexpr int J = kHistBlock;
     const int p = blockIdx.y;
-    if (p >= nprob) return;  // the whole workgroup: one problem per grid row
-    const MtProbDev P = pr[p];
-    __shared__ PsiStep q;
-    if (threadIdx.x == 0) q = psi_step(P.alpha, P.beta, k + 1, tau);
+    const MtProbDev P = a.pr[p];
+    const bool cur = blockIdx.x == gridDim.x - 1;
+    __shared__ PsiStep q[J + 2];
+    const int j0 = cur && a.N0 == 0 ? -2 : 0;
+    if (threadIdx.x < J - j0)
+        q[threadIdx.x] = psi_step(P.alpha, P.beta, a.N0 + j0 + (int)threadIdx.x + 4, a.tau);
     __syncthreads();
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x > depth) return;
-    const int a = (x < depth) ? x + 1 : k;
-    const double v = psi_calc_int(P.alpha, P.beta, a, k + 1, tau, q);
+    int s = -1, j, k;
+    if (cur) {
+        j = j0 + (int)threadIdx.x;
+        k = a.N0 + j + 3;
+        if (j >= J || k > a.capacity) return;
+    } else {
+        s = blockIdx.x * 16 + threadIdx.x / J;
+        j = threadIdx.x % J;
+        k = a.N0 + j + 3;
+        if (s >= a.N0 + j || k > a.capacity) return;
+    }
+    const double* g = a.g + (int64_t)p * a.gl;
+    const double* dg = a.dg + (int64_t)p * a.gl;
+    const double v = psi_calc_int(P.alpha, P.beta, cur ? k : s + 1, k + 1, a.tau, g, dg, q[j - j0]);
     if (!isfinite(v)) {
         // calc_int falls back to _kb here: k_psi_quad computes and stores it
-        const int slot = atomicAdd(&qcount[k & 1], 1);
-        if (slot < qcap)
-            queue[slot] = make_int2(p, x);
+        const int slot = atomicAdd(&a.qcount[(a.N0 / J) & 1], 1);
+        if (slot < a.qcap)
+            a.queue[slot] = make_int2(p, cur ? -(j + 3) : s * 32 + j);
         else
-            atomicOr(bad, 4);
+            atomicOr(a.bad, 4);
         return;
     }
-    psi_store(P, p, x, depth, v, w, ldw, w32, d0);
+    psi_store(a, P, p, s, j, v);
 }
 
-// One thread per queued (problem, interval) whose series was not finite:
-// calc_int's _kb fallback, stored as k_psi_weights stores a weight.  A value
-// that is still not finite sets bad bit 1.  Workgroup 0 clears the queue
-// length that step k + 1 appends to (step k - 1's k_psi_quad, its last
-// reader, has finished).
-__global__ __launch_bounds__(64) void k_psi_quad(const MtProbDev* __restrict__ pr, int k,
-                                                 int depth, double tau, double* __restrict__ w,
-                                                 int ldw, float* __restrict__ w32,
-                                                 double* __restrict__ d0, int* __restrict__ bad,
-                                                 const int2* __restrict__ queue, int qcap,
-                                                 int* __restrict__ qcount) {
-    const int nq = min(qcount[k & 1], qcap);
+// One thread per queued weight whose series was not finite: calc_int's _kb
+// fallback, stored as k_psi_weights stores a weight.  A value that is still
+// not finite sets bad bit 1.  Workgroup 0 clears the queue length that the
+// next block appends to (the last reader of that one, the block before's
+// k_psi_quad, has finished).
+__global__ __launch_bounds__(64) void k_psi_quad(PsiArgs a) {
+    const int par = (a.N0 / kHistBlock) & 1;
+    const int nq = min(a.qcount[par], a.qcap);
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) qcount[(k + 1) & 1] = 0;
+    if (t == 0) a.qcount[par ^ 1] = 0;
     for (int q = t; q < nq; q += gridDim.x * blockDim.x) {
-        const int2 e = queue[q];
-        const MtProbDev P = pr[e.x];
-        const int a = (e.y < depth) ? e.y + 1 : k;
-        const double gtj = pow((k + 1) * tau, P.beta);
-        const double v = psi_kb_quad(P.beta, a * tau, (a + 1) * tau, gtj, a == k, P.alpha);
-        if (!isfinite(v)) atomicOr(bad, 1);
-        psi_store(P, e.x, e.y, depth, v, w, ldw, w32, d0);
+        const int2 e = a.queue[q];
+        const MtProbDev P = a.pr[e.x];
+        const int s = e.y < 0 ? -1 : e.y >> 5, j = e.y < 0 ? -e.y - 3 : e.y & 31;
+        const int k = a.N0 + j + 3, i = s < 0 ? k : s + 1;
+        const double gtj = pow((k + 1) * a.tau, P.beta);
+        const double v = psi_kb_quad(P.beta, i * a.tau, (i + 1) * a.tau, gtj, i == k, P.alpha);
+        if (!isfinite(v)) atomicOr(a.bad, 1);
+        psi_store(a, P, e.x, s, j, v);
     }
 }
 
@@ -509,185 +577,292 @@ __global__ void k_diag_psi_kb_quad(const double* __restrict__ c, int n, double* 
     out[i] = psi_kb_quad(r[1], r[2], r[3], r[4], r[5] != 0.0, r[0]);
 }
 
-// ---------------------------------------------------------------- sweep
-struct MtSweepArgs {
+// ---------------------------------------------------------------- steps
+struct MtStepArgs {
     const MtProbDev* pr;
-    int nprob;
+    const int* order;  // problems, largest first
     double* U;
-    const double* part;
-    int nch;
+    void* hist;
     int64_t ldh;
-    const double* d0;
-    void* slot;  // history slot for the new increment, or null
-    int slot_f32;
+    const double* G;   // the block's far sums (null: no settled slots)
+    const double* w;   // weights, as k_mt_far takes them
+    int ldw;
+    const double* d0;  // per problem, or (kind psi, TAB) the block's table
+    int nprob;
+    int N0;            // the block's start (history index)
+    int k0, ks;        // steps k0 .. k0 + ks - 1, all of one block
     int picard;
 };
 
-// CM = 16 (problems of up to 1024 nodes) is held to 256 registers, two
-// wavefronts per SIMD: one problem per wavefront leaves few wavefronts to
-// hide the scans' latency, and at 290 registers (one per SIMD) the 4096
-// problems of the psi batch ran in four rounds (0.83 s over 3000 steps
-// against 0.61 s with a small spill).
+// A problem's line lies in LDS with one pad double per chunk of CM elements
+// (element e at e + e/CM): lanes reading their chunks, and lanes reading
+// consecutive elements, both spread over the banks.
 template <int CM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CM == 16 ? 2 : 1, 8))) void k_mt_sweep(MtSweepArgs a) {
-    __shared__ double xs_all[4][64 * CM + 3];  // nodes 0..N+1, N - 1 <= 64*CM
-    const int wv = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int p = blockIdx.x * 4 + wv;
-    if (p >= a.nprob) return;
-    double* xs = xs_all[wv];
-    const MtProbDev P = a.pr[p];
-    const int N = P.N, n = N - 1, e0 = lane * CM;
+__device__ __forceinline__ int pad_at(int e) {
+    return e + e / CM;
+}
+
+// What the wavefronts of a problem tell each other.
+struct MtShare {
+    double Kf[kMtMaxW], Ke[kMtMaxW];  // first and last conductivity of a wavefront
+    Mob m[kMtMaxW];                   // alpha maps
+    double fP[kMtMaxW], fQ[kMtMaxW], bP[kMtMaxW], bQ[kMtMaxW];  // beta and back maps
+    double un, x0;
+    double es[kMtMaxW];               // kind AB: squared errors
+};
+
+// Runs steps a.k0 .. a.k0 + a.ks - 1 of problem p on W wavefronts of one
+// workgroup (64 W CM >= its unknowns).  State, history sums and increments are
+// handled in element order (consecutive lanes, consecutive nodes), the Thomas
+// recurrences in chunk order (CM consecutive elements per lane); X holds the
+// current iterate's interior nodes, Y the Picard-independent part of the
+// right-hand side.  The conductivity is evaluated once per node and exchanged
+// with the neighbouring lane; a constant matrix (FORM_CONST, L1) is factored
+// once per launch.
+template <int CM, typename HT, bool TAB>
+__device__ __forceinline__ void mt_steps(const MtStepArgs& a, int p, int W, double* X, double* Y,
+                                         MtShare& sh) {
+    const int lane = threadIdx.x & 63, wl = same_on_lanes((int)(threadIdx.x >> 6));
+    const MtProbDev P = same_on_lanes(a.pr[p]);
+    const int N = P.N, n = N - 1;
+    const int g = threadIdx.x, nl = 64 * W, e0 = g * CM, last = (n - 1) / CM;
     double* Ug = a.U + P.uoff;
-    {
-        // N + 2 <= 64 CM + 3 nodes: CM + 1 loads per lane, all in flight
-        double ux[CM + 1];
+    HT* hist = static_cast<HT*>(a.hist);
+    double u[CM];
 #pragma unroll
-        for (int r = 0; r <= CM; ++r) ux[r] = Ug[min(lane + 64 * r, N + 1)];
+    for (int r = 0; r < CM; ++r) u[r] = Ug[min(r * nl + g, n - 1) + 1];
+    double xN = Ug[N];
+    if (g == 0) sh.x0 = Ug[0];
 #pragma unroll
-        for (int r = 0; r <= CM; ++r)
-            if (lane + 64 * r < N + 2) xs[lane + 64 * r] = ux[r];
+    for (int r = 0; r < CM; ++r)
+        if (r * nl + g < n) X[pad_at<CM>(r * nl + g)] = u[r];
+    const bool fixed = P.form == FRM_FORM_CONST && !TAB;
+    bool factored = false;
+    const double idL = 1.0 / P.dL;
+    double A[CM], f[CM], al[CM];
+    if constexpr (!TAB) {
+#pragma unroll
+        for (int k = 0; k < CM; ++k) A[k] = f[k] = al[k] = 0.0;
     }
-    double u0[CM], hs[CM];
-    chunk_sums<CM>(a.part, a.ldh, a.nch, P.hoff, e0, n, hs);
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    for (int st = 0; st < a.ks; ++st) {
+        const int step = a.k0 + st, h = step - 3;  // history index: slot h is this step's
+        double d0, hs[CM];
+        if constexpr (TAB) {
+            const int j = h - a.N0;
+            d0 = scalar_ptr(a.d0)[(int64_t)(j + 2) * a.nprob + p];
+            if (h > 0)
+                mt_sums<HT, CM>(hist, a.ldh, P.hoff, n, a.N0, h, a.G,
+                                a.w + ((int64_t)p * a.ldw + h - 1) * kHistBlock + j, -kHistBlock, g,
+                                nl, hs);
+        } else {
+            d0 = scalar_ptr(a.d0)[p];
+            if (h > 0)
+                mt_sums<HT, CM>(hist, a.ldh, P.hoff, n, a.N0, h, a.G, a.w + (int64_t)p * a.ldw, 1, g,
+                                nl, hs);
+        }
 #pragma unroll
-    for (int k = 0; k < CM; ++k) {
-        const int e = e0 + k;
-        u0[k] = 0.0;
-        if (e < n) u0[k] = xs[e + 1];
-    }
-    const double d0 = a.d0[p];
-    for (int it = 0; it < a.picard; ++it) {
-        double A[CM], B[CM], R[CM], om[CM];
-#pragma unroll
-        for (int k = 0; k < CM; ++k) {
-            const int e = e0 + k;
-            if (e < n) {
-                const int i = e + 1;
-                const double inv = mt_inv(P, xs[i]);
-                const double Km = mt_KK(P, xs[i - 1]), K0 = mt_KK(P, xs[i]), Kp = mt_KK(P, xs[i + 1]);
-                A[k] = P.Dg * Km * inv;
-                B[k] = P.Dg * Kp * inv;
-                R[k] = inv * (Kp + Km) * P.Dg + d0;
-                double o = -d0 * u0[k];
-                o += (K0 - Km) / P.dL;
-                o += P.Da * hs[k];
-                om[k] = o;
+        for (int r = 0; r < CM; ++r) {
+            const int e = r * nl + g;
+            double o = -d0 * u[r];
+            if (h > 0) o += P.Da * hs[r];
+            if (e < n) Y[pad_at<CM>(e)] = o;
+        }
+        for (int it = 0; it < a.picard; ++it) {
+            __syncthreads();  // X, Y and x0 are in
+            const double x0 = sh.x0;
+            // top boundary: al1 / bt1 (mt_minimal.cpp:831-834, 944-947)
+            int first_order;
+            if (P.top == FRM_TOP_DIRICHLET) first_order = 0;
+            else if (P.top == FRM_TOP_FLUX) first_order = 1;
+            else first_order = (mt_inv(P, x0) != 1e20);
+            const double al_first = first_order ? 1.0 : 0.0;
+            double b0;
+            if (P.top == FRM_TOP_DIRICHLET) {
+                b0 = P.top_val;
             } else {
-                A[k] = 0.0;
-                B[k] = 1.0;
-                R[k] = 1.0;
-                om[k] = 0.0;
+                const double Uc = 1.0 * P.dL * (P.Ev - 0.0) / mt_KK(P, x0);
+                b0 = first_order ? -Uc : -Uc * mt_KK(P, X[0]) / P.dL;
             }
-        }
-        // top boundary: al1 / bt1 (mt_minimal.cpp:831-834, 944-947)
-        const double x0 = xs[0];
-        int first_order;
-        if (P.top == FRM_TOP_DIRICHLET) first_order = 0;
-        else if (P.top == FRM_TOP_FLUX) first_order = 1;
-        else first_order = (mt_inv(P, x0) != 1e20);
-        const double al_first = first_order ? 1.0 : 0.0;
-        const double Uc = 1.0 * P.dL * (P.Ev - 0.0) / mt_KK(P, x0);
-        double b0;
-        if (P.top == FRM_TOP_DIRICHLET) b0 = P.top_val;
-        else if (first_order) b0 = -Uc;
-        else b0 = -Uc * mt_KK(P, xs[1]) / P.dL;
-        // alpha: Al[i+1] = B/(R - A Al[i]), a Moebius map of Al
-        Mob m{1.0, 0.0, 0.0, 1.0};
+            double om[CM];
+            if constexpr (TAB) {
 #pragma unroll
-        for (int k = 0; k < CM; ++k)
-            if (e0 + k < n) m = mob_mul(Mob{0.0, B[k], -A[k], R[k]}, m);
-        const Mob pre = scan_mob_up(m, lane);
-        double al = (pre.m00 * al_first + pre.m01) / (pre.m10 * al_first + pre.m11);
-#pragma unroll
-        for (int k = 0; k < CM; ++k) {
-            if (e0 + k < n) {
-                al = B[k] / (R[k] - A[k] * al);
-                R[k] = al;  // R now holds Al[i+1]
+                for (int k = 0; k < CM; ++k) A[k] = f[k] = al[k] = 0.0;
             }
-        }
-        // beta: Bt[i+1] = (Al[i+1]/B)(A Bt[i] - Om)
-        double Pp = 1.0, Qq = 0.0;
 #pragma unroll
-        for (int k = 0; k < CM; ++k) {
-            if (e0 + k < n) {
-                const double pk = R[k] * A[k] / B[k], qk = -R[k] * om[k] / B[k];
-                Qq = pk * Qq + qk;
-                Pp = pk * Pp;
+            for (int k = 0; k < CM; ++k) om[k] = e0 + k < n ? Y[g * (CM + 1) + k] : 0.0;
+            const double xp = X[pad_at<CM>(n - 1)];  // U_{N-1} of the last iterate
+            if (!(fixed && factored)) {
+                // A, B, R of al1 (B in f, R in al until the recurrence); the
+                // conductivity slides along the chunk, its ends come from
+                // the neighbouring lanes and wavefronts
+                const int el = min(e0 + CM, n) - 1 - e0;  // the chunk's last element
+                const double* xc = X + g * (CM + 1);
+                const double Kf = mt_KK(P, xc[0]), Ke = mt_KK(P, xc[max(el, 0)]);
+                double Km = __shfl_up(Ke, 1), Kr = __shfl_down(Kf, 1);
+                if (W > 1) {
+                    if (lane == 0) sh.Kf[wl] = Kf;
+                    if (lane == 63) sh.Ke[wl] = Ke;
+                    __syncthreads();
+                    if (lane == 0 && wl > 0) Km = sh.Ke[wl - 1];
+                    if (lane == 63 && wl < W - 1) Kr = sh.Kf[wl + 1];
+                }
+                const double K0 = mt_KK(P, x0), KN = mt_KK(P, xN);
+                if (g == 0) Km = K0;
+                if (g == last) Kr = KN;
+                Mob m{1.0, 0.0, 0.0, 1.0};
+                double Kc = Kf;
+#pragma unroll
+                for (int k = 0; k < CM; ++k) {
+                    double Kp = Kr;
+                    if (k < CM - 1 && k < el) Kp = k + 1 == el ? Ke : mt_KK(P, xc[k + 1]);
+                    if (e0 + k < n) {
+                        const double inv = mt_inv(P, xc[k]);
+                        A[k] = P.Dg * Km * inv;
+                        f[k] = P.Dg * Kp * inv;
+                        al[k] = inv * (Kp + Km) * P.Dg + d0;
+                        om[k] += (Kc - Km) * idL;
+                        // alpha: Al[i+1] = B/(R - A Al[i]), a Moebius map of
+                        // Al: [[0, B], [-A, R]] times the product so far
+                        const double t0 = f[k] * m.m10, t1 = f[k] * m.m11;
+                        m.m10 = al[k] * m.m10 - A[k] * m.m00;
+                        m.m11 = al[k] * m.m11 - A[k] * m.m01;
+                        m.m00 = t0;
+                        m.m01 = t1;
+                    }
+                    Km = Kc;
+                    Kc = Kp;
+                    if (k % 4 == 3) m = mob_scale(m);
+                }
+                Mob tot;
+                const Mob pre = scan_mob_up_total(m, lane, tot);
+                double ya = al_first, yb = 1.0;  // Al entering the wavefront, as a quotient
+                if (W > 1) {
+                    if (lane == 0) sh.m[wl] = tot;
+                    __syncthreads();
+                    for (int w = 0; w < wl; ++w) {
+                        const Mob q = sh.m[w];
+                        const double t = q.m00 * ya + q.m01 * yb;
+                        yb = q.m10 * ya + q.m11 * yb;
+                        ya = t;
+                    }
+                }
+                double y = (pre.m00 * ya + pre.m01 * yb) / (pre.m10 * ya + pre.m11 * yb);
+#pragma unroll
+                for (int k = 0; k < CM; ++k) {
+                    if (e0 + k < n) {
+                        const double den = 1.0 / (al[k] - A[k] * y);
+                        y = f[k] * den;
+                        al[k] = y;   // Al[i+1]
+                        f[k] = den;  // Al[i+1] / B
+                    }
+                }
+                factored = true;
             }
-        }
-        scan_affine_up(Pp, Qq, lane);
-        double bt = Pp * b0 + Qq;
+            // beta: Bt[i+1] = (Al[i+1]/B)(A Bt[i] - Om)
+            double Pp = 1.0, Qq = 0.0, Pt, Qt;
 #pragma unroll
-        for (int k = 0; k < CM; ++k) {
-            if (e0 + k < n) {
-                bt = (R[k] / B[k]) * (A[k] * bt - om[k]);
-                om[k] = bt;  // om now holds Bt[i+1]
+            for (int k = 0; k < CM; ++k) {
+                if (e0 + k < n) {
+                    const double pk = f[k] * A[k], qk = -f[k] * om[k];
+                    Qq = pk * Qq + qk;
+                    Pp = pk * Pp;
+                }
             }
-        }
-        // bottom boundary (mt_minimal.cpp:987-1020), gamma = 1 so Qb = -0
-        const int last = (n - 1) / CM;
-        double UN_l = 0.0;
-#pragma unroll
-        for (int k = 0; k < CM; ++k) {
-            if (e0 + k == n - 1) {
-                const double BtN = om[k], AlN = R[k], Qb = -0.0;
-                if (P.bottom_cond == 1)
-                    UN_l = P.Hbottom;
-                else if (fabs(BtN + Qb) > 1e-15)
-                    UN_l = (fabs(1.0 - AlN) > 1e-15) ? (BtN + Qb) / (1.0 - AlN) : xs[N - 1] + Qb;
-                else
-                    UN_l = (fabs(1.0 - AlN) > 1e-15) ? 0.0 : xs[N - 1] + Qb;
+            scan_affine_up_total(Pp, Qq, lane, Pt, Qt);
+            double bt = b0;  // value entering the wavefront
+            if (W > 1) {
+                if (lane == 0) {
+                    sh.fP[wl] = Pt;
+                    sh.fQ[wl] = Qt;
+                }
+                __syncthreads();
+                for (int w = 0; w < wl; ++w) bt = sh.fP[w] * bt + sh.fQ[w];
             }
-        }
-        const double UN = __shfl(UN_l, last);
-        // back substitution U_i = Al[i+1] U_{i+1} + Bt[i+1]
-        Pp = 1.0;
-        Qq = 0.0;
+            bt = Pp * bt + Qq;
 #pragma unroll
-        for (int k = CM - 1; k >= 0; --k) {
-            if (e0 + k < n) {
-                Qq = R[k] * Qq + om[k];
-                Pp = R[k] * Pp;
+            for (int k = 0; k < CM; ++k) {
+                if (e0 + k < n) {
+                    bt = f[k] * (A[k] * bt - om[k]);
+                    om[k] = bt;  // om now holds Bt[i+1]
+                }
             }
-        }
-        scan_affine_down(Pp, Qq, lane);
-        double y = Pp * UN + Qq;
-        double v[CM];
+            // bottom boundary (mt_minimal.cpp:987-1020), gamma = 1 so Qb = -0
 #pragma unroll
-        for (int k = CM - 1; k >= 0; --k) {
-            v[k] = 0.0;
-            if (e0 + k < n) {
-                y = R[k] * y + om[k];
-                v[k] = y;
+            for (int k = 0; k < CM; ++k) {
+                if (e0 + k == n - 1) {
+                    const double BtN = om[k], AlN = al[k], Qb = -0.0;
+                    double UN;
+                    if (P.bottom_cond == 1)
+                        UN = P.Hbottom;
+                    else if (fabs(BtN + Qb) > 1e-15)
+                        UN = (fabs(1.0 - AlN) > 1e-15) ? (BtN + Qb) / (1.0 - AlN) : xp + Qb;
+                    else
+                        UN = (fabs(1.0 - AlN) > 1e-15) ? 0.0 : xp + Qb;
+                    sh.un = UN;
+                }
             }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            // back substitution U_i = Al[i+1] U_{i+1} + Bt[i+1]
+            Pp = 1.0;
+            Qq = 0.0;
 #pragma unroll
-        for (int k = 0; k < CM; ++k)
-            if (e0 + k < n) xs[e0 + k + 1] = v[k];
-        if (lane == 0) {
-            xs[0] = al_first * v[0] + b0;
-            xs[N] = UN;
-            xs[N + 1] = UN;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    }
-    for (int q = lane; q < N + 2; q += 64) Ug[q] = xs[q];
-    if (a.slot) {
+            for (int k = CM - 1; k >= 0; --k) {
+                if (e0 + k < n) {
+                    Qq = al[k] * Qq + om[k];
+                    Pp = al[k] * Pp;
+                }
+            }
+            scan_affine_down_total(Pp, Qq, lane, Pt, Qt);
+            if (lane == 0) {
+                sh.bP[wl] = Pt;
+                sh.bQ[wl] = Qt;
+            }
+            __syncthreads();
+            xN = sh.un;
+            double y = xN;
+            for (int w = W - 1; w > wl; --w) y = sh.bP[w] * y + sh.bQ[w];
+            y = Pp * y + Qq;
 #pragma unroll
-        for (int k = 0; k < CM; ++k) {
-            const int e = e0 + k;
+            for (int k = CM - 1; k >= 0; --k) {
+                if (e0 + k < n) {
+                    y = al[k] * y + om[k];
+                    X[g * (CM + 1) + k] = y;
+                }
+            }
+            if (g == 0) sh.x0 = al_first * y + b0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < CM; ++r) {
+            const int e = r * nl + g;
             if (e < n) {
-                const double d = xs[e + 1] - u0[k];
-                if (a.slot_f32)
-                    static_cast<float*>(a.slot)[P.hoff + e] = (float)d;
-                else
-                    static_cast<double*>(a.slot)[P.hoff + e] = d;
+                const double v = X[pad_at<CM>(e)];
+                if (h >= 0) hist[(int64_t)h * a.ldh + P.hoff + e] = (HT)(v - u[r]);
+                u[r] = v;
             }
         }
     }
+#pragma unroll
+    for (int r = 0; r < CM; ++r)
+        if (r * nl + g < n) Ug[r * nl + g + 1] = u[r];
+    if (g == 0) {
+        Ug[0] = sh.x0;
+        Ug[N] = xN;
+        Ug[N + 1] = xN;
+    }
+}
+
+// One workgroup per problem, a wavefront per 64 kMtCM of the largest problem's
+// unknowns; wavefronts that a smaller problem does not need leave at once, and
+// a workgroup's place is free as soon as its own problem is done.
+template <typename HT, bool TAB>
+__global__ __launch_bounds__(64 * kMtMaxW) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_mt_steps(MtStepArgs a) {
+    constexpr int CM = kMtCM;
+    __shared__ double X[64 * kMtMaxW * (CM + 1)], Y[64 * kMtMaxW * (CM + 1)];
+    __shared__ MtShare sh;
+    const int p = same_on_lanes(a.order[blockIdx.x]);
+    const int W = (same_on_lanes(a.pr[p].N) - 1 + 64 * CM - 1) / (64 * CM);
+    if ((int)(threadIdx.x >> 6) >= W) return;
+    mt_steps<CM, HT, TAB>(a, p, W, X, Y, sh);
 }
 
 // ---------------------------------------------------------------- AB kind
@@ -702,95 +877,199 @@ __host__ __device__ inline double ab_CC(int F, double x, double t) {
     return 0.0;
 }
 
-__device__ inline double ab_f(int F, double x, double t, double a, double E) {
+// sp, cp: sin and cos of pi x (F = 2 only; the same in every step)
+__device__ inline double ab_f(int F, double x, double t, double a, double E, double sp, double cp) {
     if (F == 0) return (24.0 / (1.0 - a)) * t * t * t * t * E;
     if (F == 1) return (2.0 * x - 1.0) * t * t - 2 * t * t + (2.0 / (1.0 - a)) * x * (x - 1.0) * t * t * E;
     if (F == 2)
-        return (120.0 / (1.0 - a)) * t * t * t * t * t * sin(kAbPi * x) * E +
-               kAbPi * t * t * t * t * t * (kAbPi * sin(kAbPi * x) + cos(kAbPi * x));
+        return (120.0 / (1.0 - a)) * t * t * t * t * t * sp * E +
+               kAbPi * t * t * t * t * t * (kAbPi * sp + cp);
     return 0.0;
 }
 
-struct AbSweepArgs {
+__device__ inline double ab_CC_in(int F, double x, double t, double sp) {
+    return F == 2 ? t * t * t * t * t * sp : ab_CC(F, x, t);
+}
+
+struct AbStepArgs {
     const MtProbDev* pr;
-    int nprob;
+    const int* order;    // problems, largest first
     double* U;
-    const double* part;  // history sums sum_k I(lag+1) (C^{k+1}-C^k)/tau, [nch][ldh];
-                         // series problems: MF_intF_choice's value in row 0
-    int nch;
+    double* hist;        // slot k - 1 takes step k's (C^k - C^{k-1})/tau
     int64_t ldh;
+    const double* G;     // the block's far sums (null: no settled slots)
+    const double* w;     // lag-indexed I(lag+1) per problem
+    int ldw;
     const double* d0;    // I(1)/(1-alpha) per problem
     const double* cf;    // per history node: -1/(B - A Al_{j-1})
     const double* cal;   // per history node: -Al_j
     const double* ml;    // [nprob][ldml] source factor at step k
     int ldml;
-    int k;               // step being taken (1-based), t = k tau
+    const double* ser;   // series problems: MF_intF_choice's value per history node
+    int N0;              // the block's start (history index)
+    int k0, ks;          // steps k0 .. k0 + ks - 1, t = k tau; ks = 1 with series problems
     double tau;
-    double* slot;        // history slot for (C^k - C^{k-1})/tau
     double* err;         // per problem: running sum of (C_j - CC)^2
 };
 
-// One wavefront per problem: right-hand side Rp_j = I(1)/(1-a) C_j + f -
-// history/(1-a) (MF_int_series.cpp:922-931), the Thomas sweep with the
-// exact Dirichlet ends (935-945) through the scan-seeded line solve (the
-// constant alpha recurrence is precomputed), the increment push and the
-// squared error against CC (947-951).
+// Steps a.k0 .. of problem p on W wavefronts of one workgroup: right-hand side
+// Rp_j = I(1)/(1-a) C_j + f - history/(1-a) (MF_int_series.cpp:922-931), the
+// Thomas sweep with the exact Dirichlet ends (935-945) through the scan-seeded
+// line solve (the constant alpha recurrence is precomputed), the increment
+// push and the squared error against CC (947-951).  Everything but the
+// recurrences runs in element order; the source's sines are taken once per
+// launch.
 template <int CM>
-__global__ __launch_bounds__(256) void k_ab1d_sweep(AbSweepArgs a) {
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int p = blockIdx.x * 4 + wv;
-    if (p >= a.nprob) return;  // whole wavefront; the kernel has no block barrier
-    const MtProbDev P = a.pr[p];
-    const int m = P.N, n = m - 1, e0 = lane * CM;
-    const double h = P.dL, al = P.alpha;
-    const double t = a.k * a.tau;
-    const double E = a.ml[(int64_t)p * a.ldml + (a.k - 1)];
-    const double Ii1a = a.d0[p];
+__device__ __forceinline__ void ab_steps(const AbStepArgs& a, int p, int W, double* X, MtShare& sh) {
+    const int lane = threadIdx.x & 63, wl = same_on_lanes((int)(threadIdx.x >> 6));
+    const MtProbDev P = same_on_lanes(a.pr[p]);
+    const int m = P.N, n = m - 1;
+    const int g = threadIdx.x, nl = 64 * W, e0 = g * CM;
+    const double h = P.dL, alpha = P.alpha, i1a = 1.0 / (1.0 - alpha), Ii1a = scalar_ptr(a.d0)[p];
     const double A = -(1.0 / (h * h)) - (1.0 / (2.0 * h));
     double* C = a.U + P.uoff;
-    double ca[CM], cf[CM], cal[CM], v[CM], c0[CM], hs[CM];
-    chunk_sums<CM>(a.part, a.ldh, (a.k >= 2 && !P.ser) ? a.nch : 0, P.hoff, e0, n, hs);
+    double c0[CM], sp[CM], cp[CM];
+#pragma unroll
+    for (int r = 0; r < CM; ++r) {
+        const int e = min(r * nl + g, n - 1);
+        c0[r] = C[e + 1];
+        sp[r] = cp[r] = 0.0;
+        if (P.src == 2) {
+            sp[r] = sinpi((e + 1) * h);
+            cp[r] = cospi((e + 1) * h);
+        }
+    }
+    double cf[CM], cal[CM];
 #pragma unroll
     for (int k = 0; k < CM; ++k) {
-        const int e = e0 + k;
-        ca[k] = cf[k] = cal[k] = v[k] = c0[k] = 0.0;
-        if (e < n) {
-            const int j = e + 1;
-            c0[k] = C[j];
-            double rp = Ii1a * c0[k] + ab_f(P.src, j * h, t, al, E);
-            if (a.k >= 2) {
-                if (P.ser)  // MF_intF_choice's value, already over (1 - a)
-                    rp -= a.part[P.hoff + e];
-                else
-                    rp -= hs[k] / (1.0 - al);
+        const int e = min(e0 + k, n - 1);
+        cf[k] = a.cf[P.hoff + e];
+        cal[k] = a.cal[P.hoff + e];
+    }
+    double es = a.err[p], b0 = 0.0, un = 0.0;
+    for (int st = 0; st < a.ks; ++st) {
+        const int step = a.k0 + st, hi = step - 1;  // history index: slot hi is this step's
+        const double t = step * a.tau;
+        const double E = scalar_ptr(a.ml)[(int64_t)p * a.ldml + hi];
+        double hs[CM];
+        if (hi > 0) {
+            if (P.ser) {  // MF_intF_choice's value, already over (1 - a)
+#pragma unroll
+                for (int r = 0; r < CM; ++r) hs[r] = a.ser[P.hoff + min(r * nl + g, n - 1)];
+            } else {
+                mt_sums<double, CM>(a.hist, a.ldh, P.hoff, n, a.N0, hi, a.G, a.w + (int64_t)p * a.ldw,
+                                    1, g, nl, hs);
+#pragma unroll
+                for (int r = 0; r < CM; ++r) hs[r] *= i1a;
             }
-            v[k] = rp;
-            ca[k] = A;
-            cf[k] = a.cf[P.hoff + e];
-            cal[k] = a.cal[P.hoff + e];
         }
-    }
-    const double b0 = ab_CC(P.src, 0.0, t), un = ab_CC(P.src, m * h, t);
-    line_solve<CM>(ca, cf, cal, v, e0, n, b0, lane, &un);
-    double es = 0.0;
 #pragma unroll
-    for (int k = 0; k < CM; ++k) {
-        const int e = e0 + k;
-        if (e < n) {
-            const int j = e + 1;
-            C[j] = v[k];
-            if (a.slot) a.slot[P.hoff + e] = (v[k] - c0[k]) / a.tau;
-            const double d = fabs(v[k] - ab_CC(P.src, h * j, t));
-            es += d * d;
+        for (int r = 0; r < CM; ++r) {
+            const int e = r * nl + g;
+            double rp = Ii1a * c0[r] + ab_f(P.src, (e + 1) * h, t, alpha, E, sp[r], cp[r]);
+            if (hi > 0) rp -= hs[r];
+            if (e < n) X[pad_at<CM>(e)] = rp;
         }
+        __syncthreads();
+        b0 = ab_CC(P.src, 0.0, t);
+        un = ab_CC(P.src, m * h, t);
+        double v[CM], Pp = 1.0, Qq = 0.0, Pt, Qt;
+#pragma unroll
+        for (int k = 0; k < CM; ++k) v[k] = e0 + k < n ? X[g * (CM + 1) + k] : 0.0;
+#pragma unroll
+        for (int k = 0; k < CM; ++k) {
+            if (e0 + k < n) {
+                const double pk = cf[k] * A, qk = -cf[k] * v[k];
+                Qq = pk * Qq + qk;
+                Pp = pk * Pp;
+            }
+        }
+        scan_affine_up_total(Pp, Qq, lane, Pt, Qt);
+        double y = b0;  // value entering the wavefront
+        if (W > 1) {
+            if (lane == 0) {
+                sh.fP[wl] = Pt;
+                sh.fQ[wl] = Qt;
+            }
+            __syncthreads();
+            for (int w = 0; w < wl; ++w) y = sh.fP[w] * y + sh.fQ[w];
+        }
+        y = Pp * y + Qq;
+#pragma unroll
+        for (int k = 0; k < CM; ++k) {
+            if (e0 + k < n) {
+                y = cf[k] * (A * y - v[k]);
+                v[k] = y;
+            }
+        }
+        Pp = 1.0;
+        Qq = 0.0;
+#pragma unroll
+        for (int k = CM - 1; k >= 0; --k) {
+            if (e0 + k < n) {
+                Qq = cal[k] * Qq + v[k];
+                Pp = cal[k] * Pp;
+            }
+        }
+        scan_affine_down_total(Pp, Qq, lane, Pt, Qt);
+        y = un;
+        if (W > 1) {
+            if (lane == 0) {
+                sh.bP[wl] = Pt;
+                sh.bQ[wl] = Qt;
+            }
+            __syncthreads();
+            for (int w = W - 1; w > wl; --w) y = sh.bP[w] * y + sh.bQ[w];
+        }
+        y = Pp * y + Qq;
+#pragma unroll
+        for (int k = CM - 1; k >= 0; --k) {
+            if (e0 + k < n) {
+                y = cal[k] * y + v[k];
+                X[g * (CM + 1) + k] = y;
+            }
+        }
+        __syncthreads();
+        double d2 = 0.0;
+#pragma unroll
+        for (int r = 0; r < CM; ++r) {
+            const int e = r * nl + g;
+            if (e < n) {
+                const double c = X[pad_at<CM>(e)];
+                a.hist[(int64_t)hi * a.ldh + P.hoff + e] = (c - c0[r]) / a.tau;
+                c0[r] = c;
+                const double d = fabs(c - ab_CC_in(P.src, h * (e + 1), t, sp[r]));
+                d2 += d * d;
+            }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) d2 += __shfl_xor(d2, o);
+        if (W > 1) {
+            if (lane == 0) sh.es[wl] = d2;
+            __syncthreads();
+            d2 = sh.es[0];
+            for (int w = 1; w < W; ++w) d2 += sh.es[w];
+        }
+        es += d2;  // the two ends equal CC exactly
     }
-    if (lane == 0) {
+#pragma unroll
+    for (int r = 0; r < CM; ++r)
+        if (r * nl + g < n) C[r * nl + g + 1] = c0[r];
+    if (g == 0) {
         C[0] = b0;  // bt[0] - al[0] C[1] with al[0] = 0
         C[m] = un;
+        a.err[p] = es;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) es += __shfl_xor(es, o);
-    if (lane == 0) a.err[p] += es;  // the two ends equal CC exactly
+}
+
+__global__ __launch_bounds__(64 * kMtMaxW) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_ab_steps(AbStepArgs a) {
+    constexpr int CM = kMtCM;
+    __shared__ double X[64 * kMtMaxW * (CM + 1)];
+    __shared__ MtShare sh;
+    const int p = same_on_lanes(a.order[blockIdx.x]);
+    const int W = (same_on_lanes(a.pr[p].N) - 1 + 64 * CM - 1) / (64 * CM);
+    if ((int)(threadIdx.x >> 6) >= W) return;
+    ab_steps<CM>(a, p, W, X, sh);
 }
 
 // ---------------------------------------------------------------- AB series history
@@ -1088,8 +1367,8 @@ namespace frm {
 struct KRec {
     const void* func = nullptr;
     dim3 grid, block;
-    int step = 0;         // step of the recorded run it belongs to
     bool branch = false;  // weights formed ahead (kind psi): a branch of the graph
+    bool join = false;    // the first launch that reads weights formed on the branch
     alignas(16) unsigned char buf[448];
     size_t used = 0;
     size_t off[16];
@@ -1107,14 +1386,14 @@ struct KRec {
     }
 };
 // The launches of up to kGraphSteps consecutive steps as an instantiated
-// graph (each step's kernel nodes in a chain; for kind psi the next step's
-// weights on a branch beside it), reused for every run of steps that issues
-// the same kernels in the same order: only the nodes' arguments and grids
-// change between launches.
+// graph (kernel nodes in a chain; for kind psi the next block's weights on a
+// branch beside it), reused for every run of steps that issues the same
+// kernels in the same order: only the nodes' arguments and grids change
+// between launches.
 constexpr int kGraphSteps = 32;
 struct StepGraph {
     std::vector<const void*> funcs;
-    std::vector<int> tags;  // step * 2 + branch of every node
+    std::vector<int> tags;  // join * 2 + branch of every node
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     std::vector<hipGraphNode_t> nodes;
@@ -1134,28 +1413,32 @@ struct frm_mt1d {
     MtProbDev* probs = nullptr;
     int* gprob = nullptr;
     int* gvalid = nullptr;    // real nodes per group (0 for padding groups)
-    int min_chunk = kMinChunk;      // history block length: shortest time chunk of the memory term
+    int* order = nullptr;     // problems by size, largest first
+    int min_chunk = 32;       // fewest slots a wavefront of a split far pass takes
     int graph = 0;                  // steps as HIP graphs, built once per launch sequence
     std::vector<frm::StepGraph> graphs;  // one instantiated graph per launch sequence
     std::vector<frm::KRec>* rec = nullptr;  // while set, launches are recorded, not issued
-    int rec_step = 0;                        // step of the recorded run being recorded
+    bool rec_join = false;                   // the next launch waits for the branch
     hipStream_t lstream = nullptr;          // while set, launches go to this stream
-    // kind psi: the weights of step k + 1 are formed on the context's second
-    // stream while step k's memory term and sweep run on its stream (the
-    // weights do not depend on the state); w, w32 and d0 then hold two
-    // buffers, step k using buffer k & 1.  wready[b]: buffer b's weights are
-    // formed; wfree[b]: the last step that read buffer b is done.
+    // kind psi: the weights of block b + 1 are formed on the context's second
+    // stream while block b's steps run on its stream (the weights do not
+    // depend on the state); w and d0 then hold two buffers, block b using
+    // buffer b & 1.  wready[q]: buffer q's weights are formed; wfree[q]: the
+    // last launch that read buffer q is done.
     hipStream_t wstream = nullptr;
     hipEvent_t wready[2] = {nullptr, nullptr}, wfree[2] = {nullptr, nullptr};
-    int wahead = 0;                         // step whose weights were launched ahead (0: none)
+    int wblock = -1;                        // the block whose weights the stream's work has
+    int wahead = -1;                        // the block whose weights were launched ahead
     size_t wsz = 0;                         // elements of one w buffer (0: one buffer)
     int64_t hnodes = 0, hnodes_mt = 0;  // real history nodes (all; full-history problems)
     double* U = nullptr;
     void* hist = nullptr;     // slots * ldh (FP64 or FP32)
-    double* part = nullptr;   // kMaxChunks * ldh
-    double* w = nullptr;      // nprob * ldw FP64 weights (lag-indexed)
-    float* w32 = nullptr;     // FP32 copy for FRM_PREC_F32C
-    double* d0 = nullptr;     // per-problem current-step coefficient
+    double* part = nullptr;   // series problems: the series value per node
+    double* far = nullptr;    // [kHistBlock][ldh] far sums of the current block
+    double* w = nullptr;      // nprob * ldw weights, lag-indexed; kind psi: a block's table
+    double* d0 = nullptr;     // per-problem current-step coefficient (kind psi: per step too)
+    double* psi_g = nullptr;  // kind psi: g(a tau) and the inverse's derivative there,
+                              // [2][nprob][capacity + 2]
     int* bad = nullptr;       // set when a psi weight is not finite
     int ldw = 0;
     // kind AB
@@ -1200,8 +1483,11 @@ static hipError_t mt_launch(frm_mt1d* s, void (*kern)(KArgs...), dim3 grid, dim3
     r.block = block;
     (r.arg(static_cast<std::decay_t<KArgs>>(args)), ...);
     if (s->rec) {
-        r.step = s->rec_step;
         r.branch = s->lstream != nullptr;
+        if (!r.branch) {
+            r.join = s->rec_join;
+            s->rec_join = false;
+        }
         s->rec->push_back(r);
         return hipSuccess;
     }
@@ -1210,171 +1496,134 @@ static hipError_t mt_launch(frm_mt1d* s, void (*kern)(KArgs...), dim3 grid, dim3
     return hipLaunchKernel(r.func, grid, block, p, 0, s->lstream ? s->lstream : s->ctx->stream);
 }
 
-// The weight buffers of step k (kind psi: two, by step parity).
-static double* mt_w(const frm_mt1d* s, int k) {
-    return s->w + (s->wsz ? (size_t)(k & 1) * s->wsz : 0);
+// The weight buffers of block b (kind psi: two, by parity).
+static double* mt_w(const frm_mt1d* s, int b) {
+    return s->w + (s->wsz ? (size_t)(b & 1) * s->wsz : 0);
 }
-static float* mt_w32(const frm_mt1d* s, int k) {
-    return s->w32 ? s->w32 + (s->wsz ? (size_t)(k & 1) * s->wsz : 0) : nullptr;
-}
-static double* mt_d0(const frm_mt1d* s, int k) {
-    return s->d0 + (s->wsz ? (size_t)(k & 1) * s->nprob : 0);
+static double* mt_d0(const frm_mt1d* s, int b) {
+    return s->d0 + (s->wsz ? (size_t)(b & 1) * s->nprob * (kHistBlock + 2) : 0);
 }
 
-// Kind psi: the weights of step k at `depth` history slots, then the
-// quadrature fallback of the intervals whose series was not finite.
-static hipError_t mt_launch_psi_weights(frm_mt1d* s, int k, int depth) {
-    const int threads = 256;
-    const dim3 grid((unsigned)((depth + 1 + threads - 1) / threads), (unsigned)s->nprob);
-    hipError_t e = mt_launch(s, k_psi_weights, grid, dim3(threads), s->probs, s->nprob, k, depth,
-                             s->tau, mt_w(s, k), s->ldw, mt_w32(s, k), mt_d0(s, k), s->bad,
-                             s->psi_queue, s->psi_qcap, s->psi_qcount);
-    // a fixed grid: threads beyond the queue's length exit at once
-    if (e == hipSuccess)
-        e = mt_launch(s, k_psi_quad, dim3(64), dim3(64), s->probs, k, depth, s->tau, mt_w(s, k),
-                      s->ldw, mt_w32(s, k), mt_d0(s, k), s->bad, s->psi_queue, s->psi_qcap,
-                      s->psi_qcount);
-    return e;
-}
-
-// The same on the weight stream, once the last reader of step k's buffers
-// is done; wready of the buffer marks the end.  While a graph is recorded
-// the launches become a branch of it, ordered by the graph's edges instead.
-static hipError_t mt_launch_psi_weights_ahead(frm_mt1d* s, int k, int depth) {
-    hipError_t e = s->rec ? hipSuccess : hipStreamWaitEvent(s->wstream, s->wfree[k & 1], 0);
-    s->lstream = s->wstream;
-    if (e == hipSuccess) e = mt_launch_psi_weights(s, k, depth);
-    s->lstream = nullptr;
-    if (e == hipSuccess && !s->rec) e = hipEventRecord(s->wready[k & 1], s->wstream);
-    return e;
-}
-
-// Time chunks of the memory term at `depth` history slots: one, unless the
-// nodes alone give fewer than kMemtermWaves wavefronts; chunks are at least
-// `min_chunk` slots (the history block length) and at most kMaxChunks.
-static int mt_chunks(const frm_mt1d* s, int depth, int min_chunk) {
-    const int64_t waves = s->ldh / (2 * kWave);
-    int nch = 1;
-    if (waves < kMemtermWaves) nch = (int)((kMemtermWaves + waves - 1) / waves);
-    return std::max(1, std::min<int>({nch, (depth + min_chunk - 1) / min_chunk, kMaxChunks}));
-}
-
-// The memory term of step k: `depth` history slots in `nch` time chunks.
-static hipError_t mt_launch_memterm(frm_mt1d* s, int k, int depth, int nch) {
-    const int chunk = (depth + nch - 1) / nch;
-    const dim3 grid((unsigned)(s->ldh / 2 / kMemtermThreads), (unsigned)nch);
-    if (s->precision == FRM_PREC_F32C) {
-        // four nodes per lane where the batch fills the GPU with half the wavefronts
-        if (nch == 1 && s->ldh / (4 * kWave) >= kMemtermWaves) {
-            const dim3 g4((unsigned)((s->ldh / 4 + kMemtermThreads - 1) / kMemtermThreads), 1);
-            return mt_launch(s, k_mt_memterm_f32c<4>, g4, dim3(kMemtermThreads),
-                             (const float*)s->hist, s->ldh, depth, mt_w32(s, k), s->ldw, s->gprob,
-                             s->gvalid, chunk, s->part);
-        }
-        return mt_launch(s, k_mt_memterm_f32c<2>, grid, dim3(kMemtermThreads), (const float*)s->hist,
-                         s->ldh, depth, mt_w32(s, k), s->ldw, s->gprob, s->gvalid, chunk, s->part);
-    }
-    return mt_launch(s, k_mt_memterm_f64, grid, dim3(kMemtermThreads), (const double*)s->hist,
-                     s->ldh, depth, mt_w(s, k), s->ldw, s->gprob_mt ? s->gprob_mt : s->gprob,
-                     s->gvalid, chunk, s->part);
-}
-
-// The sweep of step k over the memory term's `nch` chunks; the step's
-// increment goes to history slot `depth` when `push`.
-static hipError_t mt_launch_sweep(frm_mt1d* s, int k, int depth, int nch, bool push) {
-    const dim3 g((unsigned)((s->nprob + 3) / 4));
-    const int cm = mt_pick_cm(s->maxN);
-    const size_t esz = s->precision == FRM_PREC_F32C ? sizeof(float) : sizeof(double);
-    if (s->kind == FRM_MT_AB) {
-        AbSweepArgs b;
-        b.pr = s->probs;
-        b.nprob = s->nprob;
-        b.U = s->U;
-        b.part = s->part;
-        b.nch = nch;
-        b.ldh = s->ldh;
-        b.d0 = mt_d0(s, k);
-        b.cf = s->ab_cf;
-        b.cal = s->ab_cal;
-        b.ml = s->ab_ml;
-        b.ldml = s->capacity;
-        b.k = k;
-        b.tau = s->tau;
-        b.slot = (double*)s->hist + (size_t)depth * s->ldh;
-        b.err = s->ab_err;
-        switch (cm) {
-            case 4: return mt_launch(s, k_ab1d_sweep<4>, g, dim3(256), b);
-            case 8: return mt_launch(s, k_ab1d_sweep<8>, g, dim3(256), b);
-            default: return mt_launch(s, k_ab1d_sweep<16>, g, dim3(256), b);
-        }
-    }
-    MtSweepArgs a;
+// Kind psi: the weights of block b, then the quadrature fallback of those
+// whose series was not finite.
+static hipError_t mt_launch_psi_weights(frm_mt1d* s, int b) {
+    PsiArgs a;
     a.pr = s->probs;
     a.nprob = s->nprob;
-    a.U = s->U;
-    a.part = s->part;
-    a.nch = nch;
-    a.ldh = s->ldh;
-    a.d0 = mt_d0(s, k);
-    a.slot = push ? (void*)((char*)s->hist + esz * (size_t)depth * s->ldh) : nullptr;
-    a.slot_f32 = s->precision == FRM_PREC_F32C;
-    a.picard = s->picard;
-    switch (cm) {
-        case 4: return mt_launch(s, k_mt_sweep<4>, g, dim3(256), a);
-        case 8: return mt_launch(s, k_mt_sweep<8>, g, dim3(256), a);
-        default: return mt_launch(s, k_mt_sweep<16>, g, dim3(256), a);
-    }
+    a.N0 = b * kHistBlock;
+    a.capacity = s->capacity;
+    a.tau = s->tau;
+    a.gl = s->capacity + 2;
+    a.g = s->psi_g;
+    a.dg = s->psi_g + (size_t)s->nprob * a.gl;
+    a.w = mt_w(s, b);
+    a.ldw = s->ldw;
+    a.d0 = mt_d0(s, b);
+    a.bad = s->bad;
+    a.queue = s->psi_queue;
+    a.qcap = s->psi_qcap;
+    a.qcount = s->psi_qcount;
+    // 16 slots per workgroup up to the block's last step's newest, and one
+    // workgroup for the current-step factors
+    const dim3 grid((unsigned)(b + 2), (unsigned)s->nprob);
+    hipError_t e = mt_launch(s, k_psi_weights, grid, dim3(256), a);
+    // a fixed grid: threads beyond the queue's length exit at once
+    if (e == hipSuccess) e = mt_launch(s, k_psi_quad, dim3(64), dim3(64), a);
+    return e;
 }
 
-// Autotuner of the history block length, the shortest time chunk of the
-// memory term.  With few nodes the history is split into time chunks so that
-// enough wavefronts stream it, and the sweep then adds the chunks' partial
-// sums: shorter chunks give the memory term more wavefronts and the sweep
-// more partials to add.  Each candidate length's memory term and sweep are
-// timed at the run's mean depth (capacity / 2 history slots) on the solver's
-// own buffers, before any state is set (the state is zeroed first; the
-// sweeps of kinds L1 and psi write no history slot, the AB sweep writes slot
-// D, which a step overwrites before it is read), and the fastest is kept.
-// A batch whose nodes alone fill the GPU takes one chunk whatever the length
-// and is not timed.
-static int mt_tune_block(frm_ctx* ctx, frm_mt1d* s, int force) {
-    if (force > 0) {
-        s->min_chunk = force;
-        return FRM_OK;
+// The same on the weight stream, once the last reader of block b's buffers
+// is done; wready of the buffer marks the end.  While a graph is recorded
+// the launches become a branch of it, ordered by the graph's edges instead.
+static hipError_t mt_launch_psi_weights_ahead(frm_mt1d* s, int b) {
+    hipError_t e = s->rec ? hipSuccess : hipStreamWaitEvent(s->wstream, s->wfree[b & 1], 0);
+    s->lstream = s->wstream;
+    if (e == hipSuccess) e = mt_launch_psi_weights(s, b);
+    s->lstream = nullptr;
+    if (e == hipSuccess && !s->rec) e = hipEventRecord(s->wready[b & 1], s->wstream);
+    return e;
+}
+
+// Wavefronts that share a tile of the far pass over N0 slots: one where the
+// batch has the tiles for kMemtermWaves wavefronts of four nodes per lane;
+// else as many as bring its one-node tiles there, none of them with fewer
+// than min_chunk slots (the history block length).
+static int mt_far_split(const frm_mt1d* s, int N0) {
+    if (s->ldh / (4 * 16) >= kMemtermWaves) return 1;
+    const int64_t tiles = s->ldh / 16;
+    int ks = 2;
+    while (ks < kFarSplit && ks * tiles < kMemtermWaves && N0 / (2 * ks) >= s->min_chunk) ks *= 2;
+    return ks;
+}
+
+template <typename HT, bool TAB>
+static hipError_t mt_launch_far_t(frm_mt1d* s, int N0) {
+    const int ks = mt_far_split(s, N0);
+    const int* gprob = s->gprob_mt ? s->gprob_mt : s->gprob;
+    const double* w = mt_w(s, N0 / kHistBlock);
+    if (ks == 1)
+        return mt_launch(s, k_mt_far<HT, TAB, false>, dim3((unsigned)(s->ldh / 256)), dim3(256),
+                         (const HT*)s->hist, s->ldh, N0, w, s->ldw, gprob, s->gvalid, s->far);
+    return mt_launch(s, k_mt_far<HT, TAB, true>, dim3((unsigned)(s->ldh / 16)),
+                     dim3((unsigned)(64 * ks)), (const HT*)s->hist, s->ldh, N0, w, s->ldw, gprob,
+                     s->gvalid, s->far);
+}
+
+// The far sums of the block that starts at history index N0.
+static hipError_t mt_launch_far(frm_mt1d* s, int N0) {
+    const bool tab = s->kind == FRM_MT_PSI;
+    if (s->precision == FRM_PREC_F32C)
+        return tab ? mt_launch_far_t<float, true>(s, N0) : mt_launch_far_t<float, false>(s, N0);
+    return tab ? mt_launch_far_t<double, true>(s, N0) : mt_launch_far_t<double, false>(s, N0);
+}
+
+// Steps k .. k + ks - 1 of every problem, all in block b.
+static hipError_t mt_launch_steps(frm_mt1d* s, int b, int k, int ks) {
+    const dim3 g((unsigned)s->nprob), t((unsigned)(64 * ((s->maxN - 2 + 64 * kMtCM) / (64 * kMtCM))));
+    if (s->kind == FRM_MT_AB) {
+        AbStepArgs a;
+        a.pr = s->probs;
+        a.order = s->order;
+        a.U = s->U;
+        a.hist = (double*)s->hist;
+        a.ldh = s->ldh;
+        a.G = b > 0 ? s->far : nullptr;
+        a.w = s->w;
+        a.ldw = s->ldw;
+        a.d0 = s->d0;
+        a.cf = s->ab_cf;
+        a.cal = s->ab_cal;
+        a.ml = s->ab_ml;
+        a.ldml = s->capacity;
+        a.ser = s->part;
+        a.N0 = b * kHistBlock;
+        a.k0 = k;
+        a.ks = ks;
+        a.tau = s->tau;
+        a.err = s->ab_err;
+        return mt_launch(s, k_ab_steps, g, t, a);
     }
-    s->min_chunk = kMinChunk;
-    const int D = std::min(s->slots - 1, s->capacity / 2);
-    if (s->ser_count == s->nprob || s->ldh / (2 * kWave) >= kMemtermWaves || D < 32) return FRM_OK;
-    static const int kCand[] = {16, 32, 64, 128, 256, 512};
-    constexpr int kReps = 20;
-    hipEvent_t a = nullptr, b = nullptr;
-    hipError_t e = hipEventCreate(&a);
-    if (e == hipSuccess) e = hipEventCreate(&b);
-    if (e == hipSuccess) e = hipMemsetAsync(s->U, 0, sizeof(double) * s->nU, ctx->stream);
-    float best = 0.f;
-    int last_nch = -1;
-    for (int L : kCand) {
-        if (e != hipSuccess) break;
-        const int nch = mt_chunks(s, D, L);
-        if (nch == last_nch) continue;  // the same launches as the shorter length
-        last_nch = nch;
-        for (int r = -2; r < kReps && e == hipSuccess; ++r) {
-            if (r == 0) e = hipEventRecord(a, ctx->stream);
-            if (e == hipSuccess) e = mt_launch_memterm(s, 0, D, nch);
-            if (e == hipSuccess) e = mt_launch_sweep(s, 0, D, nch, false);
-        }
-        if (e == hipSuccess) e = hipEventRecord(b, ctx->stream);
-        if (e == hipSuccess) e = hipEventSynchronize(b);
-        float ms = 0.f;
-        if (e == hipSuccess) e = hipEventElapsedTime(&ms, a, b);
-        if (e == hipSuccess && (best == 0.f || ms < best)) {
-            best = ms;
-            s->min_chunk = L;
-        }
-    }
-    if (a) (void)hipEventDestroy(a);
-    if (b) (void)hipEventDestroy(b);
-    return e == hipSuccess ? FRM_OK : check_hip(ctx, e, "frm_mt1d_create: history block tuning");
+    MtStepArgs a;
+    a.pr = s->probs;
+    a.order = s->order;
+    a.U = s->U;
+    a.hist = s->hist;
+    a.ldh = s->ldh;
+    a.G = b > 0 ? s->far : nullptr;
+    a.w = mt_w(s, b);
+    a.ldw = s->ldw;
+    a.d0 = mt_d0(s, b);
+    a.nprob = s->nprob;
+    a.N0 = b * kHistBlock;
+    a.k0 = k;
+    a.ks = ks;
+    a.picard = s->picard;
+    const bool psi = s->kind == FRM_MT_PSI;
+    if (s->precision == FRM_PREC_F32C)
+        return psi ? mt_launch(s, k_mt_steps<float, true>, g, t, a)
+                   : mt_launch(s, k_mt_steps<float, false>, g, t, a);
+    return psi ? mt_launch(s, k_mt_steps<double, true>, g, t, a)
+               : mt_launch(s, k_mt_steps<double, false>, g, t, a);
 }
 
 static void mt_free(frm_mt1d* s) {
@@ -1382,6 +1631,7 @@ static void mt_free(frm_mt1d* s) {
     (void)hipFree(s->probs);
     (void)hipFree(s->gprob);
     (void)hipFree(s->gvalid);
+    (void)hipFree(s->order);
     for (auto& g : s->graphs) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (g.graph) (void)hipGraphDestroy(g.graph);
@@ -1389,14 +1639,15 @@ static void mt_free(frm_mt1d* s) {
     (void)hipFree(s->U);
     (void)hipFree(s->hist);
     (void)hipFree(s->part);
+    (void)hipFree(s->far);
     if (s->wstream) (void)hipStreamSynchronize(s->wstream);  // the context's, shared
     for (int b = 0; b < 2; ++b) {
         if (s->wready[b]) (void)hipEventDestroy(s->wready[b]);
         if (s->wfree[b]) (void)hipEventDestroy(s->wfree[b]);
     }
     (void)hipFree(s->w);
-    (void)hipFree(s->w32);
     (void)hipFree(s->d0);
+    (void)hipFree(s->psi_g);
     (void)hipFree(s->bad);
     (void)hipFree(s->ab_cf);
     (void)hipFree(s->ab_cal);
@@ -1457,7 +1708,7 @@ static int ab_setup(frm_ctx* ctx, frm_mt1d* s, const frm_mt1d_desc* d) {
         }
         const std::vector<double>& I = it->second;
         const double Ii = I[0];
-        for (int l = 1; l <= s->ldw; ++l) w[(size_t)p * s->ldw + l - 1] = I[l];
+        for (int l = 1; l <= s->slots; ++l) w[(size_t)p * s->ldw + l - 1] = I[l];
         d0[p] = Ii / (1.0 - a);
         const int m = P.N;
         const double h = 1.0 / m;
@@ -1587,7 +1838,9 @@ int frm_mt1d_create(frm_ctx* ctx, const frm_mt1d_desc* d, frm_mt1d** out) {
     // L1/psi: increments enter from step 3 on; AB: every increment
     const bool is_ab = d->kind == FRM_MT_AB;
     s->slots = is_ab ? d->capacity : std::max(1, d->capacity - 2);
-    s->ldw = s->slots;
+    // weights up to the lag of a block's last step, 0 past the slots
+    s->ldw = s->slots + kHistBlock;
+    s->min_chunk = d->hist_block > 0 ? d->hist_block : s->min_chunk;
     std::vector<int> gp, gv;
     int64_t uoff = 0, hoff = 0;
     for (int p = 0; p < d->nprob; ++p) {
@@ -1655,14 +1908,25 @@ int frm_mt1d_create(frm_ctx* ctx, const frm_mt1d_desc* d, frm_mt1d** out) {
     if (e == hipSuccess) e = hipMalloc(&s->gvalid, sizeof(int) * gv.size());
     if (e == hipSuccess) e = hipMalloc(&s->U, sizeof(double) * s->nU);
     if (e == hipSuccess) e = hipMalloc(&s->hist, esz * (size_t)s->slots * s->ldh);
-    if (e == hipSuccess) e = hipMalloc(&s->part, sizeof(double) * (size_t)kMaxChunks * s->ldh);
-    // kind psi: two buffers of weights, the next step's formed ahead
-    const size_t nwb = d->kind == FRM_MT_PSI ? 2 : 1;
-    if (d->kind == FRM_MT_PSI) s->wsz = (size_t)d->nprob * s->ldw;
-    if (e == hipSuccess) e = hipMalloc(&s->w, sizeof(double) * nwb * (size_t)d->nprob * s->ldw);
-    if (e == hipSuccess && d->precision == FRM_PREC_F32C)
-        e = hipMalloc(&s->w32, sizeof(float) * nwb * (size_t)d->nprob * s->ldw);
-    if (e == hipSuccess) e = hipMalloc(&s->d0, sizeof(double) * nwb * d->nprob);
+    if (e == hipSuccess && s->ser_count > 0) e = hipMalloc(&s->part, sizeof(double) * s->ldh);
+    if (e == hipSuccess && s->slots > kHistBlock)
+        e = hipMalloc(&s->far, sizeof(double) * (size_t)kHistBlock * s->ldh);
+    std::vector<int> order(d->nprob);
+    for (int p = 0; p < d->nprob; ++p) order[p] = p;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int x, int y) { return s->hprobs[x].N > s->hprobs[y].N; });
+    if (e == hipSuccess) e = hipMalloc(&s->order, sizeof(int) * d->nprob);
+    if (e == hipSuccess)
+        e = hipMemcpy(s->order, order.data(), sizeof(int) * d->nprob, hipMemcpyHostToDevice);
+    // kind psi: two buffers of a block's weights, the next block's formed ahead
+    const bool psi = d->kind == FRM_MT_PSI;
+    const size_t wn = (size_t)d->nprob * s->ldw * (psi ? kHistBlock : 1);
+    const size_t dn = (size_t)d->nprob * (psi ? kHistBlock + 2 : 1);
+    if (psi) s->wsz = wn;
+    if (e == hipSuccess) e = hipMalloc(&s->w, sizeof(double) * (psi ? 2 : 1) * wn);
+    if (e == hipSuccess) e = hipMalloc(&s->d0, sizeof(double) * (psi ? 2 : 1) * dn);
+    if (e == hipSuccess && psi)
+        e = hipMalloc(&s->psi_g, sizeof(double) * 2 * (size_t)d->nprob * (s->capacity + 2));
     if (e == hipSuccess && d->kind == FRM_MT_PSI) {
         if (!ctx->aux_stream) e = hipStreamCreateWithFlags(&ctx->aux_stream, hipStreamNonBlocking);
         s->wstream = ctx->aux_stream;
@@ -1673,8 +1937,9 @@ int frm_mt1d_create(frm_ctx* ctx, const frm_mt1d_desc* d, frm_mt1d** out) {
     }
     if (e == hipSuccess) e = hipMalloc(&s->bad, sizeof(int));
     if (e == hipSuccess && d->kind == FRM_MT_PSI) {
-        // one entry per weight of a step, up to 2^20 (more set bad bit 4)
-        s->psi_qcap = (int)std::min<int64_t>((int64_t)d->nprob * (s->capacity + 1), 1 << 20);
+        // one entry per weight of a block, up to 2^20 per step (more set bad bit 4)
+        s->psi_qcap = (int)std::min<int64_t>(
+            (int64_t)d->nprob * (s->capacity + 1) * (kHistBlock + 2), (1 << 20) * kHistBlock);
         e = hipMalloc(&s->psi_queue, sizeof(int2) * s->psi_qcap);
         if (e == hipSuccess) e = hipMalloc(&s->psi_qcount, 2 * sizeof(int));
         if (e == hipSuccess) e = hipMemset(s->psi_qcount, 0, 2 * sizeof(int));
@@ -1685,25 +1950,34 @@ int frm_mt1d_create(frm_ctx* ctx, const frm_mt1d_desc* d, frm_mt1d** out) {
     }
     // L1 weights: kappa(l+2) = (l+2)^(1-a) - (l+1)^(1-a) as the reference forms
     // them (mt_minimal.cpp:926-931); psi weights are rebuilt every step.
-    std::vector<double> w((size_t)d->nprob * s->ldw, 0.0), d0(d->nprob);
-    std::vector<float> w32(d->precision == FRM_PREC_F32C ? w.size() : 0);
-    for (int p = 0; p < d->nprob; ++p) {
+    std::vector<double> w(psi ? 0 : wn, 0.0), d0(psi ? 0 : dn);
+    for (int p = 0; p < d->nprob && !psi; ++p) {
         const double a = d->probs[p].alpha;
         d0[p] = s->hprobs[p].Da;
         if (d->kind == FRM_MT_L1)
-            for (int l = 0; l < s->ldw; ++l) {
-                const double kv = std::pow((double)(l + 2), 1.0 - a) - std::pow((double)(l + 1), 1.0 - a);
-                w[(size_t)p * s->ldw + l] = kv;
-                if (!w32.empty()) w32[(size_t)p * s->ldw + l] = (float)kv;
-            }
+            for (int l = 0; l < s->slots; ++l)
+                w[(size_t)p * s->ldw + l] =
+                    std::pow((double)(l + 2), 1.0 - a) - std::pow((double)(l + 1), 1.0 - a);
     }
     e = hipMemcpy(s->probs, s->hprobs.data(), sizeof(MtProbDev) * d->nprob, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(s->gprob, gp.data(), sizeof(int) * gp.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(s->gvalid, gv.data(), sizeof(int) * gv.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(s->w, w.data(), sizeof(double) * w.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess && !w32.empty())
-        e = hipMemcpy(s->w32, w32.data(), sizeof(float) * w32.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(s->d0, d0.data(), sizeof(double) * d0.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess && !psi) {
+        e = hipMemcpy(s->w, w.data(), sizeof(double) * w.size(), hipMemcpyHostToDevice);
+        if (e == hipSuccess)
+            e = hipMemcpy(s->d0, d0.data(), sizeof(double) * d0.size(), hipMemcpyHostToDevice);
+    } else if (e == hipSuccess) {
+        // steps past the capacity have no weights: zeros, not stale memory
+        e = hipMemset(s->w, 0, sizeof(double) * 2 * wn);
+        const int gl = s->capacity + 2;
+        if (e == hipSuccess) {
+            hipLaunchKernelGGL(k_psi_tables, dim3((unsigned)((gl + 255) / 256), (unsigned)d->nprob),
+                               dim3(256), 0, ctx->stream, s->probs, gl, s->tau, s->psi_g,
+                               s->psi_g + (size_t)d->nprob * gl);
+            e = hipGetLastError();
+        }
+        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    }
     if (e == hipSuccess) e = hipMemset(s->bad, 0, sizeof(int));
     if (e == hipSuccess) e = hipMemset(s->hist, 0, esz * (size_t)s->slots * s->ldh);
     if (e != hipSuccess) {
@@ -1716,10 +1990,6 @@ int frm_mt1d_create(frm_ctx* ctx, const frm_mt1d_desc* d, frm_mt1d** out) {
             mt_free(s);
             return rc;
         }
-    }
-    if (const int rc = mt_tune_block(ctx, s, d->hist_block)) {
-        mt_free(s);
-        return rc;
     }
     *out = s;
     return FRM_OK;
@@ -1739,7 +2009,8 @@ int frm_mt1d_set_state(frm_mt1d* s, const double* h_U) {
     FRM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     s->tstep = 1;
     s->depth = 0;
-    s->wahead = 0;  // weights formed ahead were for the old run (done: the stream waited on them)
+    // weights formed so far were for the old run (done: the stream waited on them)
+    s->wblock = s->wahead = -1;
     if (s->psi_qcount) {
         FRM_HIP(ctx, hipMemsetAsync(s->psi_qcount, 0, 2 * sizeof(int), ctx->stream));
         FRM_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1771,12 +2042,21 @@ int frm_mt1d_step(frm_mt1d* s, int32_t nsteps) {
         return set_error(ctx, FRM_E_RANGE, "frm_mt1d_step: %d steps exceed capacity %d",
                          s->tstep - 1 + nsteps, s->capacity);
     const size_t esz = s->precision == FRM_PREC_F32C ? sizeof(float) : sizeof(double);
-    // one step: the launches of step s->tstep, queued on the context's stream
-    auto step_once = [&]() -> int {
-        const int k = s->tstep;
-        const int depth = s->depth;  // = max(0, k - 3)
+    // the next steps, at most `most` and all of one block, queued on the
+    // context's stream; steps with observations go one by one between the
+    // kernels that score them, steps with series problems one by one after
+    // the series kernel
+    auto run_some = [&](int most) -> int {
+        constexpr int J = kHistBlock;
+        const int off = s->kind == FRM_MT_AB ? 1 : 3;  // first step that stores an increment
+        const int k = s->tstep, h = k - off, b = std::max(0, h) / J;
+        auto obs = [&](int st) { return s->nobs ? s->fit_off[st] - s->fit_off[st - 1] : 0; };
+        const int fcnt = obs(k);
+        int ks = std::min(most, (b + 1) * J - h);
+        if (fcnt > 0 || s->ser_count > 0) ks = 1;
+        for (int i = 1; i < ks; ++i)
+            if (obs(k + i) > 0) ks = i;
         FitArgs fa{};
-        const int fcnt = s->nobs ? s->fit_off[k] - s->fit_off[k - 1] : 0;
         if (fcnt > 0) {
             fa.pr = s->probs;
             fa.nprob = s->nprob;
@@ -1796,45 +2076,31 @@ int frm_mt1d_step(frm_mt1d* s, int32_t nsteps) {
             FRM_HIP(ctx, mt_launch(s, k_fit_before, dim3((unsigned)((s->nprob + 255) / 256)),
                                    dim3(256), fa));
         }
-        // the step's fitting error, once U holds the new state
-        auto fit_after = [&]() -> int {
-            if (fcnt > 0) {
-                LaunchTimer t(ctx, FRM_K_OTHER, 0.0);
-                FRM_HIP(ctx, mt_launch(s, k_fit_after, dim3((unsigned)((s->nprob + 255) / 256)),
-                                       dim3(256), fa));
-            }
-            s->tt += s->tau;
-            return FRM_OK;
-        };
-        // kind psi: the weights overlap the previous step unless launches are
-        // timed one by one (recorded for a graph: a branch of it, which the
-        // next step's first launch depends on)
-        const bool ahead = s->kind == FRM_MT_PSI && s->wstream && !ctx->timing_mask;
-        if (s->kind == FRM_MT_PSI) {
-            if (s->wahead == k) {
-                if (!s->rec) FRM_HIP(ctx, hipStreamWaitEvent(ctx->stream, s->wready[k & 1], 0));
-            } else if (ahead && !s->rec) {
-                FRM_HIP(ctx, mt_launch_psi_weights_ahead(s, k, depth));
-                FRM_HIP(ctx, hipStreamWaitEvent(ctx->stream, s->wready[k & 1], 0));
+        const bool psi_start = s->kind == FRM_MT_PSI && s->wblock != b;
+        if (psi_start) {
+            // the block's weights: formed during the block before, or here
+            if (s->wahead == b) {
+                if (s->rec) s->rec_join = true;
+                else FRM_HIP(ctx, hipStreamWaitEvent(ctx->stream, s->wready[b & 1], 0));
             } else {
                 LaunchTimer t(ctx, FRM_K_OTHER, 0.0);
-                FRM_HIP(ctx, mt_launch_psi_weights(s, k, depth));
+                FRM_HIP(ctx, mt_launch_psi_weights(s, b));
             }
-            s->wahead = 0;
-            // the next step's weights (depth + 1 slots from step 3 on), formed
-            // while this step's memory term and sweep run
-            if (ahead && k + 1 <= s->capacity) {
-                FRM_HIP(ctx, mt_launch_psi_weights_ahead(s, k + 1, k >= 3 ? depth + 1 : depth));
-                s->wahead = k + 1;
-            }
+            s->wahead = -1;
+            s->wblock = b;
         }
-        int nch = 0;
-        if (depth > 0 && s->ser_count < s->nprob) {
-            nch = mt_chunks(s, depth, s->min_chunk);
-            // algorithmic bytes: the problems' own nodes (padding lanes load nothing)
+        if (b > 0 && h == b * J && s->ser_count < s->nprob) {
+            // algorithmic bytes: the problems' own nodes
             LaunchTimer t(ctx, FRM_K_MEMTERM,
-                          (double)depth * (s->gprob_mt ? s->hnodes_mt : s->hnodes) * esz);
-            FRM_HIP(ctx, mt_launch_memterm(s, k, depth, nch));
+                          (double)(s->gprob_mt ? s->hnodes_mt : s->hnodes) *
+                              ((double)h * esz + J * sizeof(double)));
+            FRM_HIP(ctx, mt_launch_far(s, h));
+        }
+        // the next block's weights overlap this block's steps unless launches
+        // are timed one by one
+        if (psi_start && s->wstream && !ctx->timing_mask && (b + 1) * J + off <= s->capacity) {
+            FRM_HIP(ctx, mt_launch_psi_weights_ahead(s, b + 1));
+            s->wahead = b + 1;
         }
         if (s->kind == FRM_MT_AB && s->ser_count > 0 && k >= 2) {
             AbSeriesArgs c;
@@ -1843,7 +2109,7 @@ int frm_mt1d_step(frm_mt1d* s, int32_t nsteps) {
             c.ldh = s->ldh;
             c.tab = s->ser_tab;
             c.choice = s->ser_choice;
-            c.F = (const double*)s->hist + (size_t)(depth - 1) * s->ldh;  // step k - 1's increment
+            c.F = (const double*)s->hist + (size_t)(h - 1) * s->ldh;  // step k - 1's increment
             c.lc1 = s->ser_lc;
             c.lc2 = s->ser_lc + (size_t)s->ser_maxL * s->ldh;
             c.lflag = s->ser_flag;
@@ -1854,75 +2120,75 @@ int frm_mt1d_step(frm_mt1d* s, int32_t nsteps) {
             FRM_HIP(ctx, mt_launch(s, k_ab_series, dim3((unsigned)((s->ldh + 255) / 256)), dim3(256),
                                    c));
         }
-        if (s->kind == FRM_MT_AB) {
-            {
-                LaunchTimer t(ctx, FRM_K_SWEEP1D, 0.0);
-                FRM_HIP(ctx, mt_launch_sweep(s, k, depth, nch, true));
-            }
-            s->depth = depth + 1;
-            s->tstep = k + 1;
-            if (int rc = fit_after()) return rc;
-            return FRM_OK;
-        }
         {
             LaunchTimer t(ctx, FRM_K_SWEEP1D, 0.0);
-            FRM_HIP(ctx, mt_launch_sweep(s, k, depth, nch, k >= 3));
+            FRM_HIP(ctx, mt_launch_steps(s, b, k, ks));
         }
-        // the buffers of step k are free for step k + 2's weights
-        if (s->wstream && !s->rec) FRM_HIP(ctx, hipEventRecord(s->wfree[k & 1], ctx->stream));
-        if (k >= 3) s->depth = depth + 1;
-        s->tstep = k + 1;
-        if (int rc = fit_after()) return rc;
+        // once the block's last steps are through, its buffers are free
+        if (s->wstream && !s->rec) FRM_HIP(ctx, hipEventRecord(s->wfree[b & 1], ctx->stream));
+        s->tstep = k + ks;
+        s->depth = std::max(0, s->tstep - off);
+        if (fcnt > 0) {
+            LaunchTimer t(ctx, FRM_K_OTHER, 0.0);
+            FRM_HIP(ctx, mt_launch(s, k_fit_after, dim3((unsigned)((s->nprob + 255) / 256)),
+                                   dim3(256), fa));
+        }
+        for (int i = 0; i < ks; ++i) s->tt += s->tau;
         return FRM_OK;
     };
+    const int goal = s->tstep + nsteps;
     // Graph mode: the launches of up to kGraphSteps steps are recorded,
-    // matched with the graph built for the same kernel sequence (a chain of
-    // kernel nodes, instantiated once), the nodes get these steps' arguments
-    // and grids (hipGraphExecKernelNodeSetParams) and the graph is launched
-    // once.  Runs of steps differ only in arguments and grids (depth,
-    // time-chunk count, slots), so a run uses a handful of graphs.  Not while
-    // per-launch timing is on.
+    // matched with the graph built for the same kernel sequence (instantiated
+    // once), the nodes get these steps' arguments and grids
+    // (hipGraphExecKernelNodeSetParams) and the graph is launched once.  Runs
+    // of steps differ only in arguments and grids (depth, slots), so a run
+    // uses a handful of graphs.  Not while per-launch timing is on.
     if (!s->graph || ctx->timing_mask != 0) {
-        for (int it = 0; it < nsteps; ++it)
-            if (int rc = step_once()) return rc;
+        while (s->tstep < goal)
+            if (int rc = run_some(goal - s->tstep)) return rc;
         // a synchronisation of the context's stream also covers the weights
         // formed ahead
-        if (s->wahead) FRM_HIP(ctx, hipStreamWaitEvent(ctx->stream, s->wready[s->wahead & 1], 0));
+        if (s->wahead >= 0) FRM_HIP(ctx, hipStreamWaitEvent(ctx->stream, s->wready[s->wahead & 1], 0));
         return FRM_OK;
     }
     std::vector<KRec> recs;
     std::vector<void*> ptrs;
-    for (int it = 0; it < nsteps;) {
+    struct At {
+        int tstep, depth, wblock, wahead;
+        double tt;
+    };
+    auto at = [&] { return At{s->tstep, s->depth, s->wblock, s->wahead, s->tt}; };
+    auto back = [&](const At& t) {
+        s->tstep = t.tstep;
+        s->depth = t.depth;
+        s->wblock = t.wblock;
+        s->wahead = t.wahead;
+        s->tt = t.tt;
+    };
+    while (s->tstep < goal) {
         recs.clear();
-        const int tstep0 = s->tstep, depth0 = s->depth;
-        const double tt0 = s->tt;
-        // record steps until the run is full; a step that fails is taken
-        // back (the solver stays where it was before it) and ends the run
-        int done = 0, rc = FRM_OK;
-        const int wahead0 = s->wahead;
+        const At start = at();
+        const int stop = std::min(goal, s->tstep + kGraphSteps);
+        // record steps until the run is full; a launch that fails is taken
+        // back with its steps (the solver stays where it was before them)
+        // and ends the run
+        int rc = FRM_OK;
         s->rec = &recs;
-        for (; done < kGraphSteps && it + done < nsteps; ++done) {
+        s->rec_join = false;
+        while (s->tstep < stop) {
             const size_t mark = recs.size();
-            const int ts = s->tstep, dp = s->depth, wa = s->wahead;
-            const double tt = s->tt;
-            s->rec_step = done;
-            rc = step_once();
+            const At t = at();
+            rc = run_some(stop - s->tstep);
             if (rc) {
                 recs.resize(mark);
-                s->tstep = ts;
-                s->depth = dp;
-                s->tt = tt;
-                s->wahead = wa;
+                back(t);
                 break;
             }
         }
         s->rec = nullptr;
         // none of the run's steps is launched: the solver goes back to its start
         auto unrun = [&](int code) {
-            s->tstep = tstep0;
-            s->depth = depth0;
-            s->tt = tt0;
-            s->wahead = wahead0;
+            back(start);
             return code;
         };
         if (!recs.empty()) {
@@ -1931,7 +2197,7 @@ int frm_mt1d_step(frm_mt1d* s, int32_t nsteps) {
                 if (c.funcs.size() != recs.size()) continue;
                 bool same = true;
                 for (size_t i = 0; i < recs.size() && same; ++i)
-                    same = c.funcs[i] == recs[i].func && c.tags[i] == recs[i].step * 2 + recs[i].branch;
+                    same = c.funcs[i] == recs[i].func && c.tags[i] == recs[i].join * 2 + recs[i].branch;
                 if (same) {
                     g = &c;
                     break;
@@ -1951,50 +2217,28 @@ int frm_mt1d_step(frm_mt1d* s, int32_t nsteps) {
                 return q;
             };
             if (!g) {
-                // Edges: each step's own launches in order.  The weights
-                // formed ahead in step j (for step j + 1, into the buffers
-                // step j - 1 read) start after step j - 1's last launch (or
-                // after step j's weights when step j formed them itself) and
-                // after the weights formed ahead in step j - 1 (the weight
-                // kernels share the fallback queue, so they stay in order);
-                // step j + 1's first launch waits for them.  Without weights
-                // formed ahead the graph is a chain.
+                // Edges: the launches in order.  Weights formed ahead start
+                // after what was launched before them (the last reader of
+                // their buffers among it) and after the weights before them
+                // (they share the fallback queue); the block that reads them
+                // starts when they are done.
                 StepGraph ng;
                 FRM_HIP(ctx, hipGraphCreate(&ng.graph, 0));
                 hipError_t e = hipSuccess;
                 hipGraphNode_t main_last = nullptr, br_last = nullptr;
-                std::vector<hipGraphNode_t> step_last(done + 1, nullptr), step_br(done + 1, nullptr);
-                int cur = -1;
                 for (size_t i = 0; i < recs.size() && e == hipSuccess; ++i) {
                     const KRec& r = recs[i];
                     hipGraphNode_t dep[2];
                     size_t nd = 0;
-                    if (r.branch) {
-                        if (step_br[r.step]) {
-                            dep[nd++] = step_br[r.step];
-                        } else {
-                            if (cur == r.step && main_last) dep[nd++] = main_last;
-                            else if (r.step > 0 && step_last[r.step - 1]) dep[nd++] = step_last[r.step - 1];
-                            if (br_last) dep[nd++] = br_last;
-                        }
-                    } else {
-                        if (main_last) dep[nd++] = main_last;
-                        if (r.step != cur && r.step > 0 && step_br[r.step - 1]) dep[nd++] = step_br[r.step - 1];
-                    }
+                    if (main_last) dep[nd++] = main_last;
+                    if ((r.branch || r.join) && br_last) dep[nd++] = br_last;
                     hipKernelNodeParams q = params(i);
                     hipGraphNode_t node = nullptr;
                     e = hipGraphAddKernelNode(&node, ng.graph, nd ? dep : nullptr, nd, &q);
-                    if (r.branch) {
-                        br_last = node;
-                        step_br[r.step] = node;
-                    } else {
-                        main_last = node;
-                        step_last[r.step] = node;
-                        cur = r.step;
-                    }
+                    (r.branch ? br_last : main_last) = node;
                     ng.nodes.push_back(node);
                     ng.funcs.push_back(r.func);
-                    ng.tags.push_back(r.step * 2 + r.branch);
+                    ng.tags.push_back(r.join * 2 + r.branch);
                 }
                 if (e == hipSuccess) e = hipGraphInstantiate(&ng.exec, ng.graph, nullptr, nullptr, 0);
                 if (e != hipSuccess) {
@@ -2015,7 +2259,6 @@ int frm_mt1d_step(frm_mt1d* s, int32_t nsteps) {
             if (e != hipSuccess) return unrun(check_hip(ctx, e, "frm_mt1d_step: graph launch"));
         }
         if (rc) return rc;
-        it += done;
     }
     // the weight buffers' events, for steps launched eagerly later: every
     // graph so far is ahead of them on the context's stream

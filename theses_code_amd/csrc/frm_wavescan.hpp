@@ -3,7 +3,7 @@
 // A line of n unknowns is split into 64 contiguous chunks of CM elements,
 // one chunk per lane.  The Thomas forward and back-substitution recurrences
 // are first-order affine maps, so each lane composes the maps of its chunk,
-// a 6-step Kogge-Stone scan over the wavefront gives every lane the value
+// a 6-level scan over the wavefront gives every lane the value
 // entering its chunk, and the lane then replays the exact sequential Thomas
 // formulas over its chunk (method: Stone 1973 recurrence scan; the in-chunk
 // arithmetic is the reference's progonka, mt_minimal.cpp:942-1024).
@@ -12,79 +12,88 @@
 
 namespace frm {
 
+// Lane i's value of x moved by a DPP control (row_shr/row_shl within the rows of
+// 16 lanes, row_bcast across them, wave_shr/wave_shl by one lane); lanes the
+// control gives no source, and rows outside RMASK, take `old`.  A scan level
+// through DPP is a few register moves, one through __shfl two LDS round trips.
+template <int CTRL, int RMASK = 0xf>
+__device__ __forceinline__ double dpp_move(double old, double x) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(x), CTRL, RMASK, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(x), CTRL, RMASK, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+constexpr int kDppRowShr = 0x110, kDppRowShl = 0x100, kDppWaveShr1 = 0x138, kDppWaveShl1 = 0x130,
+              kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
+
+__device__ __forceinline__ double lane_value(double x, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
+                            __builtin_amdgcn_readlane(__double2loint(x), lane));
+}
+
+// One scan level: (P, Q) after the map that the control brings (the identity
+// where it brings none).
+template <int CTRL, int RMASK = 0xf>
+__device__ __forceinline__ void affine_level(double& P, double& Q) {
+    const double Po = dpp_move<CTRL, RMASK>(1.0, P), Qo = dpp_move<CTRL, RMASK>(0.0, Q);
+    Q = P * Qo + Q;
+    P = P * Po;
+}
+
 // Exclusive composition of affine maps x -> P x + Q over lanes 0..lane-1
-// (forward: earlier lanes first).
-__device__ inline void scan_affine_up(double& P, double& Q, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const double Po = __shfl_up(P, d);
-        const double Qo = __shfl_up(Q, d);
-        if (lane >= d) {
-            Q = P * Qo + Q;
-            P = P * Po;
-        }
-    }
-    const double Pe = __shfl_up(P, 1);
-    const double Qe = __shfl_up(Q, 1);
-    P = lane == 0 ? 1.0 : Pe;
-    Q = lane == 0 ? 0.0 : Qe;
-}
-
-// Exclusive composition over lanes lane+1..63 (backward: later lanes first).
-__device__ inline void scan_affine_down(double& P, double& Q, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const double Po = __shfl_down(P, d);
-        const double Qo = __shfl_down(Q, d);
-        if (lane + d < 64) {
-            Q = P * Qo + Q;
-            P = P * Po;
-        }
-    }
-    const double Pe = __shfl_down(P, 1);
-    const double Qe = __shfl_down(Q, 1);
-    P = lane == 63 ? 1.0 : Pe;
-    Q = lane == 63 ? 0.0 : Qe;
-}
-
-// Both scans with the wavefront's total map as well (lane 63's inclusive
-// forward composition, lane 0's inclusive backward composition), for lines
-// that span several wavefronts.
+// (forward: earlier lanes first), and the whole wavefront's map (Pt, Qt).
 __device__ inline void scan_affine_up_total(double& P, double& Q, int lane, double& Pt, double& Qt) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const double Po = __shfl_up(P, d);
-        const double Qo = __shfl_up(Q, d);
-        if (lane >= d) {
-            Q = P * Qo + Q;
-            P = P * Po;
-        }
-    }
-    Pt = __shfl(P, 63);
-    Qt = __shfl(Q, 63);
-    const double Pe = __shfl_up(P, 1);
-    const double Qe = __shfl_up(Q, 1);
-    P = lane == 0 ? 1.0 : Pe;
-    Q = lane == 0 ? 0.0 : Qe;
+    affine_level<kDppRowShr + 1>(P, Q);
+    affine_level<kDppRowShr + 2>(P, Q);
+    affine_level<kDppRowShr + 4>(P, Q);
+    affine_level<kDppRowShr + 8>(P, Q);
+    affine_level<kDppRowBcast15, 0xa>(P, Q);  // rows 1 and 3 after rows 0 and 2
+    affine_level<kDppRowBcast31, 0xc>(P, Q);  // rows 2 and 3 after row 1
+    Pt = lane_value(P, 63);
+    Qt = lane_value(Q, 63);
+    P = dpp_move<kDppWaveShr1>(1.0, P);
+    Q = dpp_move<kDppWaveShr1>(0.0, Q);
 }
 
+// Exclusive composition over lanes lane+1..63 (backward: later lanes first),
+// and the whole wavefront's map.
 __device__ inline void scan_affine_down_total(double& P, double& Q, int lane, double& Pt,
                                               double& Qt) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const double Po = __shfl_down(P, d);
-        const double Qo = __shfl_down(Q, d);
-        if (lane + d < 64) {
+    affine_level<kDppRowShl + 1>(P, Q);
+    affine_level<kDppRowShl + 2>(P, Q);
+    affine_level<kDppRowShl + 4>(P, Q);
+    affine_level<kDppRowShl + 8>(P, Q);
+    // rows 0 and 2 after rows 1 and 3, then rows 0 and 1 after row 2 (DPP
+    // broadcasts upwards only)
+    {
+        const double P1 = lane_value(P, 16), Q1 = lane_value(Q, 16);
+        const double P3 = lane_value(P, 48), Q3 = lane_value(Q, 48);
+        const double Po = lane < 32 ? P1 : P3, Qo = lane < 32 ? Q1 : Q3;
+        if (!(lane & 16)) {
             Q = P * Qo + Q;
             P = P * Po;
         }
     }
-    Pt = __shfl(P, 0);
-    Qt = __shfl(Q, 0);
-    const double Pe = __shfl_down(P, 1);
-    const double Qe = __shfl_down(Q, 1);
-    P = lane == 63 ? 1.0 : Pe;
-    Q = lane == 63 ? 0.0 : Qe;
+    {
+        const double Po = lane_value(P, 32), Qo = lane_value(Q, 32);
+        if (lane < 32) {
+            Q = P * Qo + Q;
+            P = P * Po;
+        }
+    }
+    Pt = lane_value(P, 0);
+    Qt = lane_value(Q, 0);
+    P = dpp_move<kDppWaveShl1>(1.0, P);
+    Q = dpp_move<kDppWaveShl1>(0.0, Q);
+}
+
+__device__ inline void scan_affine_up(double& P, double& Q, int lane) {
+    double Pt, Qt;
+    scan_affine_up_total(P, Q, lane, Pt, Qt);
+}
+
+__device__ inline void scan_affine_down(double& P, double& Q, int lane) {
+    double Pt, Qt;
+    scan_affine_down_total(P, Q, lane, Pt, Qt);
 }
 
 // Scratch in LDS for one line that spans W wavefronts.
@@ -246,12 +255,7 @@ struct Mob {
     double m00, m01, m10, m11;
 };
 
-__device__ inline Mob mob_mul(const Mob& x, const Mob& y) {  // x * y (apply y first)
-    Mob r;
-    r.m00 = x.m00 * y.m00 + x.m01 * y.m10;
-    r.m01 = x.m00 * y.m01 + x.m01 * y.m11;
-    r.m10 = x.m10 * y.m00 + x.m11 * y.m10;
-    r.m11 = x.m10 * y.m01 + x.m11 * y.m11;
+__device__ inline Mob mob_scale(Mob r) {
     const double mx = fmax(fmax(fabs(r.m00), fabs(r.m01)), fmax(fabs(r.m10), fabs(r.m11)));
     if (mx > 0.0 && isfinite(mx)) {
         int ex;
@@ -264,20 +268,38 @@ __device__ inline Mob mob_mul(const Mob& x, const Mob& y) {  // x * y (apply y f
     return r;
 }
 
-__device__ inline Mob shfl_up_mob(const Mob& m, int d) {
-    return Mob{__shfl_up(m.m00, d), __shfl_up(m.m01, d), __shfl_up(m.m10, d), __shfl_up(m.m11, d)};
+__device__ inline Mob mob_mul(const Mob& x, const Mob& y) {  // x * y (apply y first)
+    Mob r;
+    r.m00 = x.m00 * y.m00 + x.m01 * y.m10;
+    r.m01 = x.m00 * y.m01 + x.m01 * y.m11;
+    r.m10 = x.m10 * y.m00 + x.m11 * y.m10;
+    r.m11 = x.m10 * y.m01 + x.m11 * y.m11;
+    return mob_scale(r);
 }
 
-// Exclusive forward scan of Moebius maps (earlier lanes applied first).
-__device__ inline Mob scan_mob_up(Mob m, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const Mob o = shfl_up_mob(m, d);
-        if (lane >= d) m = mob_mul(m, o);
-    }
-    Mob e = shfl_up_mob(m, 1);
-    if (lane == 0) e = Mob{1.0, 0.0, 0.0, 1.0};
-    return e;
+template <int CTRL, int RMASK = 0xf>
+__device__ __forceinline__ Mob dpp_mob(const Mob& m) {  // the identity where there is no source
+    return Mob{dpp_move<CTRL, RMASK>(1.0, m.m00), dpp_move<CTRL, RMASK>(0.0, m.m01),
+               dpp_move<CTRL, RMASK>(0.0, m.m10), dpp_move<CTRL, RMASK>(1.0, m.m11)};
+}
+
+// Exclusive forward scan of Moebius maps (earlier lanes applied first), and the
+// whole wavefront's map.
+__device__ inline Mob scan_mob_up_total(Mob m, int lane, Mob& tot) {
+    m = mob_mul(m, dpp_mob<kDppRowShr + 1>(m));
+    m = mob_mul(m, dpp_mob<kDppRowShr + 2>(m));
+    m = mob_mul(m, dpp_mob<kDppRowShr + 4>(m));
+    m = mob_mul(m, dpp_mob<kDppRowShr + 8>(m));
+    m = mob_mul(m, dpp_mob<kDppRowBcast15, 0xa>(m));
+    m = mob_mul(m, dpp_mob<kDppRowBcast31, 0xc>(m));
+    tot = Mob{lane_value(m.m00, 63), lane_value(m.m01, 63), lane_value(m.m10, 63),
+              lane_value(m.m11, 63)};
+    return dpp_mob<kDppWaveShr1>(m);
+}
+
+__device__ inline Mob scan_mob_up(const Mob& m, int lane) {
+    Mob tot;
+    return scan_mob_up_total(m, lane, tot);
 }
 
 }  // namespace frm

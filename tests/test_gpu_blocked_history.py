@@ -112,3 +112,28 @@ def test_mt1d_large_batch_matches_single_problems(ctx, kind, precision, tol):
         s.calc_step(steps)
         assert relerr(got[q], s.state()[0]) <= tol, sizes[q]
         s.close()
+
+
+# The series history of several steps per launch, at the edges of its launch
+# variants (nodes per wavefront, accumulators that just fit LDS and that do
+# not), beside a full-history problem, in calls that end inside and across its
+# runs; the last case's accumulators overflow, so that sums restart from the
+# sorted pyramid.  Bar: 1e-12 against the oracle, as the series path's.
+@pytest.mark.parametrize("N_,maxl,alpha,tau,steps", [
+    (2, 3, 0.5, 0.01, 20), (64, 50, 0.6, 0.01, 40), (65, 50, 0.2, 0.01, 40), (66, 50, 0.9, 0.02, 60),
+    (129, 50, 0.7, 0.01, 40), (130, 17, 0.4, 0.02, 60), (190, 50, 0.6, 0.01, 20),
+    (200, 50, 0.6, 0.01, 20), (330, 20, 0.6, 0.01, 20), (8, 600, 0.3, 0.05, 80)])
+def test_ab_series_fused_steps_match_oracle(ctx, N_, maxl, alpha, tau, steps):
+    series = dict(N=N_, alpha=alpha, src=2, ab_maxl=maxl, ab_maxkiter=1000, ab_eps=1e-10, ab_series=1)
+    full = dict(N=40, alpha=0.6, src=1, ab_maxl=50, ab_maxkiter=1000, ab_eps=1e-10)
+    _, ref = O.ab_solve_series(alpha, steps * tau, steps, N_, maxl, 1000, 1e-10, 2)
+    _, ref_full = O.ab_solve(0.6, steps * tau, steps, 40, 50, 1000, 1e-10, 1)
+    for probs in ([series], [series, full, series]):
+        b = S.MT1DBatch(ctx, probs, tau, steps, [np.zeros(p["N"] + 2) for p in probs], kind=N.MT_AB)
+        for k in (1, 2, B - 2, steps - B - 1):
+            b.calc_step(k)
+        got = b.state()
+        b.close()
+        for q, p in enumerate(probs):
+            r = ref if "ab_series" in p else ref_full
+            assert relerr(got[q][:p["N"] + 1], r) <= 1e-12, (q, len(probs))

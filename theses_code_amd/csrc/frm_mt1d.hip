@@ -907,7 +907,8 @@ struct AbStepArgs {
     int ldml;
     const double* ser;   // series problems: MF_intF_choice's value per history node
     int N0;              // the block's start (history index)
-    int k0, ks;          // steps k0 .. k0 + ks - 1, t = k tau; ks = 1 with series problems
+    int k0, ks;          // steps k0 .. k0 + ks - 1, t = k tau; k_ab_steps takes series
+                         // problems one step at a time
     double tau;
     double* err;         // per problem: running sum of (C_j - CC)^2
 };
@@ -1092,8 +1093,8 @@ struct AbSeriesArgs {
 constexpr int kRecountMaxL = 4096;
 
 // The non-finite branch of MF_intF (MF_int_series.cpp:594-609 with
-// F_nosorting = 1, where the `else` binds to the finiteness test) for node
-// e.x, whose last non-finite term is e.y: each non-finite term replaces the
+// F_nosorting = 1, where the `else` binds to the finiteness test) for the node
+// of lc1, whose last non-finite term is `last`: each non-finite term replaces the
 // running sum by sum_sort_pyramid (200-218) of all products Lc1[l] Kc[l]
 // (0 where either is not finite), and the finite terms after the last such
 // term are added to it in increasing l.  The whole workgroup works on the
@@ -1102,25 +1103,13 @@ constexpr int kRecountMaxL = 4096;
 // into the level's last sum.  Elements of equal magnitude and opposite sign
 // may be ordered differently from std::sort; their sums are the same unless
 // such a pair straddles a pair boundary.  Every thread of the workgroup
-// calls it with the same node.
-__device__ void ab_block_recount(const AbSeriesArgs& a, int2 e, double* v, double* w) {
+// calls it with the same node; thread 0 gets the sum.
+//
+// ab_pyramid: the workgroup's sort of v[0 .. n2) (a power of two, zeros from
+// maxl on) and its pairwise sum; returns where the sum lies (v or w).
+__device__ __forceinline__ const double* ab_pyramid(double* v, double* w, int n2, int maxl) {
 #pragma clang fp contract(off)
     const int tid = threadIdx.x;
-    const int64_t h = e.x;
-    const MtProbDev& P = a.pr[a.gprob[h / kGroup]];
-    const int maxl = P.ser_maxl;
-    const double* __restrict__ T = a.tab + P.ser_off + (int64_t)(a.i - 2) * kAbSeriesRows * maxl;
-    int n2 = 1;
-    while (n2 < maxl) n2 <<= 1;
-    for (int l = tid; l < n2; l += blockDim.x) {
-        double x = 0.0;
-        if (l < maxl) {
-            const double c1 = a.lc1[(int64_t)l * a.ldh + h], kc = T[l];
-            if (isfinite(c1) && isfinite(kc)) x = c1 * kc;
-        }
-        v[l] = x;
-    }
-    __syncthreads();
     for (int k = 2; k <= n2; k <<= 1)
         for (int j = k >> 1; j > 0; j >>= 1) {
             for (int l = tid; l < n2; l += blockDim.x) {
@@ -1153,89 +1142,107 @@ __device__ void ab_block_recount(const AbSeriesArgs& a, int2 e, double* v, doubl
         dst = t;
         m = m2;
     }
-    if (tid == 0) {
-        double ret = src[0];
-        for (int l = e.y + 1; l < maxl; ++l) {
-            const double c1 = a.lc1[(int64_t)l * a.ldh + h], kc = T[l];
-            if (isfinite(c1) && isfinite(kc)) ret += c1 * kc;
-        }
-        a.part[h] = ret / (1.0 - P.alpha);
-    }
-    __syncthreads();  // v and w are reused by the next node
+    return src;
 }
 
-// One thread per node: MF_intF_choice(i, ..., on = i - 2, mn = 1, append_all
-// = 1, Fvalue = F) (MF_int_series.cpp:839-853) on the node's accumulators.
-// Both phases append to MF_intF_Fv's Lc2 (779-804: add sk F, or keep log|Lc2|
-// with its sign once the sum overflows, after which the newest term alone
-// is kept in log form); the series phase adds dp F to MF_intF's Lc1 and
-// returns sum Lc1 Kc (598-603), the integral phase returns sum of the
-// products of Lc2 and Kc with either in log form (806-822), terms in
-// increasing l, over (1 - a).  Products and sums are rounded separately, as
-// the reference's x86-64 build does.  Returns in *last_bad the last term
-// whose Lc1 or Kc was not finite (-1: none) and in *maxl_out the series
-// length.
-__device__ inline void ab_series_node(const AbSeriesArgs& a, int64_t h, int* last_bad_out,
-                                      int* maxl_out) {
+__device__ __forceinline__ double ab_block_recount(const double* lc1, int64_t ld, const double* T,
+                                                   int maxl, int last, double* v, double* w) {
 #pragma clang fp contract(off)
-    if (h >= a.ldh) return;
-    const int p = a.gprob[h / kGroup];
-    if (p < 0) return;
-    const MtProbDev& P = a.pr[p];
-    if (!P.ser || h - P.hoff >= P.N - 1) return;
-    const int maxl = P.ser_maxl;
-    const double* __restrict__ T = a.tab + P.ser_off + (int64_t)(a.i - 2) * kAbSeriesRows * maxl;
-    const bool series = a.choice[P.ser_coff + a.i - 2] == 1;
-    const double F = a.F[h];
+    int n2 = 1;
+    while (n2 < maxl) n2 <<= 1;
+    for (int l = threadIdx.x; l < n2; l += blockDim.x) {
+        double x = 0.0;
+        if (l < maxl) {
+            const double c1 = lc1[(int64_t)l * ld], kc = T[(int64_t)l * kAbSeriesRows];
+            if (isfinite(c1) && isfinite(kc)) x = c1 * kc;
+        }
+        v[l] = x;
+    }
+    __syncthreads();
+    const double* src = ab_pyramid(v, w, n2, maxl);
+    double ret = 0.0;
+    if (threadIdx.x == 0) {
+        ret = src[0];
+        for (int l = last + 1; l < maxl; ++l) {
+            const double c1 = lc1[(int64_t)l * ld], kc = T[(int64_t)l * kAbSeriesRows];
+            if (isfinite(c1) && isfinite(kc)) ret += c1 * kc;
+        }
+    }
+    __syncthreads();  // v and w are reused by the next node
+    return ret;
+}
+
+// One term of a node's step: kc, lk its value coefficient (in log form where lk
+// is not 0), k1 and k2, k2l the factors the increment F enters Lc1 and Lc2
+// with (k2l for the log form, where lF = log|F|); updates Lc1 (series phase), Lc2 and its log
+// flag, adds the term to ret.  False where the series phase met a non-finite
+// Lc1 or kc.  Products and sums are rounded separately, as the reference's
+// x86-64 build does.
+__device__ __forceinline__ bool ab_term(bool series, double kc, double lk, double k1, double k2,
+                                        double k2l, double F, double lF, double& c1, double& c2,
+                                        int& fl, double& ret) {
+#pragma clang fp contract(off)
+    if (fl == 0) {
+        const double nv = c2 + k2 * F;
+        if (!isfinite(nv)) {
+            fl = c2 > 0.0 ? 1 : -1;
+            c2 = log(fabs(c2));
+        } else {
+            c2 = nv;
+        }
+    } else {
+        c2 = k2l + lF;
+        fl = F > 0.0 ? -1 : 1;
+    }
+    if (series) {
+        c1 = c1 + k1 * F;
+        if (!isfinite(c1) || !isfinite(kc)) return false;
+        ret += c1 * kc;
+        return true;
+    }
+    double v = 0.0;
+    if (fl == 0 && lk == 0) v = c2 * kc;
+    if (fl != 0 && lk == 0) v = fl * (kc > 0.0 ? 1.0 : -1.0) * exp(c2 + log(fabs(kc)));
+    if (fl == 0 && lk != 0) v = lk * (c2 > 0.0 ? 1.0 : -1.0) * exp(kc + log(fabs(c2)));
+    if (fl != 0 && lk != 0) v = lk * fl * exp(kc + c2);
+    if (!isfinite(v)) v = 0.0;
+    ret += v;
+    return true;
+}
+
+// Terms l0 .. l1 - 1 of MF_intF_choice(i, ..., on = i - 2, mn = 1, append_all =
+// 1, Fvalue = F) (MF_int_series.cpp:839-853) on one node's accumulators, one
+// lane per node.  Both phases append to MF_intF_Fv's Lc2 (779-804: add sk F, or
+// keep log|Lc2| with its sign once the sum overflows, after which the newest
+// term alone is kept in log form); the series phase adds dp F to MF_intF's Lc1
+// and returns sum Lc1 Kc (598-603), the integral phase returns sum of the
+// products of Lc2 and Kc with either in log form (806-822), terms in increasing
+// l.  Returns in *last the last term whose Lc1 or Kc was not finite.  T: the
+// step's coefficients, the same on every lane.
+__device__ __forceinline__ double ab_series_node(const_doubles T, bool series, double F, int64_t ld,
+                                                 double* __restrict__ lc1, double* __restrict__ lc2,
+                                                 signed char* __restrict__ lflag, int l0, int l1,
+                                                 int* last) {
     // the accumulators are only this node's: no access aliases another, so
     // the loads of several terms can be in flight together
-    double* __restrict__ lc1 = a.lc1 + h;
-    double* __restrict__ lc2 = a.lc2 + h;
-    signed char* __restrict__ lflag = a.lflag + h;
-    const int64_t ld = a.ldh;
+    constexpr int R = kAbSeriesRows;
+    const double lF = log(fabs(F));
     double ret = 0.0;
-    int last_bad = -1;  // the last term whose Lc1 or Kc was not finite
     // one term: the accumulators of term l as loaded (c2, fl, c1)
     auto term = [&](int l, double c2, int fl, double c1) {
         const int64_t q = (int64_t)l * ld;
-        if (fl == 0) {
-            const double nv = c2 + T[3 * maxl + l] * F;
-            if (!isfinite(nv)) {
-                fl = c2 > 0.0 ? 1 : -1;
-                c2 = log(fabs(c2));
-            } else {
-                c2 = nv;
-            }
-        } else {
-            c2 = T[4 * maxl + l] + log(fabs(F));
-            fl = F > 0.0 ? -1 : 1;
-        }
+        const const_doubles t = T + (int64_t)l * R;
+        const int f0 = fl;
+        if (!ab_term(series, t[0], t[1], t[2], t[3], t[4], F, lF, c1, c2, fl, ret)) *last = l;
         lc2[q] = c2;
-        lflag[q] = (signed char)fl;
-        const double kc = T[l];
-        if (series) {
-            c1 = c1 + T[2 * maxl + l] * F;
-            lc1[q] = c1;
-            if (isfinite(c1) && isfinite(kc))
-                ret += c1 * kc;
-            else
-                last_bad = l;
-        } else {
-            const double lk = T[maxl + l];
-            double v = 0.0;
-            if (fl == 0 && lk == 0) v = c2 * kc;
-            if (fl != 0 && lk == 0) v = fl * (kc > 0.0 ? 1.0 : -1.0) * exp(c2 + log(fabs(kc)));
-            if (fl == 0 && lk != 0) v = lk * (c2 > 0.0 ? 1.0 : -1.0) * exp(kc + log(fabs(c2)));
-            if (fl != 0 && lk != 0) v = lk * fl * exp(kc + c2);
-            if (!isfinite(v)) v = 0.0;
-            ret += v;
-        }
+        if (fl != f0) lflag[q] = (signed char)fl;
+        if (series) lc1[q] = c1;
     };
     // the accumulators of 8 terms are loaded before any is updated (the
     // terms are still added in increasing l)
     constexpr int B = 8;
-    int l = 0;
-    for (; l + B <= maxl; l += B) {
+    int l = l0;
+    for (; l + B <= l1; l += B) {
         double c2[B], c1[B];
         int fl[B];
 #pragma unroll
@@ -1248,13 +1255,11 @@ __device__ inline void ab_series_node(const AbSeriesArgs& a, int64_t h, int* las
 #pragma unroll
         for (int u = 0; u < B; ++u) term(l + u, c2[u], fl[u], c1[u]);
     }
-    for (; l < maxl; ++l) {
+    for (; l < l1; ++l) {
         const int64_t q = (int64_t)l * ld;
         term(l, lc2[q], lflag[q], series ? lc1[q] : 0.0);
     }
-    a.part[h] = ret / (1.0 - P.alpha);
-    *last_bad_out = last_bad;
-    *maxl_out = maxl;
+    return ret;
 }
 
 // One thread per node (ab_series_node); then the workgroup recounts, one
@@ -1272,7 +1277,19 @@ __global__ __launch_bounds__(256, 3) void k_ab_series(AbSeriesArgs a) {
     __syncthreads();
     const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int last_bad = -1, maxl = 0;
-    ab_series_node(a, h, &last_bad, &maxl);
+    const int p = h < a.ldh ? a.gprob[h / kGroup] : -1;  // a wavefront's nodes are one problem's
+    if (__builtin_amdgcn_readfirstlane(p) >= 0) {
+        const MtProbDev& P = a.pr[__builtin_amdgcn_readfirstlane(p)];
+        if (P.ser && h - P.hoff < P.N - 1) {
+            maxl = P.ser_maxl;
+            const const_doubles T =
+                scalar_ptr(a.tab + same_on_lanes(P.ser_off)) +
+                (int64_t)(a.i - 2) * kAbSeriesRows * same_on_lanes(P.ser_maxl);
+            a.part[h] = ab_series_node(T, a.choice[P.ser_coff + a.i - 2] == 1, a.F[h], a.ldh,
+                                       a.lc1 + h, a.lc2 + h, a.lflag + h, 0, maxl, &last_bad) /
+                        (1.0 - P.alpha);
+        }
+    }
     if (last_bad >= 0) {
         if (maxl <= kRecountMaxL)
             todo[atomicAdd(&ntodo, 1)] = make_int2((int)h, last_bad);
@@ -1281,8 +1298,357 @@ __global__ __launch_bounds__(256, 3) void k_ab_series(AbSeriesArgs a) {
     }
     __syncthreads();
     const int n = ntodo;
-    for (int q = 0; q < n; ++q) ab_block_recount(a, todo[q], v, w);
+    for (int q = 0; q < n; ++q) {
+        const int2 e = todo[q];
+        const MtProbDev& P = a.pr[a.gprob[e.x / kGroup]];
+        const double ret = ab_block_recount(
+            a.lc1 + e.x, a.ldh,
+            a.tab + P.ser_off + (int64_t)(a.i - 2) * kAbSeriesRows * P.ser_maxl, P.ser_maxl, e.y, v, w);
+        if (threadIdx.x == 0) a.part[e.x] = ret / (1.0 - P.alpha);
+    }
 }
+
+// ---------------------------------------------------------------- AB series, fused steps
+// Steps of the problems with the series history, any number per launch: the
+// problems are independent, so one workgroup stays with a problem from step to
+// step and keeps its accumulators in LDS, where a series kernel and a sweep per
+// step moved 34 bytes per node and term through the last-level cache each time
+// (50 us of 60 us per step on 1024 problems of 100 intervals and 50 terms).
+// NG = ceil(n / 64) wavefronts hold the nodes, (WAVES - 1) / NG of them a
+// node's terms in equal runs; their partial sums meet in LDS, where one more
+// wavefront takes them for the sweep.  Three sizes of LDS, so that small
+// problems share a CU.  That batch over 600 steps: 35.5 -> 12.6 ms; the sums
+// alone take about 3.4 us of the 4.9 us a problem's step has, the sweep 2.4
+// (with the accumulators left in global memory two problems per CU did not fit
+// L2 and it ran 34 ms; in registers the unrolled terms spilled, 53 ms).
+constexpr int kSerSteps = 256;  // steps per launch of a batch with nothing else
+constexpr int kSerNodes = 320;  // the sweep's 5 nodes per lane
+
+struct SerSplit {
+    int ng, groups, terms;  // wavefronts by nodes, by terms, terms of each
+    bool fits;              // in `waves` wavefronts and `bytes` of LDS
+};
+
+// LDS: [maxl][n] (Lc1, Lc2); [groups][64 ng] partial sums; increment, state,
+// sin and cos of pi x [n]; three lines in chunk order; recount [1.5 n2];
+// last non-finite term per node [n], their count.
+__host__ __device__ inline SerSplit ser_split(int n, int maxl, int waves, int bytes) {
+    SerSplit s{(n + 63) / 64, 0, 0, false};
+    if (n > kSerNodes || s.ng > waves - 1) return s;
+    s.groups = (waves - 1) / s.ng;
+    s.terms = (maxl + s.groups - 1) / s.groups;
+    s.groups = (maxl + s.terms - 1) / s.terms;
+    int n2 = 1;
+    while (n2 < maxl) n2 <<= 1;
+    const int64_t need = (int64_t)maxl * n * 16 + (int64_t)s.groups * s.ng * 512 + 4 * n * 8 +
+                         3 * 64 * 6 * 8 + (int64_t)n2 * 12 + n * 4 + 16;
+    s.fits = s.terms <= 64 && need <= bytes;
+    return s;
+}
+
+struct SerShare {
+    double2* c12;                        // [maxl][n]
+    double *part, *F, *c, *sp, *cp, *X, *cf, *cal, *v, *w;
+    int *bad, *nbad;
+    __device__ SerShare(char* lds, int n, int maxl, const SerSplit& q) {
+        int n2 = 1;
+        while (n2 < maxl) n2 <<= 1;
+        c12 = reinterpret_cast<double2*>(lds);
+        part = reinterpret_cast<double*>(c12 + maxl * n);
+        F = part + q.groups * q.ng * 64;
+        c = F + n;
+        sp = c + n;
+        cp = sp + n;
+        X = cp + n;
+        cf = X + 64 * 6;
+        cal = cf + 64 * 6;
+        v = cal + 64 * 6;
+        w = v + n2;
+        bad = reinterpret_cast<int*>(w + (n2 + 1) / 2);
+        nbad = bad + n;
+    }
+};
+
+// The sweep of one step on one wavefront, as ab_steps: the state and the
+// increment in element order, the recurrences in chunk order.  First the part
+// of the right-hand side that does not need the series' value, then the rest;
+// returns this lane's part of the sum of (C_j - CC)^2.  One wavefront's LDS
+// accesses are in order.
+template <int CM>
+__device__ __forceinline__ void ser_rhs(const AbStepArgs& a, const MtProbDev& P, int step, double E,
+                                        double Ii1a, const SerShare& sh) {
+    const int lane = threadIdx.x & 63, n = P.N - 1;
+    const double h = P.dL, t = step * a.tau;
+#pragma unroll
+    for (int r = 0; r < CM; ++r) {
+        const int e = r * 64 + lane;
+        if (e < n)
+            sh.X[pad_at<CM>(e)] =
+                Ii1a * sh.c[e] + ab_f(P.src, (e + 1) * h, t, P.alpha, E, sh.sp[e], sh.cp[e]);
+    }
+}
+
+template <int CM>
+__device__ __forceinline__ double ser_sweep(const AbStepArgs& a, const MtProbDev& P, int step,
+                                            double i1a, double itau, int groups,
+                                            const SerShare& sh) {
+    const int lane = threadIdx.x & 63;
+    const int m = P.N, n = m - 1, e0 = lane * CM, nn = (n + 63) / 64 * 64;
+    const double h = P.dL, A = -(1.0 / (h * h)) - (1.0 / (2.0 * h)), t = step * a.tau;
+    if (step >= 2) {
+#pragma unroll
+        for (int r = 0; r < CM; ++r) {
+            const int e = r * 64 + lane;
+            if (e < n) {
+                double ret = sh.part[e];
+                for (int q = 1; q < groups; ++q) ret += sh.part[q * nn + e];
+                sh.X[pad_at<CM>(e)] -= ret * i1a;
+            }
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    const double b0 = ab_CC(P.src, 0.0, t), un = ab_CC(P.src, m * h, t);
+    double v[CM], Pp = 1.0, Qq = 0.0, Pt, Qt;
+#pragma unroll
+    for (int k = 0; k < CM; ++k) {
+        v[k] = 0.0;
+        if (e0 + k < n) {
+            const double cf = sh.cf[lane * (CM + 1) + k];
+            v[k] = sh.X[lane * (CM + 1) + k];
+            const double pk = cf * A, qk = -cf * v[k];
+            Qq = pk * Qq + qk;
+            Pp = pk * Pp;
+        }
+    }
+    scan_affine_up_total(Pp, Qq, lane, Pt, Qt);
+    double y = Pp * b0 + Qq;
+#pragma unroll
+    for (int k = 0; k < CM; ++k) {
+        if (e0 + k < n) {
+            y = sh.cf[lane * (CM + 1) + k] * (A * y - v[k]);
+            v[k] = y;
+        }
+    }
+    Pp = 1.0;
+    Qq = 0.0;
+#pragma unroll
+    for (int k = CM - 1; k >= 0; --k) {
+        if (e0 + k < n) {
+            const double cal = sh.cal[lane * (CM + 1) + k];
+            Qq = cal * Qq + v[k];
+            Pp = cal * Pp;
+        }
+    }
+    scan_affine_down_total(Pp, Qq, lane, Pt, Qt);
+    y = Pp * un + Qq;
+#pragma unroll
+    for (int k = CM - 1; k >= 0; --k) {
+        if (e0 + k < n) {
+            y = sh.cal[lane * (CM + 1) + k] * y + v[k];
+            sh.X[lane * (CM + 1) + k] = y;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    double d2 = 0.0;
+#pragma unroll
+    for (int r = 0; r < CM; ++r) {
+        const int e = r * 64 + lane;
+        if (e < n) {
+            const double c = sh.X[pad_at<CM>(e)], f = (c - sh.c[e]) * itau;
+            a.hist[(int64_t)(step - 1) * a.ldh + P.hoff + e] = f;
+            sh.F[e] = f;
+            sh.c[e] = c;
+            const double d = fabs(c - ab_CC_in(P.src, h * (e + 1), t, sh.sp[e]));
+            d2 += d * d;
+        }
+    }
+    return d2;
+}
+
+// A lane's run of terms of one step on the accumulators in LDS (c12: its node's
+// first one, the next term's n further on), as ab_term, in increasing order;
+// neg, pos: the terms whose Lc2 is in log form, by its sign.  Four terms at a
+// time, together where no lane has anything rare among them (an Lc2 that
+// overflows just now, a value that is not finite, a log form in the integral
+// phase): two multiply-adds, a product and the finiteness tests each.
+__device__ __forceinline__ double ser_terms(const_doubles T, bool series, double F, double2* c12,
+                                            int n, int terms, int l0, uint64_t& neg, uint64_t& pos,
+                                            int* last) {
+#pragma clang fp contract(off)
+    constexpr int B = 4, R = kAbSeriesRows;
+    const double lF = __any((neg | pos) != 0) ? log(fabs(F)) : 0.0;  // log forms read it
+    double ret = 0.0;
+    for (int i0 = 0; i0 < terms; i0 += B) {
+        double2 c[B];
+        double v[B];
+        const uint32_t logs = (uint32_t)((neg | pos) >> i0) & 15u;
+        int plain = 1;  // & rather than &&: no branches
+#pragma unroll
+        for (int j = 0; j < B; ++j) c[j] = c12[min(i0 + j, terms - 1) * n];
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const const_doubles t = T + min(i0 + j, terms - 1) * R;
+            const double kc = t[0];
+            const bool lg = logs >> j & 1;
+            const double n2 = c[j].y + t[3] * F;
+            plain &= (int)lg | (int)isfinite(n2);
+            c[j].y = lg ? t[4] + lF : n2;
+            if (series) {
+                c[j].x = c[j].x + t[2] * F;
+                v[j] = c[j].x * kc;
+                plain &= (int)isfinite(c[j].x) & (int)isfinite(kc);
+            } else {
+                v[j] = c[j].y * kc;
+                plain &= (int)!lg & (int)(t[1] == 0) & (int)isfinite(v[j]);
+            }
+        }
+        if (__all(plain)) {
+#pragma unroll
+            for (int j = 0; j < B; ++j) {
+                if (i0 + j < terms) {
+                    c12[(i0 + j) * n] = c[j];
+                    ret += v[j];
+                }
+            }
+            const uint64_t m = uint64_t(15) << i0, l = (uint64_t)logs << i0;
+            neg = (neg & ~m) | (F > 0.0 ? l : 0);
+            pos = (pos & ~m) | (F > 0.0 ? 0 : l);
+        } else {
+#pragma unroll 1
+            for (int i = i0; i < min(i0 + B, terms); ++i) {
+                const const_doubles t = T + i * R;
+                double2 x = c12[i * n];
+                int fl = (int)(pos >> i & 1) - (int)(neg >> i & 1);
+                if (!ab_term(series, t[0], t[1], t[2], t[3], t[4], F, lF, x.x, x.y, fl, ret))
+                    *last = l0 + i;
+                c12[i * n] = x;
+                neg = (neg & ~(uint64_t(1) << i)) | (uint64_t)(fl < 0) << i;
+                pos = (pos & ~(uint64_t(1) << i)) | (uint64_t)(fl > 0) << i;
+            }
+        }
+    }
+    return ret;
+}
+
+// After a step's series sums: the nodes that met a non-finite term, one after
+// another, by the whole workgroup (sh.bad, sh.nbad).
+__device__ __forceinline__ void ser_recounts(const double* T, int n, int maxl, int groups, int nn,
+                                             const SerShare& sh) {
+    for (int q = 0; q < n; ++q) {
+        const int lb = sh.bad[q];  // the same on every lane
+        if (lb < 0) continue;
+        const double ret = ab_block_recount(&sh.c12[q].x, 2 * n, T, maxl, lb, sh.v, sh.w);
+        if (threadIdx.x == 0) {
+            sh.part[q] = ret;
+            for (int g = 1; g < groups; ++g) sh.part[g * nn + q] = 0.0;
+        }
+    }
+    __syncthreads();
+}
+
+template <int WAVES, int BYTES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_ab_series_steps(
+    AbStepArgs a, AbSeriesArgs b) {
+    __shared__ __attribute__((aligned(16))) char lds[BYTES];
+    const int lane = threadIdx.x & 63, wv = same_on_lanes((int)(threadIdx.x >> 6));
+    const int p = same_on_lanes(a.order[blockIdx.x]);
+    const MtProbDev P = same_on_lanes(a.pr[p]);
+    const int m = P.N, n = m - 1, maxl = P.ser_maxl;
+    const SerSplit sp = ser_split(n, maxl, WAVES, BYTES);
+    const SerShare sh(lds, n, maxl, sp);
+    const int nn = 64 * sp.ng, sweeper = sp.ng * sp.groups;
+    if (wv > sweeper) return;  // before any barrier
+    const int64_t ld = a.ldh, tstep = (int64_t)maxl * kAbSeriesRows;
+    const double* tab = b.tab + P.ser_off;
+    if (wv == sweeper) {
+        const int cm = n <= 128 ? 2 : 5;
+        double* C = a.U + P.uoff;
+        for (int e = lane; e < n; e += 64) {
+            const double x = (e + 1) * P.dL;
+            sh.c[e] = C[e + 1];
+            sh.F[e] = a.k0 >= 2 ? a.hist[(int64_t)(a.k0 - 2) * ld + P.hoff + e] : 0.0;
+            sh.sp[e] = P.src == 2 ? sinpi(x) : 0.0;
+            sh.cp[e] = P.src == 2 ? cospi(x) : 0.0;
+            sh.cf[e + e / cm] = a.cf[P.hoff + e];
+            sh.cal[e + e / cm] = a.cal[P.hoff + e];
+            sh.bad[e] = -1;
+        }
+        if (lane == 0) *sh.nbad = 0;
+        const double Ii1a = scalar_ptr(a.d0)[p], i1a = 1.0 / (1.0 - P.alpha), itau = 1.0 / a.tau;
+        double es = 0.0;
+        __syncthreads();
+        for (int st = 0; st < a.ks; ++st) {
+            const int step = a.k0 + st;
+            const double E = scalar_ptr(a.ml)[(int64_t)p * a.ldml + step - 1];
+            if (cm == 2) ser_rhs<2>(a, P, step, E, Ii1a, sh);
+            else ser_rhs<5>(a, P, step, E, Ii1a, sh);
+            __syncthreads();  // the series' sums are in
+            if (*sh.nbad) {
+                ser_recounts(tab + (step - 2) * tstep, n, maxl, sp.groups, nn, sh);
+                for (int e = lane; e < n; e += 64) sh.bad[e] = -1;
+                if (lane == 0) *sh.nbad = 0;
+            }
+            double d2 = cm == 2 ? ser_sweep<2>(a, P, step, i1a, itau, sp.groups, sh)
+                                : ser_sweep<5>(a, P, step, i1a, itau, sp.groups, sh);
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) d2 += __shfl_xor(d2, o);
+            es += d2;  // the two ends equal CC exactly
+            __syncthreads();  // the increment is in
+        }
+        for (int e = lane; e < n; e += 64) C[e + 1] = sh.c[e];
+        if (lane == 0) {
+            const double t = (a.k0 + a.ks - 1) * a.tau;
+            C[0] = ab_CC(P.src, 0.0, t);
+            C[m] = ab_CC(P.src, m * P.dL, t);
+            a.err[p] += es;
+        }
+        return;
+    }
+    const int tg = wv / sp.ng, l0 = tg * sp.terms, e = (wv - tg * sp.ng) * 64 + lane;
+    const int terms = min(sp.terms, maxl - l0);
+    const bool live = e < n;
+    double2* c12 = sh.c12 + (int64_t)l0 * n + min(e, n - 1);
+    uint64_t neg = 0, pos = 0;
+    if (live)
+        for (int i = 0; i < terms; ++i) {
+            const int64_t q = (int64_t)(l0 + i) * ld + P.hoff + e;
+            c12[i * n] = make_double2(b.lc1[q], b.lc2[q]);
+            const int f = b.lflag[q];
+            neg |= (uint64_t)(f < 0) << i;
+            pos |= (uint64_t)(f > 0) << i;
+        }
+    __syncthreads();
+    for (int st = 0; st < a.ks; ++st) {
+        const int step = a.k0 + st;
+        if (step >= 2) {
+            double ret = 0.0;
+            int last = -1;
+            if (live)
+                ret = ser_terms(scalar_ptr(tab + (step - 2) * tstep + (int64_t)l0 * kAbSeriesRows),
+                                same_on_lanes(b.choice[P.ser_coff + step - 2]) == 1, sh.F[e], c12, n,
+                                terms, l0, neg, pos, &last);
+            sh.part[tg * nn + e] = ret;
+            if (last >= 0) {
+                atomicMax(&sh.bad[e], last);
+                *sh.nbad = 1;
+            }
+        }
+        __syncthreads();
+        if (step >= 2 && *sh.nbad) ser_recounts(tab + (step - 2) * tstep, n, maxl, sp.groups, nn, sh);
+        __syncthreads();
+    }
+    if (live)
+        for (int i = 0; i < terms; ++i) {
+            const int64_t q = (int64_t)(l0 + i) * ld + P.hoff + e;
+            const double2 x = c12[i * n];
+            b.lc1[q] = x.x;
+            b.lc2[q] = x.y;
+            b.lflag[q] = (signed char)((int)(pos >> i & 1) - (int)(neg >> i & 1));
+        }
+}
+
+// The variants, smallest first: wavefronts and LDS of a workgroup.
+#define FRM_SER_CASES(X) X(4, 36 * 1024) X(8, 76 * 1024) X(16, 156 * 1024)
 
 // ---------------------------------------------------------------- fitting error
 // solve_and_test (mt_minimal.cpp:1277-1330) for every problem of the batch:
@@ -1448,6 +1814,8 @@ struct frm_mt1d {
     double* ab_err = nullptr; // [nprob]
     // kind AB, series history (ab_series)
     int ser_maxL = 0, ser_count = 0;
+    int ser_waves = 0;  // k_ab_series_steps: the variant's wavefronts (0: not all series
+                        // problems fit one)
     int* gprob_mt = nullptr;  // group -> problem for the full-history sums (-1: series)
     double* ser_tab = nullptr;
     int* ser_choice = nullptr;
@@ -1458,6 +1826,7 @@ struct frm_mt1d {
     int* psi_qcount = nullptr;       // [2] queue lengths (by step parity)
     int psi_qcap = 0;
     std::vector<double> ser_bytes;   // per step i >= 2: algorithmic bytes of k_ab_series
+    double ser_state_bytes = 0.0;    // the accumulators read and written once
     // fitting error (solve_and_test)
     int nobs = 0;
     std::vector<double> obs_T;       // host copy: which observations fall in which step
@@ -1569,6 +1938,24 @@ static hipError_t mt_launch_far_t(frm_mt1d* s, int N0) {
                      s->gvalid, s->far);
 }
 
+// The series problems' step k (>= 2 for k_ab_series, which reads F).
+static AbSeriesArgs mt_series_args(const frm_mt1d* s, int k) {
+    AbSeriesArgs c;
+    c.pr = s->probs;
+    c.gprob = s->gprob;
+    c.ldh = s->ldh;
+    c.tab = s->ser_tab;
+    c.choice = s->ser_choice;
+    c.F = k >= 2 ? (const double*)s->hist + (size_t)(k - 2) * s->ldh : nullptr;  // step k - 1's
+    c.lc1 = s->ser_lc;
+    c.lc2 = s->ser_lc + (size_t)s->ser_maxL * s->ldh;
+    c.lflag = s->ser_flag;
+    c.part = s->part;
+    c.i = k;
+    c.bad = s->bad;
+    return c;
+}
+
 // The far sums of the block that starts at history index N0.
 static hipError_t mt_launch_far(frm_mt1d* s, int N0) {
     const bool tab = s->kind == FRM_MT_PSI;
@@ -1577,9 +1964,11 @@ static hipError_t mt_launch_far(frm_mt1d* s, int N0) {
     return tab ? mt_launch_far_t<double, true>(s, N0) : mt_launch_far_t<double, false>(s, N0);
 }
 
-// Steps k .. k + ks - 1 of every problem, all in block b.
+// Steps k .. k + ks - 1 of every problem, all in block b (a batch of nothing
+// but fused series problems has no blocks).
 static hipError_t mt_launch_steps(frm_mt1d* s, int b, int k, int ks) {
-    const dim3 g((unsigned)s->nprob), t((unsigned)(64 * ((s->maxN - 2 + 64 * kMtCM) / (64 * kMtCM))));
+    const int fused = s->ser_waves ? s->ser_count : 0;
+    const dim3 g((unsigned)(s->nprob - fused)), t((unsigned)(64 * ((s->maxN - 2 + 64 * kMtCM) / (64 * kMtCM))));
     if (s->kind == FRM_MT_AB) {
         AbStepArgs a;
         a.pr = s->probs;
@@ -1601,7 +1990,18 @@ static hipError_t mt_launch_steps(frm_mt1d* s, int b, int k, int ks) {
         a.ks = ks;
         a.tau = s->tau;
         a.err = s->ab_err;
-        return mt_launch(s, k_ab_steps, g, t, a);
+        if (fused < s->nprob) {
+            const hipError_t e = mt_launch(s, k_ab_steps, g, t, a);
+            if (e != hipSuccess || fused == 0) return e;
+        }
+        a.order = s->order + (s->nprob - fused);
+        const AbSeriesArgs c = mt_series_args(s, k);
+        const dim3 gs((unsigned)fused), ts((unsigned)(64 * s->ser_waves));
+#define X(WAVES, BYTES) \
+    if (s->ser_waves == WAVES) return mt_launch(s, k_ab_series_steps<WAVES, BYTES>, gs, ts, a, c);
+        FRM_SER_CASES(X)
+#undef X
+        return hipErrorInvalidValue;
     }
     MtStepArgs a;
     a.pr = s->probs;
@@ -1769,6 +2169,7 @@ static int ab_setup(frm_ctx* ctx, frm_mt1d* s, const frm_mt1d_desc* d) {
         for (int p = 0; p < s->nprob; ++p) {
             const MtProbDev& P = s->hprobs[p];
             if (!P.ser) continue;
+            s->ser_state_bytes += 34.0 * P.ser_maxl * (P.N - 1);
             for (int i = 2; i <= cap; ++i) {
                 const bool series = sch[P.ser_coff + i - 2] == 1;
                 s->ser_bytes[i - 2] += (double)(P.N - 1) * (P.ser_maxl * (series ? 34.0 : 18.0) + 16.0);
@@ -1913,8 +2314,20 @@ int frm_mt1d_create(frm_ctx* ctx, const frm_mt1d_desc* d, frm_mt1d** out) {
         e = hipMalloc(&s->far, sizeof(double) * (size_t)kHistBlock * s->ldh);
     std::vector<int> order(d->nprob);
     for (int p = 0; p < d->nprob; ++p) order[p] = p;
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int x, int y) { return s->hprobs[x].N > s->hprobs[y].N; });
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+        const MtProbDev &X = s->hprobs[x], &Y = s->hprobs[y];  // series problems last
+        return X.ser != Y.ser ? X.ser < Y.ser : X.N > Y.N;
+    });
+    // the smallest variant of the fused series kernel that every series problem fits
+#define X(WAVES, BYTES)                                                       \
+    if (s->ser_count > 0 && !s->ser_waves) {                                  \
+        s->ser_waves = WAVES;                                                 \
+        for (const MtProbDev& P : s->hprobs)                                  \
+            if (P.ser && !ser_split(P.N - 1, P.ser_maxl, WAVES, BYTES).fits)  \
+                s->ser_waves = 0;                                             \
+    }
+    FRM_SER_CASES(X)
+#undef X
     if (e == hipSuccess) e = hipMalloc(&s->order, sizeof(int) * d->nprob);
     if (e == hipSuccess)
         e = hipMemcpy(s->order, order.data(), sizeof(int) * d->nprob, hipMemcpyHostToDevice);
@@ -2052,8 +2465,9 @@ int frm_mt1d_step(frm_mt1d* s, int32_t nsteps) {
         const int k = s->tstep, h = k - off, b = std::max(0, h) / J;
         auto obs = [&](int st) { return s->nobs ? s->fit_off[st] - s->fit_off[st - 1] : 0; };
         const int fcnt = obs(k);
-        int ks = std::min(most, (b + 1) * J - h);
-        if (fcnt > 0 || s->ser_count > 0) ks = 1;
+        const bool all_fused = s->ser_waves && s->ser_count == s->nprob;  // no history sums
+        int ks = std::min(most, all_fused ? kSerSteps : (b + 1) * J - h);
+        if (fcnt > 0 || (s->ser_count > 0 && !s->ser_waves)) ks = 1;
         for (int i = 1; i < ks; ++i)
             if (obs(k + i) > 0) ks = i;
         FitArgs fa{};
@@ -2102,26 +2516,16 @@ int frm_mt1d_step(frm_mt1d* s, int32_t nsteps) {
             FRM_HIP(ctx, mt_launch_psi_weights_ahead(s, b + 1));
             s->wahead = b + 1;
         }
-        if (s->kind == FRM_MT_AB && s->ser_count > 0 && k >= 2) {
-            AbSeriesArgs c;
-            c.pr = s->probs;
-            c.gprob = s->gprob;
-            c.ldh = s->ldh;
-            c.tab = s->ser_tab;
-            c.choice = s->ser_choice;
-            c.F = (const double*)s->hist + (size_t)(h - 1) * s->ldh;  // step k - 1's increment
-            c.lc1 = s->ser_lc;
-            c.lc2 = s->ser_lc + (size_t)s->ser_maxL * s->ldh;
-            c.lflag = s->ser_flag;
-            c.part = s->part;
-            c.i = k;
-            c.bad = s->bad;
+        if (s->kind == FRM_MT_AB && s->ser_count > 0 && !s->ser_waves && k >= 2) {
+            const AbSeriesArgs c = mt_series_args(s, k);
             LaunchTimer t(ctx, FRM_K_MEMTERM, s->ser_bytes.empty() ? 0.0 : s->ser_bytes[k - 2]);
             FRM_HIP(ctx, mt_launch(s, k_ab_series, dim3((unsigned)((s->ldh + 255) / 256)), dim3(256),
                                    c));
         }
         {
-            LaunchTimer t(ctx, FRM_K_SWEEP1D, 0.0);
+            // fused series problems: their accumulators in and out, once
+            const bool fused = s->ser_waves != 0;
+            LaunchTimer t(ctx, fused ? FRM_K_MEMTERM : FRM_K_SWEEP1D, fused ? s->ser_state_bytes : 0.0);
             FRM_HIP(ctx, mt_launch_steps(s, b, k, ks));
         }
         // once the block's last steps are through, its buffers are free

@@ -311,11 +311,11 @@ void ab_series_tables(double a, double tau, int maxl, int maxkiter, double eps, 
                          std::log(std::fabs(spectral(a, vk)));
                 }
             }
-            T[0 * maxl + l] = kc;
-            T[1 * maxl + l] = lg;
-            T[2 * maxl + l] = dp;
-            T[3 * maxl + l] = std::exp(std::pow(vk, 1.0 / a) * t * tau) - std::exp(std::pow(vk, 1.0 / a) * ((t + 1) * tau));
-            T[4 * maxl + l] = std::pow(vk, 1.0 / a) * t * tau + std::log(std::exp(std::pow(vk, 1.0 / a) * tau) - 1);
+            T[(size_t)l * kAbSeriesRows + 0] = kc;
+            T[(size_t)l * kAbSeriesRows + 1] = lg;
+            T[(size_t)l * kAbSeriesRows + 2] = dp;
+            T[(size_t)l * kAbSeriesRows + 3] = std::exp(std::pow(vk, 1.0 / a) * t * tau) - std::exp(std::pow(vk, 1.0 / a) * ((t + 1) * tau));
+            T[(size_t)l * kAbSeriesRows + 4] = std::pow(vk, 1.0 / a) * t * tau + std::log(std::exp(std::pow(vk, 1.0 / a) * tau) - 1);
         }
     }
 }

@@ -38,11 +38,11 @@ class FvNodes {
     double wk1_, wk2_, wk3_, mC1_, mC2_;
 };
 
-// Rows per step of ab_series_tables: Kc, its log flag, dp, sk, log sk.
+// Values per step and term of ab_series_tables: Kc, its log flag, dp, sk, log sk.
 constexpr int kAbSeriesRows = 5;
 
 // Node-independent coefficients of the series history of solve_and_check
-// (simple = 0) for steps i = 2..cap: tab[(i-2)*kAbSeriesRows*maxl ...],
+// (simple = 0) for steps i = 2..cap: tab[((i-2)*maxl + l)*kAbSeriesRows ...],
 // choice[i-2] = 1 (series) or 2 (integral form).
 void ab_series_tables(double a, double tau, int maxl, int maxkiter, double eps, int cap,
                       double* tab, int* choice);

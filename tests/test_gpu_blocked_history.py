@@ -33,10 +33,12 @@ def _case(sN, M):
     return S.coefs_advection(vx, vy, 1e-3, 1.0 / (sN + 1)), rng.uniform(0, 1, nn)
 
 
-# fewer nodes than 2^15, than 2^18, and more (one launch variant each)
+# the one-workgroup path at the edges of its lanes, nodes per thread and LDS;
+# then fewer nodes than 2^15, than 2^18, and more (one launch variant each)
 @pytest.mark.parametrize("precision,tol", [(N.PREC_F64, 1e-12), (N.PREC_F32C, 1e-6),
                                            (N.PREC_SOE, 1e-6), (N.PREC_MFMA_BF16, 1e-6)])
-@pytest.mark.parametrize("sN,M", [(3, 2), (41, 33), (201, 188), (530, 511)])
+@pytest.mark.parametrize("sN,M", [(2, 2), (3, 2), (33, 32), (33, 34), (40, 33), (65, 20), (20, 65),
+                                  (66, 20), (41, 33), (201, 188), (530, 511)])
 def test_lod2d_blocks_match_oracle(ctx, sN, M, precision, tol):
     coefs, C0 = _case(sN, M)
     steps = 2 * B + 5

@@ -62,6 +62,7 @@ struct frm_lod2d {
     int ldw = 0;               // capacity + kHistBlock
     double* far = nullptr;     // far sums of the current block: [2][kHistBlock][hist->ld]
                                // (full history) or [2][kSoeBlock][hist->ld] (SOE, FP64 states)
+    bool small = false;        // the grid takes k_lod_small, not the sweeps
     int ring = 0;              // slots of an increment ring (0: the whole history is stored)
     double* rcoef = nullptr;   // rows:    a, f, al interleaved per line (load_coefs)
     double* ccoef = nullptr;   // columns: the same
@@ -468,6 +469,254 @@ __global__ __launch_bounds__((col_width<CM, W>() * kWave * W)) void k_lod_cols(C
                     p.slot[q] = d;
             }
         }
+    }
+}
+
+// ------------------------------------------------------------- small grids
+// Steps n0 .. n0 + ks - 1 (one block's) of a small grid in one workgroup: the
+// sweeps' lines and the block's increments stay in LDS, the state and each
+// line's coefficients in registers, and a barrier stands where the other path
+// ends a kernel.  A line is one 16-lane row of a wavefront, CM elements per lane,
+// so that four lines share each scan's instructions and 64 rows of lanes hold
+// every line of a direction.  Memory-term sums, right-hand sides and increments
+// go node by node in storage order.  What it takes: lines of at most
+// kSmallLine in both directions, and 128 bytes of LDS per node for the field
+// and the 15 increments that a block's steps read (1270 nodes).  40 x 33: 16.1
+// us per step with its three launches, 4.0 here, bound by the instructions of 16
+// wavefronts on one CU.  (Increments read back from memory: 8.4 us; kept in
+// registers, two nodes per thread: spills, 17 us; a wavefront per line: 10 us.)
+constexpr int kSmallLine = 64;
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallLds = 159 * 1024;
+
+struct SmallArgs {
+    double* C;             // state, reference layout
+    const double *rcoef, *ccoef;  // [3][lines][n]
+    void* hist;
+    int64_t ldh;
+    const double *far;     // far sums of the block [2][kHistBlock][ldh], or null
+    const double* w;       // lag-indexed [2][ldw]
+    int ldw;
+    int ld, NX, NY, N0, n0, ks;
+    double r_negsk, c_negsk, S_half, sg, kch, C1;
+};
+
+// stride of a row in LDS: odd, so that a column's elements spread over the banks
+__host__ __device__ constexpr int small_stride(int NX) { return NX | 1; }
+
+// Bytes of LDS: the field and kHistBlock - 1 increments.
+static int64_t small_bytes(int NX, int NY, size_t esz) {
+    return (int64_t)NY * small_stride(NX) * 8 + (int64_t)(kHistBlock - 1) * NX * NY * esz;
+}
+
+// A barrier for LDS alone: __syncthreads also waits for global loads and
+// stores, which here only their own thread looks at.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// One line per 16-lane row: its element e is x[e se] on entry (the right-hand
+// side) and on exit (the solution), for lanes with `store`; first: the value
+// before element 0 (line_solve's b0).  v0: the first element's solution on the
+// row's first lane.  Returns u_n.
+template <int CM>
+__device__ __forceinline__ double small_line(const double (&a)[CM], const double (&f)[CM],
+                                             const double (&al)[CM], double* x, int se, int n,
+                                             double first, bool store, double& v0) {
+    const int lane = threadIdx.x & 63, e0 = (lane & 15) * CM;
+    double v[CM], P = 1.0, Q = 0.0;
+#pragma unroll
+    for (int k = 0; k < CM; ++k) v[k] = x[min(e0 + k, n - 1) * se];
+#pragma unroll
+    for (int k = 0; k < CM; ++k) {
+        if (e0 + k < n) {
+            const double p = f[k] * a[k], q = -f[k] * v[k];
+            Q = p * Q + q;
+            P = p * P;
+        }
+    }
+    affine_level<kDppRowShr + 1>(P, Q);
+    affine_level<kDppRowShr + 2>(P, Q);
+    affine_level<kDppRowShr + 4>(P, Q);
+    affine_level<kDppRowShr + 8>(P, Q);
+    double y = dpp_move<kDppRowShr + 1>(1.0, P) * first + dpp_move<kDppRowShr + 1>(0.0, Q);
+    double un = 0.0;
+#pragma unroll
+    for (int k = 0; k < CM; ++k) {
+        if (e0 + k < n) {
+            y = f[k] * (a[k] * y - v[k]);
+            v[k] = y;
+        }
+        if (e0 + k == n - 1) un = y / (1.0 - al[k]);
+    }
+    un = __shfl(un, (lane & 48) + (n - 1) / CM);
+    P = 1.0;
+    Q = 0.0;
+#pragma unroll
+    for (int k = CM - 1; k >= 0; --k) {
+        if (e0 + k < n) {
+            Q = al[k] * Q + v[k];
+            P = al[k] * P;
+        }
+    }
+    affine_level<kDppRowShl + 1>(P, Q);
+    affine_level<kDppRowShl + 2>(P, Q);
+    affine_level<kDppRowShl + 4>(P, Q);
+    affine_level<kDppRowShl + 8>(P, Q);
+    y = dpp_move<kDppRowShl + 1>(1.0, P) * un + dpp_move<kDppRowShl + 1>(0.0, Q);
+#pragma unroll
+    for (int k = CM - 1; k >= 0; --k) {
+        if (e0 + k < n) {
+            y = al[k] * y + v[k];
+            if (store) x[(e0 + k) * se] = y;
+        }
+    }
+    v0 = y;
+    return un;
+}
+
+// R nodes per thread; CX, CY elements per lane of the rows and columns.
+template <typename HT, int R, int CX, int CY>
+__global__ __launch_bounds__(kSmallThreads) void k_lod_small(SmallArgs p) {
+    constexpr int J = kHistBlock;
+    __shared__ __attribute__((aligned(8))) char lds[kSmallLds];
+    const int NX = p.NX, NY = p.NY, SX = small_stride(NX), nodes = NX * NY;
+    double* M = reinterpret_cast<double*>(lds);       // right-hand side of a sweep, then its solution
+    HT* inc = reinterpret_cast<HT*>(M + NY * SX);     // [J - 1][nodes] the block's increments
+    const int tid = threadIdx.x, j0 = p.n0 - p.N0, L = tid >> 4, e0 = tid & 15;
+    HT* hist = static_cast<HT*>(p.hist) + (int64_t)p.N0 * p.ldh;
+    // this thread's nodes (one past the end repeats the last and stores nothing)
+    int q[R], at[R];
+    double c[R], fr[R], fc[R];
+    bool mine[R];
+    // wavefronts without a line skip the sweep: the instructions of 16
+    // wavefronts are what bounds a step
+    const int wv0 = __builtin_amdgcn_readfirstlane(tid) & ~63;
+    const bool rows = wv0 / 16 < NY, cols = wv0 / 16 < NX;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        mine[r] = tid + r * kSmallThreads < nodes;
+        q[r] = min(tid + r * kSmallThreads, nodes - 1);
+        const int y = q[r] / NX, x = q[r] - y * NX;
+        at[r] = y * SX + x;
+        c[r] = p.C[(int64_t)(y + 1) * p.ld + x + 1];
+        fr[r] = p.far ? p.far[(int64_t)j0 * p.ldh + q[r]] : 0.0;
+        fc[r] = p.far ? p.far[(int64_t)(J + j0) * p.ldh + q[r]] : 0.0;
+        for (int u = 0; u < j0; ++u) {
+            const HT x = hist[(int64_t)u * p.ldh + q[r]];
+            if (mine[r]) inc[u * nodes + q[r]] = x;
+        }
+    }
+    // this row of lanes' line in each direction (spare rows repeat the last)
+    double ra[CX], rf[CX], rl[CX], ca[CY], cf[CY], cl[CY];
+    const int Lr = min(L, NY - 1), Lc = min(L, NX - 1);
+#pragma unroll
+    for (int k = 0; k < CX; ++k) {
+        const int e = Lr * NX + min(e0 * CX + k, NX - 1);
+        ra[k] = p.rcoef[e];
+        rf[k] = p.rcoef[nodes + e];
+        rl[k] = p.rcoef[2 * nodes + e];
+    }
+#pragma unroll
+    for (int k = 0; k < CY; ++k) {
+        const int e = Lc * NY + min(e0 * CY + k, NY - 1);
+        ca[k] = p.ccoef[e];
+        cf[k] = p.ccoef[nodes + e];
+        cl[k] = p.ccoef[2 * nodes + e];
+    }
+    // read-only data at addresses the same on every lane: scalar loads
+    typedef const __attribute__((address_space(4))) double* const_doubles;
+    const const_doubles wr = (const_doubles)p.w, wc = (const_doubles)(p.w + p.ldw);
+    for (int st = 0; st < p.ks; ++st) {
+        const int j = j0 + st;
+        const bool out = st == p.ks - 1;
+        // both targets' sums (own nodes: no barrier) and the rows' right-hand side
+        double ts[R], tc[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            ts[r] = fr[r];
+            tc[r] = fc[r];
+        }
+        constexpr int G = 5;  // lags whose reads go out together
+        static_assert((J - 1) % G == 0, "whole groups");
+#pragma unroll
+        for (int l0 = 1; l0 < J; l0 += G) {
+            if (l0 <= j) {  // lags past the block's first slot read that slot and weigh 0
+                double x[G][R];
+#pragma unroll
+                for (int g = 0; g < G; ++g)
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        x[g][r] = (double)inc[max(j - l0 - g, 0) * nodes + q[r]];
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const double a = l0 + g <= j ? wr[l0 + g - 1] : 0.0;
+                    const double b = l0 + g <= j ? wc[l0 + g - 1] : 0.0;
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        ts[r] += a * x[g][r];
+                        tc[r] += b * x[g][r];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            double om = p.r_negsk * c[r];
+            om += p.S_half;
+            om += p.sg * ts[r];
+            if (mine[r]) M[at[r]] = om;
+            if (p.far && !out) {  // the next step's far sums, on their way during the sweeps
+                fr[r] = p.far[(int64_t)(j + 1) * p.ldh + q[r]];
+                fc[r] = p.far[(int64_t)(J + j + 1) * p.ldh + q[r]];
+            }
+        }
+        lds_barrier();
+        // the boundary nodes, which no sweep reads, are written with the last step
+        double v0 = 0.0, un = 0.0;
+        if (rows) un = small_line<CX>(ra, rf, rl, M + Lr * SX, 1, NX, p.C1, L < NY, v0);
+        if (out && e0 == 0 && L < NY) {
+            double* Crow = p.C + (int64_t)(L + 1) * p.ld;
+            Crow[0] = p.C1;
+            Crow[NX + 1] = un;
+            Crow[NX + 2] = un;
+        }
+        lds_barrier();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const double u = M[at[r]], t = tc[r] + p.kch * (c[r] - u);
+            double om = p.c_negsk * u;
+            om += p.S_half;
+            om += p.sg * t;
+            if (mine[r]) M[at[r]] = om;
+        }
+        lds_barrier();
+        if (cols) un = small_line<CY>(ca, cf, cl, M + Lc, SX, NY, 0.0, L < NX, v0);
+        if (out && e0 == 0 && L < NX) {
+            double* Ccol = p.C + (L + 1);
+            Ccol[0] = v0;
+            Ccol[(int64_t)(NY + 1) * p.ld] = un;
+            Ccol[(int64_t)(NY + 2) * p.ld] = un;
+        }
+        lds_barrier();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const double u = M[at[r]];
+            const HT x = (HT)(u - c[r]);
+            c[r] = u;
+            if (mine[r]) {
+                hist[(int64_t)j * p.ldh + q[r]] = x;
+                if (j < J - 1) inc[j * nodes + q[r]] = x;
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int y = q[r] / NX, x = q[r] - y * NX;
+        if (mine[r]) p.C[(int64_t)(y + 1) * p.ld + x + 1] = c[r];
     }
 }
 
@@ -912,6 +1161,55 @@ static hipError_t upload_coefs(frm_lod2d* s, bool rows, SweepShape sh) {
         interleave_coefs(rows ? s->rplain : s->cplain, lines, n, sh.cm, kWave * sh.w);
     return hipMemcpy(rows ? s->rcoef : s->ccoef, lay.data(), lay.size() * sizeof(double),
                      hipMemcpyHostToDevice);
+}
+
+// Whether a grid takes the one-workgroup path (k_lod_small): full history with
+// lag-only weights, no sweep shape asked for, and what the kernel holds.
+static bool takes_small(const frm_lod2d* s, const frm_lod2d_desc* d) {
+    const bool f32 = s->precision == FRM_PREC_F32C;
+    const bool full = f32 || (s->precision == FRM_PREC_F64 && s->g_func == 0);
+    return full && !d->sweep_w && std::max(s->NX, s->NY) <= kSmallLine &&
+           (int64_t)s->NX * s->NY <= 2 * kSmallThreads &&
+           small_bytes(s->NX, s->NY, f32 ? sizeof(float) : sizeof(double)) <= kSmallLds;
+}
+
+static hipError_t launch_small(frm_lod2d* s, int n, int ks, bool far) {
+    SmallArgs a;
+    a.C = s->C;
+    a.rcoef = s->rcoef;
+    a.ccoef = s->ccoef;
+    a.hist = s->hist->data;
+    a.ldh = s->hist->ld;
+    a.far = far ? s->far : nullptr;
+    a.w = s->w;
+    a.ldw = s->ldw;
+    a.ld = s->ld;
+    a.NX = s->NX;
+    a.NY = s->NY;
+    a.N0 = n / kHistBlock * kHistBlock;
+    a.n0 = n;
+    a.ks = ks;
+    a.r_negsk = -s->sg * s->kr0;
+    a.c_negsk = -s->sg * s->kc0;
+    a.S_half = s->S * 0.5;
+    a.sg = s->sg;
+    a.kch = s->kch;
+    a.C1 = s->C1;
+    const dim3 g(1), t(kSmallThreads);
+    const bool f32 = s->precision == FRM_PREC_F32C;
+    auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, g, t, 0, s->ctx->stream, a);
+        return hipGetLastError();
+    };
+    const bool one = s->NX * s->NY <= kSmallThreads;
+    const int cx = s->NX <= 32 ? 2 : 4, cy = s->NY <= 32 ? 2 : 4;
+#define X(CX, CY)                                                                                \
+    if (cx == CX && cy == CY)                                                                    \
+        return f32 ? launch(one ? k_lod_small<float, 1, CX, CY> : k_lod_small<float, 2, CX, CY>) \
+                   : launch(one ? k_lod_small<double, 1, CX, CY> : k_lod_small<double, 2, CX, CY>);
+    X(2, 2) X(2, 4) X(4, 2) X(4, 4)
+#undef X
+    return hipErrorInvalidValue;
 }
 
 // Autotuner of the sweep launch shape: for every wavefronts-per-line count
@@ -1426,7 +1724,19 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         lod_free(s);
         return check_hip(ctx, e, "hipMemcpy(lod2d setup)");
     }
-    rc = tune_sweeps(s, d->sweep_w);
+    s->small = takes_small(s, d);
+    if (s->small) {
+        s->rsh = SweepShape{pick_cm(s->NX, 1), 1};
+        s->csh = SweepShape{pick_cm(s->NY, 1), 1};
+        e = hipMemcpy(s->rcoef, s->rplain.data(), s->rplain.size() * sizeof(double),
+                      hipMemcpyHostToDevice);
+        if (e == hipSuccess)
+            e = hipMemcpy(s->ccoef, s->cplain.data(), s->cplain.size() * sizeof(double),
+                          hipMemcpyHostToDevice);
+        if (e != hipSuccess) rc = check_hip(ctx, e, "sweep coefficients");
+    } else {
+        rc = tune_sweeps(s, d->sweep_w);
+    }
     if (rc) {
         lod_free(s);
         return rc;
@@ -1488,7 +1798,7 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
     if (s->tstep + nsteps > s->capacity)
         return set_error(ctx, FRM_E_RANGE, "frm_lod2d_step: %d steps exceed capacity %d",
                          s->tstep + nsteps, s->capacity);
-    for (int it = 0; it < nsteps; ++it) {
+    for (const int goal = s->tstep + nsteps; s->tstep < goal;) {
         const int n = s->tstep;
         int nch = 0;
         bool far = false, mid = false;
@@ -1614,6 +1924,14 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
                                               first, N0, s->w, s->ldw, s->far);
                 if (rc) return check_hip(ctx, hipGetLastError(), "hist_far");
             }
+        }
+        if (s->small) {
+            const int ks = std::min(goal - n, n / kHistBlock * kHistBlock + kHistBlock - n);
+            LaunchTimer t(ctx, FRM_K_ROWS, 0.0);
+            FRM_HIP(ctx, launch_small(s, n, ks, far));
+            s->hist->depth += ks;
+            s->tstep = n + ks;
+            continue;
         }
         {
             LaunchTimer t(ctx, FRM_K_ROWS, 0.0);

@@ -30,11 +30,23 @@ __device__ __forceinline__ double lane_value(double x, int lane) {
                             __builtin_amdgcn_readlane(__double2loint(x), lane));
 }
 
+// The same with 0 where there is no source (the control's own zero: no moves to
+// set it up).
+template <int CTRL>
+__device__ __forceinline__ double dpp_zero(double x) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
 // One scan level: (P, Q) after the map that the control brings (the identity
 // where it brings none).
 template <int CTRL, int RMASK = 0xf>
 __device__ __forceinline__ void affine_level(double& P, double& Q) {
-    const double Po = dpp_move<CTRL, RMASK>(1.0, P), Qo = dpp_move<CTRL, RMASK>(0.0, Q);
+    const double Po = dpp_move<CTRL, RMASK>(1.0, P);
+    double Qo;
+    if constexpr (RMASK == 0xf) Qo = dpp_zero<CTRL>(Q);
+    else Qo = dpp_move<CTRL, RMASK>(0.0, Q);
     Q = P * Qo + Q;
     P = P * Po;
 }

@@ -12,9 +12,9 @@
 // (fr_d_t_g_2d.cpp:3340-3437).
 //
 // Measured (512 x 512 FP64, 1000 steps): the pass over the history went from
-// 150 us per step (7.0 TB/s) to 238 us per 16 steps plus 4 us per step for the
-// newest slots in the row kernel, the run from 166 to 32.5 ms; 1024 x 1024
-// with FP32 increments, 500 steps: from 110 to 30.3 ms.  J = 16 makes each
+// 150 us per step (7.0 TB/s) to 177 us per 16 steps plus 4 us per step for the
+// newest slots in the row kernel, the run from 166 to 27.4 ms; 1024 x 1024
+// with FP32 increments, 500 steps: from 110 to 28.2 ms.  J = 16 makes each
 // target one 16-row tile: 64 multiply-adds per FP64 value read, 16 per byte
 // and target pair, so the product takes about as long on the matrix cores
 // (70 TFLOP/s) as its read from memory.
@@ -60,11 +60,13 @@ __device__ __forceinline__ void load_nodes(const HT* p, int m, double (&x)[NC]) 
 // Wavefront tile: 2 targets x 16 steps (one 16-row tile each) by 16 NC nodes,
 // on v_mfma_f64_16x16x4_f64: per 4 slots a lane holds A[i = l%16][k = l/16] =
 // w_t(N0 + i - s0 - k), B[k = l/16][l%16] = Delta_{s0+k} and, per tile, the
-// four rows 4 r + l/16 of D.  KS wavefronts of a workgroup share a tile's
+// four rows 4 r + l/16 of D.  Loads run two products ahead (512 x 512 FP64 at
+// 500 slots: 238 -> 177 us, 6.3 TB/s; held to three wavefronts per SIMD, the
+// sums stay in ordinary registers: 190 us otherwise).  KS wavefronts of a workgroup share a tile's
 // slots and add their sums through LDS in wavefront order, so that a small
 // grid, which has too few tiles to fill the chip, still uses all of it.
 template <typename HT, typename GT, int NC, int KS>
-__global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_hist_far(
+__global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_hist_far(
     const HT* __restrict__ hist, int64_t ld, int first, int N0, const double* __restrict__ w,
     int ldw, GT* __restrict__ G) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -85,16 +87,21 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_hist_far(
         for (int c = 0; c < NC; ++c) acc[t][c] = f64x4{0.0, 0.0, 0.0, 0.0};
     const HT* hp = hist + (int64_t)(a + kg) * ld + i0;
     const double* wp = w + (N0 - a - 1 + m - kg);
-    constexpr int U = NC == 1 ? 8 : 4;  // 4-slot products whose loads go out together
-    int s = a;
-    for (; s + 4 * U <= b; s += 4 * U) {
-        double x[U][NC], v[U][2];
+    // two batches of U 4-slot products: one's loads are in flight during the
+    // other's products
+    constexpr int U = NC == 1 ? 4 : 2;
+    double xa[U][NC], va[U][2], xb[U][NC], vb[U][2];
+    auto load = [&](double (&x)[U][NC], double (&v)[U][2]) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             load_nodes<NC, HT>(hp + (int64_t)(4 * u) * ld, m, x[u]);
             v[u][0] = wp[-4 * u];
             v[u][1] = wp[ldw - 4 * u];
         }
+        hp += (int64_t)(4 * U) * ld;
+        wp -= 4 * U;
+    };
+    auto mul = [&](const double (&x)[U][NC], const double (&v)[U][2]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -102,8 +109,15 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_hist_far(
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
                     acc[t][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[u][t], x[u][c], acc[t][c], 0, 0, 0);
-        hp += (int64_t)(4 * U) * ld;
-        wp -= 4 * U;
+    };
+    const int nb = (b - a) / (4 * U);
+    int s = a + nb * 4 * U;
+    if (nb > 0) load(xa, va);
+    for (int k = 0; k < nb; k += 2) {
+        if (k + 1 < nb) load(xb, vb);
+        mul(xa, va);
+        if (k + 2 < nb) load(xa, va);
+        if (k + 1 < nb) mul(xb, vb);
     }
     for (; s < b; s += 4) {
         double x[NC];

@@ -46,7 +46,7 @@ __global__ __launch_bounds__(256) void k_tridiag(TriArgs p) {
     Mob m{1.0, 0.0, 0.0, 1.0};
 #pragma unroll
     for (int k = 0; k < CM; ++k)
-        if (e0 + k < n) m = mob_mul(Mob{0.0, c[k], -a[k], b[k]}, m);
+        if (e0 + k < n) m = mob_scale(mob_mul(Mob{0.0, c[k], -a[k], b[k]}, m));
     const Mob pre = scan_mob_up(m, lane);
     double cp = pre.m01 / pre.m11;  // applied to (0, 1)
     // reuse c[] for cp_k and b[] for 1/(b_k - a_k cp_{k-1})

@@ -286,7 +286,7 @@ __device__ inline Mob mob_mul(const Mob& x, const Mob& y) {  // x * y (apply y f
     r.m01 = x.m00 * y.m01 + x.m01 * y.m11;
     r.m10 = x.m10 * y.m00 + x.m11 * y.m10;
     r.m11 = x.m10 * y.m01 + x.m11 * y.m11;
-    return mob_scale(r);
+    return r;
 }
 
 template <int CTRL, int RMASK = 0xf>
@@ -295,15 +295,25 @@ __device__ __forceinline__ Mob dpp_mob(const Mob& m) {  // the identity where th
                dpp_move<CTRL, RMASK>(0.0, m.m10), dpp_move<CTRL, RMASK>(1.0, m.m11)};
 }
 
+template <int CTRL, int RMASK, bool SCALE>
+__device__ __forceinline__ void mob_level(Mob& m) {
+    m = mob_mul(m, dpp_mob<CTRL, RMASK>(m));
+    if (SCALE) m = mob_scale(m);
+}
+
 // Exclusive forward scan of Moebius maps (earlier lanes applied first), and the
-// whole wavefront's map.
+// whole wavefront's map.  The maps come scaled (mob_scale).  SCALE: rescaled on
+// every level, for any matrix; without, once at the end: for rows with diagonal
+// R > A + B >= 0, whose elimination divides by at least about R/2, 64 scaled
+// maps stay far inside the range.
+template <bool SCALE>
 __device__ inline Mob scan_mob_up_total(Mob m, int lane, Mob& tot) {
-    m = mob_mul(m, dpp_mob<kDppRowShr + 1>(m));
-    m = mob_mul(m, dpp_mob<kDppRowShr + 2>(m));
-    m = mob_mul(m, dpp_mob<kDppRowShr + 4>(m));
-    m = mob_mul(m, dpp_mob<kDppRowShr + 8>(m));
-    m = mob_mul(m, dpp_mob<kDppRowBcast15, 0xa>(m));
-    m = mob_mul(m, dpp_mob<kDppRowBcast31, 0xc>(m));
+    mob_level<kDppRowShr + 1, 0xf, SCALE>(m);
+    mob_level<kDppRowShr + 2, 0xf, SCALE>(m);
+    mob_level<kDppRowShr + 4, 0xf, SCALE>(m);
+    mob_level<kDppRowShr + 8, 0xf, SCALE>(m);
+    mob_level<kDppRowBcast15, 0xa, SCALE>(m);
+    mob_level<kDppRowBcast31, 0xc, true>(m);
     tot = Mob{lane_value(m.m00, 63), lane_value(m.m01, 63), lane_value(m.m10, 63),
               lane_value(m.m11, 63)};
     return dpp_mob<kDppWaveShr1>(m);
@@ -311,7 +321,7 @@ __device__ inline Mob scan_mob_up_total(Mob m, int lane, Mob& tot) {
 
 __device__ inline Mob scan_mob_up(const Mob& m, int lane) {
     Mob tot;
-    return scan_mob_up_total(m, lane, tot);
+    return scan_mob_up_total<true>(m, lane, tot);
 }
 
 }  // namespace frm

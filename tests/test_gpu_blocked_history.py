@@ -58,6 +58,33 @@ def test_lod2d_blocks_match_oracle(ctx, sN, M, precision, tol):
     g.close()
 
 
+# coefficients that all rows, all columns, both or all but one line share (the
+# sweeps then read one line's); 1e-12 as above, 1e-9 for g(t) = t^p, whose
+# weights' series stop at int_err = 1e-10 on both sides
+@pytest.mark.parametrize("g", [dict(), dict(g_func=3, g_pow=0.8, int_err=1e-10)])
+@pytest.mark.parametrize("alike", ["rows", "cols", "both", "all but the last row's last"])
+def test_lod2d_lines_with_the_same_coefficients(ctx, alike, g):
+    sN, M, steps = 70, 67, 5
+    rng = np.random.default_rng(5)
+    vx = np.full((M + 2, sN + 2), 0.03)
+    vy = np.full((M + 2, sN + 2), -0.02)
+    if alike == "rows":
+        vx[:], vy[:] = rng.uniform(-0.1, 0.1, (2, sN + 2))
+    elif alike == "cols":
+        vx[:], vy[:] = rng.uniform(-0.1, 0.1, (2, M + 2))[:, :, None]
+    elif alike != "both":
+        vx[M - 1, sN - 1] = 0.1
+    coefs = S.coefs_advection(vx.reshape(-1), vy.reshape(-1), 1e-3, 1.0 / (sN + 1))
+    C0 = rng.uniform(0, 1, (sN + 2) * (M + 2))
+    orc = dict(func=3, fpow=g["g_pow"], int_err=g["int_err"]) if g else {}
+    o = O.TGSolver(sN, M, 0.7, 1e-3, 1.0, 0.0, 0.05, *coefs, C0, **orc)
+    s = S.TGSolver(ctx, sN, M, 0.7, 1e-3, 1.0, coefs, C0, capacity=steps, C1=0.0, S=0.05, **g)
+    o.step(steps)
+    s.calc_step(steps)
+    assert relerr(s.b_C, o.state().reshape(M + 2, sN + 2)) <= (1e-9 if g else 1e-12)
+    s.close()
+
+
 @pytest.mark.parametrize("keep", [1, B - 1, B, B + 5, 2 * B])
 def test_lod2d_restricted_sums_across_blocks(ctx, keep):
     sN, M, steps = 41, 33, 3 * B + 2

@@ -58,6 +58,27 @@ def test_lod2d_blocks_match_oracle(ctx, sN, M, precision, tol):
     g.close()
 
 
+# chunks of 6, 12 and 24 unknowns per lane: lines that fill their last lane, and
+# one unknown more than the shape before holds
+@pytest.mark.parametrize("precision,tol", [(N.PREC_F64, 1e-12), (N.PREC_MFMA_BF16, 1e-6)])
+@pytest.mark.parametrize("W,n", [(1, 257), (1, 384), (1, 513), (1, 768), (1, 1025), (1, 1536),
+                                 (2, 768), (2, 1025), (2, 3072), (4, 1536), (4, 3072), (4, 4097),
+                                 (4, 6144)])
+def test_lod2d_chunks_of_six_twelve_and_24(ctx, W, n, precision, tol):
+    for sN, M in ((n + 1, 11), (11, n + 1)):
+        coefs, C0 = _case(sN, M)
+        steps = 3
+        o = O.TGSolver(sN, M, 0.7, 1e-3, 1.0, 0.0, 0.05, *coefs, C0)
+        g = S.TGSolver(ctx, sN, M, 0.7, 1e-3, 1.0, coefs, C0, capacity=steps, C1=0.0, S=0.05,
+                       precision=precision, sweep_w=W)
+        cm = g.sweep_shape[0 if sN > M else 1][0]
+        assert cm in (6, 12, 24) and 64 * W * cm >= n
+        o.step(steps)
+        g.calc_step(steps)
+        assert relerr(g.b_C, o.state().reshape(M + 2, sN + 2)) <= tol
+        g.close()
+
+
 # coefficients that all rows, all columns, both or all but one line share (the
 # sweeps then read one line's); 1e-12 as above, 1e-9 for g(t) = t^p, whose
 # weights' series stop at int_err = 1e-10 on both sides

@@ -40,9 +40,10 @@
 #include "frm_weights.hpp"
 
 namespace frm {
-// Launch shape of a sweep: chunk length CM and wavefronts per line W.
+// Launch shape of a sweep: chunk length CM, wavefronts per line W, and for the
+// columns the lines per workgroup LW.
 struct SweepShape {
-    int cm = 0, w = 1;
+    int cm = 0, w = 1, lw = 0;
 };
 }  // namespace frm
 
@@ -68,7 +69,6 @@ struct frm_lod2d {
     double* ccoef = nullptr;   // columns: the same
     bool rsame = false, csame = false;  // one line's coefficients serve all
     frm::SweepShape rsh, csh;  // launch shapes of the row / column sweeps
-    std::vector<double> rplain, cplain;  // [3][lines][n] coefficients, for re-layout
     int precision = FRM_PREC_F64;
     std::vector<double> hw;    // host copy: kr0, kc0, kch, then [2][capacity] weights
     // sum-of-exponentials form
@@ -373,21 +373,22 @@ struct ColArgs {
     const double* coef;  // interleaved, see load_coefs
     int same;            // one line's coefficients serve all
     int ld, lines, n, NX;
-    int groups;          // column groups of col_width lines
+    int groups;          // column groups of LW lines
     double b0, al1;
 };
 
-// Column lines per workgroup: a row segment of col_width columns is one
-// contiguous piece of the state and right-hand sides; workgroups stay at
-// 512 threads and within the LDS the staging needs.
-template <int CM, int W>
-__host__ __device__ constexpr int col_width() {
-    return (CM * W >= 32 ? 4 : 8) / W > 0 ? (CM * W >= 32 ? 4 : 8) / W : 1;
+// Column lines per workgroup LW: a row segment of LW columns is one contiguous
+// piece of the state and right-hand sides, so wider is better for the memory,
+// but the workgroups of one chip's worth of lines get fewer; timed at creation.
+// A workgroup has 256 threads or more and at most what its registers allow.
+constexpr int kColWidths[] = {1, 2, 4, 8};
+__host__ __device__ constexpr bool col_fits(int CM, int W, int LW) {
+    return LW * W >= 4 && LW * W <= (CM >= 24 ? 4 : CM >= 12 ? 8 : 16) && (LW > 1 || CM >= 24);
 }
 
-template <int CM, int W>
-__global__ __launch_bounds__((col_width<CM, W>() * kWave * W)) void k_lod_cols(ColArgs p) {
-    constexpr int kColW = col_width<CM, W>();
+template <int CM, int W, int LW>
+__global__ __launch_bounds__((LW * kWave * W), CM == 12 ? 4 : 1) void k_lod_cols(ColArgs p) {
+    constexpr int kColW = LW;
     constexpr int S = CM + 1;
     constexpr int NL = kWave * W;
     __shared__ double lds[kColW][NL * S];
@@ -414,6 +415,9 @@ __global__ __launch_bounds__((col_width<CM, W>() * kWave * W)) void k_lod_cols(C
     // thread keeps its C_n values for the increment push and is the only one
     // that overwrites them
     constexpr bool kEarly = CM <= 8;
+    // From 12 elements on, C_n is read between the passes, so that 12 elements
+    // fit in 128 registers and two workgroups in a CU (1531 x 1531: 33.7 -> 29.5 us).
+    constexpr bool kLate = CM >= 12;
     double a[CM], f[CM], al[CM], v[CM], cp[CM];
 #pragma unroll
     for (int k = 0; k < CM; ++k) a[k] = f[k] = al[k] = v[k] = cp[k] = 0.0;
@@ -427,7 +431,8 @@ __global__ __launch_bounds__((col_width<CM, W>() * kWave * W)) void k_lod_cols(C
         for (int r = 0; r < CM; ++r)
             om[r] = q0[(int64_t)min(r * NL + tr, n - 1) * p.NX];  // node (i, j = e+1)
 #pragma unroll
-        for (int r = 0; r < CM; ++r) cp[r] = cc[(int64_t)(min(r * NL + tr, n - 1) + 1) * ld];
+        for (int r = 0; r < CM && !kLate; ++r)
+            cp[r] = cc[(int64_t)(min(r * NL + tr, n - 1) + 1) * ld];
 #pragma unroll
         for (int r = 0; r < CM; ++r) {
             const int e = r * NL + tr;
@@ -440,7 +445,15 @@ __global__ __launch_bounds__((col_width<CM, W>() * kWave * W)) void k_lod_cols(C
 #pragma unroll
         for (int k = 0; k < CM; ++k) v[k] = e0 + k < n ? lds[li][g * S + k] : 0.0;
     }
-    const double un = line_solve_mw<CM, W>(a, f, al, v, e0, n, p.b0, lane, wl, &share[li], live);
+    const double un = line_solve_mw(
+        a, f, al, v, e0, n, p.b0, lane, wl, &share[li], live, nullptr, [&] {
+            if (kLate && tlive) {
+                const double* __restrict__ cc = p.C + (tline + 1);
+#pragma unroll
+                for (int r = 0; r < CM; ++r)
+                    cp[r] = cc[(int64_t)(min(r * NL + tr, n - 1) + 1) * ld];
+            }
+        });
     if (live) {
 #pragma unroll
         for (int k = 0; k < CM; ++k)
@@ -767,6 +780,18 @@ __global__ __launch_bounds__(64) void k_line_coefs(const double* __restrict__ A,
     }
 }
 
+// [3][lines][n] (a, f, al) -> the interleaved layout of load_coefs, for the
+// first `stored` lines; zeros past a line's end.
+__global__ __launch_bounds__(256) void k_layout_coefs(const double* __restrict__ plain, int lines,
+                                                      int stored, int n, int cm, int nl,
+                                                      double* __restrict__ out) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= (int64_t)stored * 3 * cm * nl) return;
+    const int e = (int)(q % nl) * cm + (int)(q / nl % cm);
+    const int64_t lc = q / ((int64_t)cm * nl);  // line * 3 + array
+    out[q] = e < n ? plain[(lc % 3 * lines + lc / 3) * n + e] : 0.0;
+}
+
 // ------------------------------------------------------------- ia/ibk memory term
 // The reference's dt_alg 4 (calc_va, fr_d_t_g_2d.cpp:490-741) for every node:
 // each direction's plan step (frm_iaibk.cpp) evaluates the node's valid
@@ -1005,20 +1030,6 @@ static float bf16_round(double x) {
     return f;
 }
 
-// [3][lines][n] (a, f, al per line) -> the interleaved layout of load_coefs
-// of the first `stored` lines
-static std::vector<double> interleave_coefs(const std::vector<double>& plain, int lines, int stored,
-                                            int n, int cm, int nl) {
-    std::vector<double> out((size_t)stored * 3 * cm * nl, 0.0);
-    for (int L = 0; L < stored; ++L)
-        for (int c = 0; c < 3; ++c)
-            for (int e = 0; e < n; ++e) {
-                const int g = e / cm, k = e % cm;
-                out[(((size_t)L * 3 + c) * cm + k) * nl + g] = plain[((size_t)c * lines + L) * n + e];
-            }
-    return out;
-}
-
 // Whether all lines' coefficients ([arrays][lines][n]) are equal.
 static bool same_lines(const double* p, int arrays, int lines, int n) {
     for (int c = 0; c < arrays; ++c, p += (size_t)lines * n) {
@@ -1030,14 +1041,14 @@ static bool same_lines(const double* p, int arrays, int lines, int n) {
 
 // smallest chunk length that fits n unknowns on 64 W lanes (0: none)
 static int pick_cm(int n, int W) {
-    for (int cm : {4, 8, 16, 32})
+    for (int cm : {4, 6, 8, 12, 16, 24, 32})
         if (n <= kWave * W * cm) return cm;
     return 0;
 }
 
 
-#define FRM_SWEEP_CASES(X) X(4, 1) X(8, 1) X(16, 1) X(32, 1) X(4, 2) X(8, 2) X(16, 2) X(32, 2) \
-    X(4, 4) X(8, 4) X(16, 4) X(32, 4)
+#define FRM_SWEEP_CM(X, W) X(4, W) X(6, W) X(8, W) X(12, W) X(16, W) X(24, W) X(32, W)
+#define FRM_SWEEP_CASES(X) FRM_SWEEP_CM(X, 1) FRM_SWEEP_CM(X, 2) FRM_SWEEP_CM(X, 4)
 
 template <int SRC>
 static hipError_t launch_rows(SweepShape sh, hipStream_t st, const RowArgs& a) {
@@ -1071,23 +1082,24 @@ static hipError_t launch_rows(const frm_lod2d* s, hipStream_t st, const RowArgs&
     }
 }
 
-static int col_groups(SweepShape sh, int lines) {
-    int cw = 0;
-#define X(CM, W) \
-    if (sh.cm == CM && sh.w == W) cw = col_width<CM, W>();
-    FRM_SWEEP_CASES(X)
-#undef X
-    return cw ? (lines + cw - 1) / cw : 0;
+template <int CM, int W, int LW>
+static bool launch_cols_as(SweepShape sh, hipStream_t st, const ColArgs& a) {
+    if constexpr (col_fits(CM, W, LW)) {
+        if (sh.lw != LW) return false;
+        const dim3 grid((unsigned)((a.groups + 7) / 8 * 8));
+        hipLaunchKernelGGL((k_lod_cols<CM, W, LW>), grid, dim3(LW * kWave * W), 0, st, a);
+        return true;
+    } else {
+        return false;
+    }
 }
 
 static hipError_t launch_cols(SweepShape sh, hipStream_t st, const ColArgs& a) {
-    const dim3 grid((unsigned)((a.groups + 7) / 8 * 8));
-#define X(CM, W)                                                                                 \
-    if (sh.cm == CM && sh.w == W) {                                                              \
-        hipLaunchKernelGGL((k_lod_cols<CM, W>), grid, dim3(col_width<CM, W>() * kWave * W), 0, \
-                           st, a);                                                               \
-        return hipGetLastError();                                                                \
-    }
+#define X(CM, W)                                                                        \
+    if (sh.cm == CM && sh.w == W &&                                                     \
+        (launch_cols_as<CM, W, 1>(sh, st, a) || launch_cols_as<CM, W, 2>(sh, st, a) ||  \
+         launch_cols_as<CM, W, 4>(sh, st, a) || launch_cols_as<CM, W, 8>(sh, st, a)))   \
+        return hipGetLastError();
     FRM_SWEEP_CASES(X)
 #undef X
     return hipErrorInvalidValue;
@@ -1158,17 +1170,19 @@ static ColArgs col_args(frm_lod2d* s, int n) {
     a.NX = s->NX;
     a.b0 = 0.0;
     a.al1 = 1.0;
-    a.groups = col_groups(s->csh, a.lines);
+    a.groups = (a.lines + s->csh.lw - 1) / s->csh.lw;
     return a;
 }
 
-static hipError_t upload_coefs(frm_lod2d* s, bool rows, SweepShape sh) {
+// Lays a direction's coefficients ([3][lines][n] in plain) out for a shape.
+static hipError_t layout_coefs(frm_lod2d* s, bool rows, SweepShape sh, const double* plain) {
     const int lines = rows ? s->M - 1 : s->sN - 1, n = rows ? s->NX : s->NY;
-    const std::vector<double> lay =
-        interleave_coefs(rows ? s->rplain : s->cplain, lines, (rows ? s->rsame : s->csame) ? 1 : lines,
-                         n, sh.cm, kWave * sh.w);
-    return hipMemcpy(rows ? s->rcoef : s->ccoef, lay.data(), lay.size() * sizeof(double),
-                     hipMemcpyHostToDevice);
+    const int stored = (rows ? s->rsame : s->csame) ? 1 : lines, nl = kWave * sh.w;
+    const int64_t total = (int64_t)stored * 3 * sh.cm * nl;
+    hipLaunchKernelGGL(k_layout_coefs, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                       s->ctx->stream, plain, lines, stored, n, sh.cm, nl,
+                       rows ? s->rcoef : s->ccoef);
+    return hipGetLastError();
 }
 
 // Whether a grid takes the one-workgroup path (k_lod_small): full history with
@@ -1221,58 +1235,73 @@ static hipError_t launch_small(frm_lod2d* s, int n, int ks, bool far) {
 }
 
 // Autotuner of the sweep launch shape: for every wavefronts-per-line count
-// W in {1, 2, 4} that fits the line (or only `force`), lay the coefficients
-// out for it and time the row and the column sweep on the solver's own
-// buffers (zero state, one chunk of memory-term partials as every step
-// after the first has: a step's full memory traffic and arithmetic), then
-// keep the fastest shape of each.  Runs at creation, before the initial
-// state is set; the state and the history slot it writes are overwritten
-// by frm_lod2d_set_state and the first step.
-static int tune_sweeps(frm_lod2d* s, int force) {
+// W in {1, 2, 4} that fits the line (or only `force`) and every column width,
+// lay the coefficients out for it and time steps' two sweeps on the solver's own
+// buffers (zero state, a block's steps in turn with their far sums, which then
+// come from memory as they do in a run), with the other direction's shape held;
+// then keep the fastest of each.  Runs at creation, before the initial state is set; the state and the
+// history slot it writes are overwritten by frm_lod2d_set_state and the first
+// step.  (Timed on one step of a block, alone or not, a sweep finds its data closer than
+// a run does: 1531 x 1531 rows ran in 36.8 us in the shape chosen that way, 33.7
+// in another.)  rplain, cplain: the rows' and the columns' coefficients on the
+// device, [3][lines][n].
+static int tune_sweeps(frm_lod2d* s, int force, const double* rplain, const double* cplain) {
     frm_ctx* ctx = s->ctx;
     // the one chunk of partials the timed sweeps read: zeros
     FRM_HIP(ctx, hipMemsetAsync(s->hist->part, 0, sizeof(double) * 2 * s->hist->ld, ctx->stream));
     hipEvent_t e0, e1;
     FRM_HIP(ctx, hipEventCreate(&e0));
     FRM_HIP(ctx, hipEventCreate(&e1));
-    constexpr int kWarm = 3, kReps = 20;
-    const int mid = std::min(kHistBlock / 2, s->hist->capacity);
+    constexpr int kWarm = 4, kReps = kHistBlock;
+    const int block = std::min(kHistBlock, s->capacity);
+    const bool far = s->far || s->F;
     int rc = FRM_OK;
+    // a first shape of the columns, for the rows' turn
+    for (int W : {4, 2, 1})
+        if ((!force || W == force) && pick_cm(s->NY, W))
+            for (int lw : kColWidths)
+                if (!s->csh.cm && col_fits(pick_cm(s->NY, W), W, lw))
+                    s->csh = SweepShape{pick_cm(s->NY, W), W, lw};
+    hipError_t e = layout_coefs(s, false, s->csh, cplain);
+    if (e != hipSuccess) rc = check_hip(ctx, e, "sweep coefficients");
     for (int pass = 0; pass < 2 && rc == FRM_OK; ++pass) {
         const bool rows = pass == 0;
         const int n = rows ? s->NX : s->NY;
+        SweepShape& cur = rows ? s->rsh : s->csh;
+        const double* plain = rows ? rplain : cplain;
         float best = 1e30f;
         SweepShape pick;
         for (int W : {1, 2, 4}) {
-            if ((force && W != force) || !pick_cm(n, W)) continue;
-            const SweepShape sh{pick_cm(n, W), W};
-            hipError_t e = upload_coefs(s, rows, sh);
-            if (rows) s->rsh = sh;
-            else s->csh = sh;
-            float ms = 0.f;
-            for (int it = 0; it < kWarm + kReps && e == hipSuccess; ++it) {
-                if (it == kWarm) e = hipEventRecord(e0, ctx->stream);
+            const int cm = pick_cm(n, W);
+            if ((force && W != force) || !cm) continue;
+            e = layout_coefs(s, rows, SweepShape{cm, W}, plain);
+            for (int lw : kColWidths) {
+                if (rows ? lw > 1 : !col_fits(cm, W, lw)) continue;
+                cur = SweepShape{cm, W, rows ? 0 : lw};
+                float ms = 0.f;
+                for (int it = 0; it < kWarm + kReps && e == hipSuccess; ++it) {
+                    if (it == kWarm) e = hipEventRecord(e0, ctx->stream);
+                    if (e == hipSuccess)
+                        e = launch_rows(s, ctx->stream, row_args(s, 1, it % block, far, far && s->G));
+                    if (e == hipSuccess) e = launch_cols(s->csh, ctx->stream, col_args(s, it % block));
+                }
+                if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
+                if (e == hipSuccess) e = hipEventSynchronize(e1);
+                if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
                 if (e != hipSuccess) break;
-                // a step in the middle of a block, without far sums
-                e = rows ? launch_rows(s, ctx->stream, row_args(s, 1, mid, false, false))
-                         : launch_cols(sh, ctx->stream, col_args(s, 0));
+                if (ms < best) {
+                    best = ms;
+                    pick = cur;
+                }
             }
-            if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
-            if (e == hipSuccess) e = hipEventSynchronize(e1);
-            if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
             if (e != hipSuccess) {
                 rc = check_hip(ctx, e, "sweep autotuning");
                 break;
             }
-            if (ms < best) {
-                best = ms;
-                pick = sh;
-            }
         }
         if (rc == FRM_OK) {
-            if (rows) s->rsh = pick;
-            else s->csh = pick;
-            const hipError_t e = upload_coefs(s, rows, pick);
+            cur = pick;
+            e = layout_coefs(s, rows, pick, plain);
             if (e != hipSuccess) rc = check_hip(ctx, e, "sweep coefficients");
         }
     }
@@ -1577,8 +1606,6 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         lod_free(s);
         return check_hip(ctx, e, "hipMalloc(lod2d coefficients)");
     }
-    s->rplain = std::move(rc3);
-    s->cplain = std::move(cc3);
     s->hw.assign({s->kr0, s->kc0, s->kch});
     s->hw.insert(s->hw.end(), w.begin(), w.end());
     std::vector<double> near_w;  // SOE with FP64 states: [2][kSoeBlock] weights by lag
@@ -1744,17 +1771,28 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         lod_free(s);
         return check_hip(ctx, e, "hipMemcpy(lod2d setup)");
     }
-    if (s->small) {
+    double *rplain = s->rcoef, *cplain = s->ccoef;  // the small path reads them as they are
+    if (!s->small) {
+        rplain = cplain = nullptr;
+        e = hipMalloc(&rplain, rc3.size() * sizeof(double));
+        if (e == hipSuccess) e = hipMalloc(&cplain, cc3.size() * sizeof(double));
+    }
+    if (e == hipSuccess)
+        e = hipMemcpy(rplain, rc3.data(), rc3.size() * sizeof(double), hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+        e = hipMemcpy(cplain, cc3.data(), cc3.size() * sizeof(double), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        rc = check_hip(ctx, e, "sweep coefficients");
+    } else if (s->small) {
         s->rsh = SweepShape{pick_cm(s->NX, 1), 1};
         s->csh = SweepShape{pick_cm(s->NY, 1), 1};
-        e = hipMemcpy(s->rcoef, s->rplain.data(), s->rplain.size() * sizeof(double),
-                      hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = hipMemcpy(s->ccoef, s->cplain.data(), s->cplain.size() * sizeof(double),
-                          hipMemcpyHostToDevice);
-        if (e != hipSuccess) rc = check_hip(ctx, e, "sweep coefficients");
     } else {
-        rc = tune_sweeps(s, d->sweep_w);
+        rc = tune_sweeps(s, d->sweep_w, rplain, cplain);
+    }
+    if (!s->small) {
+        (void)hipStreamSynchronize(ctx->stream);
+        (void)hipFree(rplain);
+        (void)hipFree(cplain);
     }
     if (rc) {
         lod_free(s);

@@ -126,6 +126,16 @@ __device__ inline double line_solve_mw(const double (&a)[CM], const double (&f)[
                                        const double (&al)[CM], double (&v)[CM], int e0, int n,
                                        double b0, int lane, int wl, LineShare<W>* sh, bool active,
                                        const double* un_fixed = nullptr) {
+    return line_solve_mw(a, f, al, v, e0, n, b0, lane, wl, sh, active, un_fixed, [] {});
+}
+
+// mid() runs between the passes, where a and f are no longer needed: loads for
+// after the solve can go out there into their registers.
+template <int CM, int W, typename Mid>
+__device__ inline double line_solve_mw(const double (&a)[CM], const double (&f)[CM],
+                                       const double (&al)[CM], double (&v)[CM], int e0, int n,
+                                       double b0, int lane, int wl, LineShare<W>* sh, bool active,
+                                       const double* un_fixed, Mid mid) {
     // ---- forward
     double P = 1.0, Q = 0.0, Pt = 1.0, Qt = 0.0;
 #pragma unroll
@@ -161,6 +171,7 @@ __device__ inline double line_solve_mw(const double (&a)[CM], const double (&f)[
         for (int k = 0; k < CM; ++k)
             if (e0 + k == n - 1) sh->un = un_fixed ? *un_fixed : v[k] / (1.0 - al[k]);
     }
+    mid();
     __syncthreads();
     const double un = active ? sh->un : 0.0;
     // ---- backward

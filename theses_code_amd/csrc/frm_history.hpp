@@ -29,13 +29,15 @@ int hist_alloc(frm_ctx* ctx, int64_t n_nodes, int32_t capacity, int32_t precisio
 // number of chunks written (0 when there is nothing to sum).  An FP32 store
 // (FRM_PREC_F32C) takes one target and its FP32 weights in d_w32.  With
 // `part` given, the partials go there instead (nchunks * ntargets * ld
-// doubles, see memterm_chunks) and no timing events are recorded.
+// doubles, see memterm_chunks) and no timing events are recorded.  With `sum`
+// given, one chunk of one target goes there instead (n_nodes doubles).
 int memterm_partials(frm_ctx* ctx, frm_hist* h, int ntargets, const double* d_w, int ldw,
                      int* nchunks, int first = 0, const float* d_w32 = nullptr,
-                     double* part = nullptr);
+                     double* part = nullptr, double* sum = nullptr);
 // Time chunks memterm_partials splits slots first .. depth-1 into.
 int memterm_chunks(const frm_hist* h, int first = 0);
-// out[i] = sum_c part[c*ld + i] for one target (chunk order, deterministic)
-int memterm_reduce1(frm_ctx* ctx, const frm_hist* h, int nchunks, double* d_out);
+// One target's sums over slots first .. depth-1 into d_out (n_nodes doubles).
+int memterm_sum1(frm_ctx* ctx, frm_hist* h, const double* d_w, int ldw, int first,
+                 const float* d_w32, double* d_out);
 
 }  // namespace frm

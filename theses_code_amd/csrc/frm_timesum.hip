@@ -323,10 +323,7 @@ int frm_timesum_eval(frm_timesum* s, const frm_timesum_args* a, double* d_S) {
                                     hipMemcpyHostToDevice, ctx->stream));
     }
     FRM_HIP(ctx, hipEventRecord(s->staged, ctx->stream));
-    int nch = 0;
-    int rc = memterm_partials(ctx, h, 1, s->w, depth, &nch, depth - L, f32 ? s->w32 : nullptr);
-    if (rc) return rc;
-    return memterm_reduce1(ctx, h, nch, d_S);
+    return memterm_sum1(ctx, h, s->w, depth, depth - L, f32 ? s->w32 : nullptr, d_S);
 }
 
 }  // extern "C"

@@ -18,6 +18,12 @@
 // target one 16-row tile: 64 multiply-adds per FP64 value read, 16 per byte
 // and target pair, so the product takes about as long on the matrix cores
 // (70 TFLOP/s) as its read from memory.
+//
+// FP32 sums (the MFMA form's mid sums) are rounded, and where a block ends decides
+// what is rounded: they keep blocks of kMidBlock = 8 steps, both targets in one
+// 16-row tile (1024 x 1024, 64 to 112 slots: 90 us, 5.0 TB/s).  Blocks of 16 took
+// 116 us for twice the steps but 4 us more per step in the rows, and moved that
+// form's results by up to 1e-9 of themselves.
 #include "frm_blockhist.hpp"
 
 #include <type_traits>
@@ -57,9 +63,9 @@ __device__ __forceinline__ void load_nodes(const HT* p, int m, double (&x)[NC]) 
     }
 }
 
-// Wavefront tile: 2 targets x 16 steps (one 16-row tile each) by 16 NC nodes,
-// on v_mfma_f64_16x16x4_f64: per 4 slots a lane holds A[i = l%16][k = l/16] =
-// w_t(N0 + i - s0 - k), B[k = l/16][l%16] = Delta_{s0+k} and, per tile, the
+// Wavefront tile: 2 targets x 16 steps (one 16-row tile each; FP32 sums: 2 x 8
+// steps, one tile) by 16 NC nodes, on v_mfma_f64_16x16x4_f64: per 4 slots a lane
+// holds A[i = l%16][k = l/16] = w_t(N0 + i - s0 - k) (w_{i/8}(N0 + i%8 - ...)), B[k = l/16][l%16] = Delta_{s0+k} and, per tile, the
 // four rows 4 r + l/16 of D.  Loads run two products ahead (512 x 512 FP64 at
 // 500 slots: 238 -> 177 us, 6.3 TB/s; held to three wavefronts per SIMD, the
 // sums stay in ordinary registers: 190 us otherwise).  KS wavefronts of a workgroup share a tile's
@@ -69,6 +75,7 @@ template <typename HT, typename GT, int NC, int KS>
 __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_hist_far(
     const HT* __restrict__ hist, int64_t ld, int first, int N0, const double* __restrict__ w,
     int ldw, GT* __restrict__ G) {
+    constexpr int T = sizeof(GT) == 4 ? 1 : 2;  // 16-row tiles
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int m = lane & 15, kg = lane >> 4;
     const int64_t tile = KS == 1 ? (int64_t)blockIdx.x * 4 + wv : blockIdx.x;
@@ -80,34 +87,35 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) __attribute__((amdgpu_wave
         a = min(N0, first + wv * per);
         b = min(N0, a + per);
     }
-    f64x4 acc[2][NC];
+    f64x4 acc[T][NC];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < T; ++t)
 #pragma unroll
         for (int c = 0; c < NC; ++c) acc[t][c] = f64x4{0.0, 0.0, 0.0, 0.0};
     const HT* hp = hist + (int64_t)(a + kg) * ld + i0;
-    const double* wp = w + (N0 - a - 1 + m - kg);
+    const double* wp =
+        w + (N0 - a - 1 - kg) + (T == 1 ? (m >> 3) * ldw + (m & (kMidBlock - 1)) : m);
     // two batches of U 4-slot products: one's loads are in flight during the
     // other's products
     constexpr int U = NC == 1 ? 4 : 2;
-    double xa[U][NC], va[U][2], xb[U][NC], vb[U][2];
-    auto load = [&](double (&x)[U][NC], double (&v)[U][2]) {
+    double xa[U][NC], va[U][T], xb[U][NC], vb[U][T];
+    auto load = [&](double (&x)[U][NC], double (&v)[U][T]) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             load_nodes<NC, HT>(hp + (int64_t)(4 * u) * ld, m, x[u]);
-            v[u][0] = wp[-4 * u];
-            v[u][1] = wp[ldw - 4 * u];
+#pragma unroll
+            for (int t = 0; t < T; ++t) v[u][t] = wp[t * ldw - 4 * u];
         }
         hp += (int64_t)(4 * U) * ld;
         wp -= 4 * U;
     };
-    auto mul = [&](const double (&x)[U][NC], const double (&v)[U][2]) {
+    auto mul = [&](const double (&x)[U][NC], const double (&v)[U][T]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
+                for (int t = 0; t < T; ++t)
                     acc[t][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[u][t], x[u][c], acc[t][c], 0, 0, 0);
     };
     const int nb = (b - a) / (4 * U);
@@ -122,39 +130,40 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) __attribute__((amdgpu_wave
     for (; s < b; s += 4) {
         double x[NC];
         load_nodes<NC, HT>(hp, m, x);
-        const double v0 = wp[0], v1 = wp[ldw];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            acc[0][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(v0, x[c], acc[0][c], 0, 0, 0);
-            acc[1][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(v1, x[c], acc[1][c], 0, 0, 0);
+        for (int t = 0; t < T; ++t) {
+            const double v = wp[t * ldw];
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                acc[t][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(v, x[c], acc[t][c], 0, 0, 0);
         }
         hp += 4 * ld;
         wp -= 4;
     }
     if constexpr (KS == 1) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < T; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                GT* g = G + (int64_t)(t * kHistBlock + 4 * r + kg) * ld + i0;
+                GT* g = G + (int64_t)(16 * t + 4 * r + kg) * ld + i0;
 #pragma unroll
                 for (int c = 0; c < NC; ++c) g[node_of<NC, HT>(c, m)] = (GT)acc[t][c][r];
             }
     } else {
-        __shared__ double part[KS][2 * NC * 4][64];
+        __shared__ double part[KS][T * NC * 4][64];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < T; ++t)
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) part[wv][(t * NC + c) * 4 + r][lane] = acc[t][c][r];
         __syncthreads();
-        for (int q = wv; q < 2 * NC * 4; q += KS) {
+        for (int q = wv; q < T * NC * 4; q += KS) {
             double v = 0.0;
 #pragma unroll
             for (int p = 0; p < KS; ++p) v += part[p][q][lane];
             const int r = q & 3, c = (q >> 2) % NC, t = (q >> 2) / NC;
-            G[(int64_t)(t * kHistBlock + 4 * r + kg) * ld + i0 + node_of<NC, HT>(c, m)] = (GT)v;
+            G[(int64_t)(16 * t + 4 * r + kg) * ld + i0 + node_of<NC, HT>(c, m)] = (GT)v;
         }
     }
 }
@@ -162,8 +171,9 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) __attribute__((amdgpu_wave
 template <typename HT, typename GT>
 static int far_launch(hipStream_t st, const HT* hist, int64_t ld, int first, int N0,
                       const double* w, int ldw, GT* G) {
-    if (!hist || !w || !G || ld <= 0 || ld % 1024 || N0 <= 0 || N0 % kHistBlock || first < 0 ||
-        first >= N0 || ldw < N0 + kHistBlock - 1)
+    constexpr int J = sizeof(GT) == 4 ? kMidBlock : kHistBlock;
+    if (!hist || !w || !G || ld <= 0 || ld % 1024 || N0 <= 0 || N0 % J || first < 0 ||
+        first >= N0 || ldw < N0 + J - 1)
         return -1;
     first = first / 4 * 4;
     if (ld >= 262144) {

@@ -97,7 +97,7 @@ struct frm_lod2d {
     int mfma_nprod = 6;        // 3 (two parts) or 6 (three parts)
     int far_slices = 8;        // node slices of a block's far product (1 to 64)
     float* F = nullptr;        // [2][128][ld]: far parts of this block and the next
-    float* G = nullptr;        // [2][kHistBlock][ld] mid part of the current sub-block
+    float* G = nullptr;        // [2][kMidBlock][ld] mid part of the current sub-block
     // g(t) = t^p (g_func 3): the weights and the sweeps' Thomas coefficients
     // are rebuilt every step
     int g_func = 0;
@@ -1113,7 +1113,8 @@ static RowArgs row_args(frm_lod2d* s, int nch, int n, bool far, bool mid) {
     a.crhs = s->crhs;
     const int64_t hld = s->hist->ld;
     const bool soe = s->precision == FRM_PREC_SOE;
-    const int J = soe ? kSoeBlock : kHistBlock;
+    const bool mf = s->precision == FRM_PREC_MFMA_BF16;
+    const int J = soe ? kSoeBlock : mf ? kMidBlock : kHistBlock;
     const int N0 = n / J * J, j = n - N0;
     a.near.hist = s->hist->data;
     a.near.ld = hld;
@@ -1125,14 +1126,14 @@ static RowArgs row_args(frm_lod2d* s, int nch, int n, bool far, bool mid) {
     a.near.f0 = far ? s->far + (int64_t)j * hld : nullptr;
     a.near.f1 = far ? s->far + (int64_t)(J + j) * hld : nullptr;
     a.near.m0 = a.near.m1 = nullptr;
-    if (s->precision == FRM_PREC_MFMA_BF16) {
+    if (mf) {
         // the 64-step block's far rows (by block parity), the sub-block's mid rows
         const int b = n / kBlockSteps, q = n % kBlockSteps;
         const float* F = s->F + (size_t)(b & 1) * 2 * kBlockSteps * hld;
         a.near.f0 = far ? F + (int64_t)q * hld : nullptr;
         a.near.f1 = far ? F + (int64_t)(kBlockSteps + q) * hld : nullptr;
         a.near.m0 = mid ? s->G + (int64_t)j * hld : nullptr;
-        a.near.m1 = mid ? s->G + (int64_t)(kHistBlock + j) * hld : nullptr;
+        a.near.m1 = mid ? s->G + (int64_t)(kMidBlock + j) * hld : nullptr;
     }
     a.coef = s->rcoef;
     a.same = s->rsame;
@@ -1747,7 +1748,7 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         e = hipMalloc(&s->atab, tab.size() * sizeof(uint16_t));
         // two far buffers: the current block's and the next one's, formed in slices
         if (e == hipSuccess) e = hipMalloc(&s->F, sizeof(float) * 2 * 2 * kBlockSteps * s->hist->ld);
-        if (e == hipSuccess) e = hipMalloc(&s->G, sizeof(float) * 2 * kHistBlock * s->hist->ld);
+        if (e == hipSuccess) e = hipMalloc(&s->G, sizeof(float) * 2 * kMidBlock * s->hist->ld);
         if (e == hipSuccess)
             e = hipMemcpy(s->atab, tab.data(), tab.size() * sizeof(uint16_t), hipMemcpyHostToDevice);
         if (e != hipSuccess) {
@@ -1948,13 +1949,13 @@ int frm_lod2d_step(frm_lod2d* s, int32_t nsteps) {
             }
             // the slots from P0 up to the sub-block start, once per sub-block,
             // summed in FP64; the row kernel adds the newest ones
-            const int N1 = n / kHistBlock * kHistBlock;
+            const int N1 = n / kMidBlock * kMidBlock;
             nch = 1;
             far = P0 > 0;
             mid = N1 > P0;
             if (mid && n == N1) {
                 LaunchTimer t(ctx, FRM_K_MEMTERM,
-                              (double)ld * ((N1 - P0) * 4.0 + 2 * kHistBlock * 4));
+                              (double)ld * ((N1 - P0) * 4.0 + 2 * kMidBlock * 4));
                 if (hist_far(ctx->stream, h32, ld, P0, N1, s->w, s->ldw, s->G))
                     return check_hip(ctx, hipGetLastError(), "hist_far");
             }

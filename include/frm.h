@@ -35,7 +35,7 @@ enum {
 /* memory-term precision forms */
 enum {
     FRM_PREC_F64 = 0,      /* plain FP64 history and FP64 accumulation */
-    FRM_PREC_F32C = 1,     /* FP32 history, compensated (Kahan) FP32 sums */
+    FRM_PREC_F32C = 1,     /* FP32 increments; FP64 sums (time sums: Kahan FP32) */
     FRM_PREC_MFMA_BF16 = 2, /* blocked Toeplitz on MFMA, split hi+lo BF16, FP32 acc */
     FRM_PREC_SOE = 3,       /* sum-of-exponentials recurrences (series history) */
     FRM_PREC_BINOMIAL = 4,  /* the reference's single-series expansion of the history
@@ -168,7 +168,7 @@ typedef struct frm_lod2d_desc {
     int32_t sN, M;
     int32_t capacity;  /* max number of steps (history depth) */
     int32_t precision; /* FRM_PREC_* for the memory term (FRM_PREC_F32C: FP32
-                          increments, 4 B per node and slot; weights and sums
+                          increments, 4 B per node and slot, and weights; sums
                           in FP64) */
     double alpha, tau, sigma, C1, S;
     const double* rowA; /* host arrays of (sN+2)*(M+2) values */

@@ -1764,6 +1764,9 @@ int frm_lod2d_create(frm_ctx* ctx, const frm_lod2d_desc* d, frm_lod2d** out) {
         for (int t = 0; t < 2 && near_w.empty(); ++t)
             std::copy(w.begin() + (size_t)t * d->capacity, w.begin() + (size_t)(t + 1) * d->capacity,
                       wp.begin() + (size_t)t * s->ldw);
+        // FP32 increments go with FP32 weights; the sums over both are FP64
+        if (s->precision == FRM_PREC_F32C)
+            for (double& q : wp) q = (double)(float)q;
         e = hipMemcpy(s->w, wp.data(), wp.size() * sizeof(double), hipMemcpyHostToDevice);
     }
     if (e == hipSuccess) e = hipMemset(s->C, 0, nn * sizeof(double));

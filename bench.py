@@ -248,16 +248,10 @@ def run_mt1d(args, cfg_name):
                        "tau": cfg["tau"], "picard": picard, "parallelism": "1 GPU"},
             "kernels_ms": {k: v[1] for k, v in kt.items()}}
     ms, nb = kt["memterm"][1], kt["memterm"][2]
-    traffic = None
-    tf = os.path.join(REPO, "profiles", "mt1d_psi_traffic.json")
-    if cfg_name == "c3" and os.path.exists(tf) and kt["memterm"][0]:
-        # PMC-measured ratio of HBM to algorithmic bytes of this kernel
-        with open(tf) as f:
-            traffic = json.load(f)["traffic_over_algorithmic"] * nb / kt["memterm"][0]
     line["roofline"] = {"bound": "hbm", "achieved": nb / (ms * 1e-3) / 1e9 if ms else 0.0,
                         "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": (nb / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS) if ms else 0.0,
-                        "traffic": traffic, "kernel": "k_mt_memterm_f64"}
+                        "traffic": None, "kernel": "k_mt_far<double> (one launch per 16 steps)"}
     line["config"]["hist_block"] = hist_block
     if patterns:
         line["launch_patterns"] = patterns
@@ -332,21 +326,21 @@ def run_mt1d(args, cfg_name):
             "kernels_ms": {k: v[1] for k, v in kt32.items()}}
         line["batched_fp64"] = {"value": nodes * K / dt, "seconds": dt,
                                 "kernels_ms": line["kernels_ms"], "roofline": line["roofline"]}
-        # the value's form: the compensated FP32 memory term (4 B per slot and
-        # node of the problems' own nodes; four nodes per lane at this size)
+        # the value's form: the far sums over FP32 increments (4 B per slot and
+        # node of the problems' own nodes, once per 16 steps)
         ms32, nb32 = kt32["memterm"][1], kt32["memterm"][2]
         a32 = nb32 / (ms32 * 1e-3) / 1e9 if ms32 else 0.0
         line["roofline"] = {"bound": "hbm", "achieved": a32, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                             "frac": a32 / HBM_PEAK_GBS, "traffic": None,
                             "traffic_source": "not profiled (no counter pass over this command)",
-                            "kernel": "k_mt_memterm_f32c",
+                            "kernel": "k_mt_far<float>",
                             "launches": kt32["memterm"][0],
                             "avg_launch_ms": ms32 / kt32["memterm"][0] if kt32["memterm"][0] else None,
-                            "bytes_model": "4 B x depth x the problems' own nodes (padding lanes "
-                                           "load nothing)"}
+                            "bytes_model": "(4 B x depth + 16 x 8 B of sums) x the problems' "
+                                           "own nodes, per 16 steps"}
         line["value"] = nodes * K / dt32
         line["ms_per_step"] = dt32 * 1e3 / K
-        line["dtype"] = "f64 weights/Thomas/state, f32 compensated history"
+        line["dtype"] = "f64 weights/sums/Thomas/state, f32 increments"
         if per_problem:
             line["plain_fp64_per_problem"] = per_problem
             line["speedup_vs_plain_fp64"] = line["value"] / per_problem["value"]
@@ -372,7 +366,7 @@ def run_ab1d(args, series=False):
     else:
         cfg = Wl.AB1D_WORKLOAD
         probs = Wl.ab1d_case(nprob=args.nprob or cfg["nprob"])
-        oracle_solve, kernel, n_cpu = O.ab_solve, "k_mt_memterm_f64", 4
+        oracle_solve, kernel, n_cpu = O.ab_solve, "k_mt_far<double>", 4
         plain_cap = args.plain_sample
     K = args.steps if args.steps is not None else cfg["steps"]
     tau = cfg["tau"]
@@ -505,8 +499,7 @@ def _lod_run(ctx, N, case, alpha, tau, sigma, T, precision, window=None, warmup=
     return dt, out, kt, fit, win
 
 
-FORMS = {"f32c": "FP32 increments and weights, Kahan-compensated FP32 history sums, FP64 "
-                 "sweeps",
+FORMS = {"f32c": "FP32 increments and weights, FP64 history sums and sweeps",
          "soe": "sum-of-exponentials history (FP64 mode states unless stated)",
          "mfma": "blocked Toeplitz on MFMA: FP32 increments, split hi+lo BF16, FP32 acc, "
                  "64-step blocks, FP64 near part",
@@ -671,7 +664,6 @@ def run_lod_forms(args, cfg_name):
           and out_forms[f]["rms_rel_err_vs_fp64"] <= 1e-6]
     read_gbs = None if args.no_copy_probe else ctx.read_bandwidth()
     pw_gbs = plain_win["bytes"] / (plain_win["ms"] * 1e-3) / 1e9 if plain_win["ms"] else 0.0
-    ratio, src = _stored_ratio(f"memterm_lod2d_{'1024' if cfg_name == 'c2' else 'ab'}_traffic.json")
     plain = {"form": "plain FP64 full history (the drop-in)",
              "value": tot_nodes * K / tw_plain, "window_seconds": tw_plain,
              "window_seconds_with_events": tw_plain_ev,
@@ -680,13 +672,11 @@ def run_lod_forms(args, cfg_name):
              "roofline": {"bound": "hbm", "achieved": pw_gbs, "peak": HBM_PEAK_GBS,
                           "unit": "GB/s", "frac": pw_gbs / HBM_PEAK_GBS,
                           "frac_of_measured_read": pw_gbs / read_gbs if read_gbs else None,
-                          "kernel": "k_memterm_f64<2>", "launches": plain_win["launches"],
+                          "kernel": "k_hist_far<double> (far sums, one launch per 16 steps)",
+                          "launches": plain_win["launches"],
                           "avg_launch_ms": plain_win["ms"] / max(plain_win["launches"], 1),
                           "bytes_per_launch": plain_win["bytes"] / max(plain_win["launches"], 1),
-                          "traffic": ratio * plain_win["bytes"] / plain_win["launches"]
-                          if ratio and plain_win["launches"] else None,
-                          "traffic_source": f"stored PMC ratio ({src}) x algorithmic bytes"
-                          if ratio else None}}
+                          "traffic": None, "traffic_source": None}}
     if not ok:
         # no form meets the bar: the line is the plain path
         best, chosen = "plain_fp64", plain
@@ -699,7 +689,7 @@ def run_lod_forms(args, cfg_name):
             "scaling": "weak", "vs_baseline": None,
             "dtype": {"mfma": "bf16x2 split MFMA (fp32 acc) far history, fp64 near/sweeps",
                       "soe": "fp64 sweeps; " + ("fp32" if soe_f32 else "fp64") + " SOE states",
-                      "f32c": "f32 compensated history, fp64 sweeps",
+                      "f32c": "f32 increments, fp64 sums and sweeps",
                       "binomial": "f64", "plain_fp64": "f64"}[best],
             "data": "synthetic",
             "config": {"workload": cfg["name"], "form": best, "sets": len(runs),
@@ -750,7 +740,9 @@ def run_lod_forms(args, cfg_name):
         line["roofline"] = {
             "bound": "hbm", "achieved": a, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": a / HBM_PEAK_GBS, "frac_of_measured_read": a / read_gbs if read_gbs else None,
-            "traffic": None, "kernel": "k_soe_memterm (mode recurrences of the SOE form)",
+            "traffic": None,
+            "kernel": ("k_soe_memterm" if soe_f32 else "k_soe_block (once per 8 steps)")
+            + ", mode recurrences of the SOE form",
             "launches": mem["launches"], "avg_launch_ms": mem["ms"] / mem["launches"],
             "bytes_per_launch": mem["bytes"] / mem["launches"],
             "bytes_model": "mode planes read and written (8 or 4 B x modes x 2) + ring and "
@@ -1090,17 +1082,10 @@ def main():
     value = nodes * K / dt
 
     achieved = (nbytes / (ms * 1e-3) / 1e9) if ms > 0 else 0.0
-    # HBM bytes per launch: the PMC-measured ratio of counted to algorithmic
-    # bytes of this kernel (profiles/memterm_lod2d_512_traffic.md) times this
-    # run's algorithmic bytes per launch
-    traffic = None
-    tf = os.path.join(REPO, "profiles", "memterm_lod2d_512_traffic.json")
-    if os.path.exists(tf) and launches:
-        with open(tf) as f:
-            traffic = json.load(f)["traffic_over_algorithmic"] * nbytes / launches
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                "kernel": "k_memterm_f64<2>", "launches": launches,
+                "frac": achieved / HBM_PEAK_GBS, "traffic": None,
+                "kernel": "k_hist_far<double> (far sums, one launch per 16 steps)",
+                "launches": launches,
                 "avg_launch_ms": ms / launches if launches else None,
                 "bytes_per_launch_avg": nbytes / launches if launches else None}
 

@@ -238,7 +238,8 @@ __device__ __forceinline__ void near_sums(const NearArgs& a, int64_t q0, int g, 
     // The last batch makes one trip to memory, not one per slot.  Whole batches
     // without its tests are faster where the registers allow them: 4 elements
     // per lane (512 x 512 FP64 rows: 9.5 us, 9.8 with tests); from 6 on they cost
-    // a wavefront per SIMD (1531 x 1531, 6 elements: 37.9 us, 31.1 with tests).
+    // a wavefront per SIMD (1531 x 1531, 6 elements, up to 15 slots: 37.9 us, 31.1
+    // with tests).
     int u = 0;
     if (CM < 6)
         for (; u + U <= a.cnt; u += U) batch(u, U);

@@ -14,9 +14,9 @@
 // The reference forms every step's sum from scratch (fr_d_t_g_2d.cpp:
 // 3340-3437).  W and Delta are split into two or three BF16 parts whose
 // cross products accumulate in FP32 on v_mfma_f32_16x16x32_bf16.  The rest
-// is summed in FP64: every 16 steps the settled slots from P0 on (hist_far,
-// frm_blockhist.hip, up to 112 slots), every step, in the row kernel, the F
-// row, the mid row and at most 15 recent slots.
+// is summed in FP64: every 8 steps the settled slots from P0 on (hist_far,
+// frm_blockhist.hip, up to 120 slots), every step, in the row kernel, the F
+// row, the mid row and at most 7 recent slots.
 #include <cstring>
 
 #include "frm_mfma.hpp"

@@ -13,8 +13,8 @@
 //
 // Measured (512 x 512 FP64, 1000 steps): the pass over the history went from
 // 150 us per step (7.0 TB/s) to 177 us per 16 steps plus 4 us per step for the
-// newest slots in the row kernel, the run from 166 to 27.4 ms; 1024 x 1024
-// with FP32 increments, 500 steps: from 110 to 28.2 ms.  J = 16 makes each
+// newest slots in the row kernel, the run from 166 to 25.8 ms; 1024 x 1024
+// with FP32 increments, 500 steps: from 110 to 26.7 ms.  J = 16 makes each
 // target one 16-row tile: 64 multiply-adds per FP64 value read, 16 per byte
 // and target pair, so the product takes about as long on the matrix cores
 // (70 TFLOP/s) as its read from memory.

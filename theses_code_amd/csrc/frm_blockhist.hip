@@ -21,9 +21,9 @@
 //
 // FP32 sums (the MFMA form's mid sums) are rounded, and where a block ends decides
 // what is rounded: they keep blocks of kMidBlock = 8 steps, both targets in one
-// 16-row tile (1024 x 1024, 64 to 112 slots: 90 us, 5.0 TB/s).  Blocks of 16 took
+// 16-row tile (1024 x 1024, 64 to 120 slots: 90 us, 5.0 TB/s).  Blocks of 16 took
 // 116 us for twice the steps but 4 us more per step in the rows, and moved that
-// form's results by up to 1e-9 of themselves.
+// form's results by up to 3e-9 of themselves.
 #include "frm_blockhist.hpp"
 
 #include <type_traits>
